@@ -25,6 +25,7 @@
 #include "pp_learned.h"
 #include "pp_membench.h"
 #include "pp_topn.h"
+#include "pp_transfer.h"
 
 namespace {
 
@@ -595,16 +596,39 @@ void stage_memcpy(void* dst, const void* src, size_t n) {
     });
 }
 
+// One host array of a transfer; a transfer's arrays lie back to back in device memory.
+struct HostPart {
+    void* host;
+    size_t bytes;
+};
+
+// The stretches of the parts that bytes [off, off + n) of the device side cover, copied into (TO_STAGE) or out of a
+// pinned chunk.
+template <bool TO_STAGE>
+void stage_parts(void* stage, const HostPart* parts, size_t count, size_t off, size_t n) {
+    size_t at = 0;
+    for (size_t p = 0; p < count; at += parts[p].bytes, ++p) {
+        const size_t lo = std::max(at, off), hi = std::min(at + parts[p].bytes, off + n);
+        if (lo >= hi) continue;
+        char* const h = (char*)parts[p].host + (lo - at);
+        char* const d = (char*)stage + (lo - off);
+        if (TO_STAGE) stage_memcpy(d, h, hi - lo);
+        else stage_memcpy(h, d, hi - lo);
+    }
+}
+
 // host -> device through the two pinned chunks: the host fills one while the other's copy runs.  Queued on the
 // context's stream; the caller synchronizes before it reads the result.
-pp_status staged_h2d(pp_context* ctx, void* dev, const void* host, size_t bytes) {
+pp_status staged_h2d(pp_context* ctx, void* dev, const HostPart* parts, size_t count) {
     pp_status st;
     if ((st = ensure_staging(ctx)) != PP_OK) return st;
+    size_t bytes = 0;
+    for (size_t p = 0; p < count; ++p) bytes += parts[p].bytes;
     int k = 0;
     for (size_t off = 0; off < bytes; off += kStageChunk, k ^= 1) {
         const size_t n = std::min(kStageChunk, bytes - off);
         PP_HIP(ctx, hipEventSynchronize(ctx->stage_ev[k]));  // the chunk's previous copy has drained
-        stage_memcpy(ctx->stage[k], (const char*)host + off, n);
+        stage_parts<true>(ctx->stage[k], parts, count, off, n);
         PP_HIP(ctx, hipMemcpyAsync((char*)dev + off, ctx->stage[k], n, hipMemcpyHostToDevice, ctx->stream));
         PP_HIP(ctx, hipEventRecord(ctx->stage_ev[k], ctx->stream));
     }
@@ -612,10 +636,12 @@ pp_status staged_h2d(pp_context* ctx, void* dev, const void* host, size_t bytes)
 }
 
 // device -> host through the two pinned chunks: chunk i + 1's copy runs while the host drains chunk i.  Returns once
-// every byte is in `host`.
-pp_status staged_d2h(pp_context* ctx, void* host, const void* dev, size_t bytes) {
+// every byte is on the host.
+pp_status staged_d2h(pp_context* ctx, const HostPart* parts, size_t count, const void* dev) {
     pp_status st;
     if ((st = ensure_staging(ctx)) != PP_OK) return st;
+    size_t bytes = 0;
+    for (size_t p = 0; p < count; ++p) bytes += parts[p].bytes;
     const size_t chunks = (bytes + kStageChunk - 1) / kStageChunk;
     auto queue = [&](size_t i) -> pp_status {
         const size_t off = i * kStageChunk, n = std::min(kStageChunk, bytes - off);
@@ -628,9 +654,19 @@ pp_status staged_d2h(pp_context* ctx, void* host, const void* dev, size_t bytes)
         if (i + 1 < chunks && (st = queue(i + 1)) != PP_OK) return st;  // its chunk was drained one step ago
         PP_HIP(ctx, hipEventSynchronize(ctx->stage_ev[i & 1]));
         const size_t off = i * kStageChunk;
-        stage_memcpy((char*)host + off, ctx->stage[i & 1], std::min(kStageChunk, bytes - off));
+        stage_parts<false>(ctx->stage[i & 1], parts, count, off, std::min(kStageChunk, bytes - off));
     }
     return PP_OK;
+}
+
+pp_status staged_h2d(pp_context* ctx, void* dev, const void* host, size_t bytes) {
+    const HostPart part{const_cast<void*>(host), bytes};
+    return staged_h2d(ctx, dev, &part, 1);
+}
+
+pp_status staged_d2h(pp_context* ctx, void* host, const void* dev, size_t bytes) {
+    const HostPart part{host, bytes};
+    return staged_d2h(ctx, &part, 1, dev);
 }
 
 // ---- device rebucketing ------------------------------------------------------------------------------------------
@@ -2128,6 +2164,109 @@ int32_t pp_hash_rows(uint32_t num_qubits, uint64_t seed, uint32_t width, uint64_
     return hash_rows(num_qubits, seed, width, rows_x, rows_z);
 }
 
+// Terms from which an upload is bucketed on the device.  Its two synchronizations and six launches cost about what the
+// host's counting sort and its five copies do at 1000 terms (both 0.15-0.18 ms, allocations being most of it); at 8191
+// terms the host takes 0.33 ms, the device 0.16.
+constexpr uint64_t kDeviceUploadTerms = 1ull << 10;
+
+static pp_status upload_rows(pp_sum* s, uint32_t n, uint64_t m, int bits, unsigned char* raw, bool* done);
+
+// The n >= 1 host terms into s's first column set, bucketed on the device into the layout the host's stable counting
+// sort would make: the arrays go up as they are, a count gives every term its bucket, a scan lays the segments out, and
+// each bucket's rows are gathered in the host's order.  *done = false, nothing kept, when a bucket is longer than
+// kUploadBucketRows.
+static pp_status upload_bucketed(pp_sum* s, uint32_t n, const uint64_t* x, const uint64_t* z, const void* coeff,
+                                 bool* done) {
+    pp_context* ctx = s->ctx;
+    pp_status st;
+    *done = false;
+    const size_t cb = s->coeff_bytes(), key_bytes = (size_t)n * s->W * 8, c_bytes = ((size_t)n * cb + 15) & ~(size_t)15;
+    // the nonzero terms decide the bucket count
+    const unsigned T = host_threads(n);
+    std::vector<uint64_t> nonzero(T, 0);
+    host_parallel(T, [&](unsigned t, unsigned TT) {
+        uint64_t lo, hi, k = 0;
+        part_range(n, t, TT, lo, hi);
+        if (s->kind == PP_COEFF_F64)
+            for (uint64_t i = lo; i < hi; ++i) k += ((const double*)coeff)[i] != 0.0;
+        else
+            for (uint64_t i = lo; i < hi; ++i) k += ((const float*)coeff)[i] != 0.0f;
+        nonzero[t] = k;
+    });
+    uint64_t m = 0;
+    for (uint64_t k : nonzero) m += k;
+    if (m == 0) return PP_OK;
+    int bits = 0;
+    while (bits < s->max_bits && m > (uint64_t)ctx->tuning.bucket_target * (1ull << bits)) ++bits;
+    // the host's arrays, then each term's bucket and place
+    unsigned char* raw = nullptr;
+    if ((st = dev_alloc(ctx, (void**)&raw, 2 * key_bytes + c_bytes + (size_t)n * 8)) != PP_OK) return st;
+    const HostPart parts[3] = {{const_cast<uint64_t*>(x), key_bytes}, {const_cast<uint64_t*>(z), key_bytes},
+                               {const_cast<void*>(coeff), (size_t)n * cb}};
+    if ((st = staged_h2d(ctx, raw, parts, 3)) == PP_OK) st = upload_rows(s, n, m, bits, raw, done);
+    if (st != PP_OK || !*done) (void)hipStreamSynchronize(ctx->stream);
+    (void)hipFree(raw);
+    return st;
+}
+
+// The device half of upload_bucketed: raw holds x, z, c and room for the buckets and places.
+static pp_status upload_rows(pp_sum* s, uint32_t n, uint64_t m, int bits, unsigned char* raw, bool* done) {
+    pp_context* ctx = s->ctx;
+    pp_status st;
+    const size_t cb = s->coeff_bytes(), key_bytes = (size_t)n * s->W * 8, c_bytes = ((size_t)n * cb + 15) & ~(size_t)15;
+    const uint32_t B = 1u << bits;
+    if ((st = ensure_buckets(s, 0, B)) != PP_OK || (st = ensure_tiles(s, B)) != PP_OK) return st;
+    const BucketArrays& bk = s->bk[0];
+    PP_HIP(ctx, hipMemsetAsync(bk.len, 0, (size_t)B * 4, ctx->stream));
+    uint32_t* index = nullptr;
+    auto args = [&](auto Wc, auto Tv) {
+        constexpr int W = decltype(Wc)::value;
+        using T = decltype(Tv);
+        UploadArgs<W, T> a{};
+        a.x = (const uint64_t*)raw;
+        a.z = (const uint64_t*)(raw + key_bytes);
+        a.c = (const T*)(raw + 2 * key_bytes);
+        a.n = n;
+        a.rows = s->d_rows;
+        a.bits = bits;
+        a.num_buckets = B;
+        a.bucket = (uint32_t*)(raw + 2 * key_bytes + c_bytes);
+        a.place = a.bucket + n;
+        a.index = index;
+        a.start = bk.start;
+        a.len = bk.len;
+        a.ox = s->col[0].x;
+        a.oz = s->col[0].z;
+        a.oc = (T*)s->col[0].c;
+        a.ocap = s->col[0].cap;
+        return a;
+    };
+    hipError_t e = dispatch(s, [&](auto Wc, auto Tv) { return launch_upload_count(ctx->stream, args(Wc, Tv)); });
+    PP_HIP(ctx, e);
+    PP_HIP(ctx, launch_bucket_offsets(ctx->stream, bk.len, B, 4, 0, 0, 0, bk.start, s->d_stats + 3, s->d_tiles,
+                                      s->d_stats, kStatSlots, bk.rows));
+    PP_HIP(ctx, launch_reduce_lens(ctx->stream, bk.len, B, s->d_stats, nullptr));
+    if ((st = read_stats(s)) != PP_OK) return st;
+    const uint64_t longest = s->h_stats[1], end = s->h_stats[3];
+    if (s->h_stats[0] != m) return fail(ctx, PP_ERR_DRIVER, "upload: the bucket lengths disagree with the terms");
+    if (longest > kUploadBucketRows) return PP_OK;
+    if ((st = ensure_columns(s, 0, end)) != PP_OK) return st;
+    if ((st = dev_alloc(ctx, (void**)&index, end * 4)) != PP_OK) return st;
+    e = dispatch(s, [&](auto Wc, auto Tv) { return launch_upload_rows(ctx->stream, args(Wc, Tv)); });
+    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+    (void)hipFree(index);
+    PP_HIP(ctx, e);
+    s->len = m;
+    s->reference_bits = std::min(desired_bits(m, 1024, 128), s->max_bits);
+    s->device_bits = bits;
+    s->max_bucket = (uint32_t)longest;
+    s->cur = 0;
+    s->tail = end;
+    s->has_room = true;
+    *done = true;
+    return PP_OK;
+}
+
 pp_status pp_sum_upload(pp_context* ctx, uint32_t num_qubits, uint32_t width, pp_coeff_kind kind, uint64_t n,
                         const uint64_t* x, const uint64_t* z, const void* coeff, uint64_t hash_seed,
                         pp_sum** out) {
@@ -2166,9 +2305,17 @@ pp_status pp_sum_upload(pp_context* ctx, uint32_t num_qubits, uint32_t width, pp
     if (hipMemcpy(s->d_rows, s->rows.data(), s->rows.size() * 8, hipMemcpyHostToDevice) != hipSuccess)
         return bail(fail(ctx, PP_ERR_DRIVER, "hash rows upload"));
 
+    const size_t cb = s->coeff_bytes();
+    if (n >= kDeviceUploadTerms && n <= UINT32_MAX) {
+        bool done = false;
+        if ((st = upload_bucketed(s, (uint32_t)n, x, z, coeff, &done)) != PP_OK) return bail(st);
+        if (done) {
+            *out = s;
+            return PP_OK;
+        }
+    }
     // Keep nonzero terms, bucket them at the device bucket count (counting sort on the host), transpose to
     // word-major columns.
-    const size_t cb = s->coeff_bytes();
     std::vector<uint64_t> keep_idx;
     keep_idx.reserve(n);
     for (uint64_t i = 0; i < n; ++i) {
@@ -2470,6 +2617,81 @@ pp_status pp_sum_bucket_bits(pp_sum* s, int32_t* reference_bits, int32_t* device
     return PP_OK;
 }
 
+// The sum in canonical order, sorted on the device: each bucket of the coarser of the two bucketings in one workgroup's
+// LDS, written out term-major, then the three arrays through the pinned chunks.  *done = false when such a bucket
+// outgrows the LDS, or the two counts are more than kSortParts apart: the host sorts.
+static pp_status download_sorted(pp_sum* s, uint64_t* x, uint64_t* z, void* coeff, bool* done) {
+    pp_context* ctx = s->ctx;
+    pp_status st;
+    *done = false;
+    const uint64_t n = s->len;
+    const uint32_t B = 1u << s->device_bits, RB = 1u << s->reference_bits;
+    const bool split = RB > B;
+    const uint32_t limit = s->W == 1 ? kSortRows<1> : kSortRows<2>;
+    if ((split ? RB / B : B / RB) > kSortParts || (split && s->max_bucket > limit)) return PP_OK;
+    uint64_t* d_start = nullptr;  // dense starts, then lengths, of the reference buckets
+    if ((st = slot_scratch(s, kScrCounts, (size_t)RB * 12, &d_start)) != PP_OK) return st;
+    uint32_t* const d_len = reinterpret_cast<uint32_t*>(d_start + RB);
+    if ((st = ensure_tiles(s, RB)) != PP_OK) return st;
+    unsigned char* dev = nullptr;
+    const size_t key_bytes = n * s->W * 8;
+    auto args = [&](auto Wc, auto Tv) {
+        constexpr int W = decltype(Wc)::value;
+        using T = decltype(Tv);
+        SortExportArgs<W, T> a{};
+        a.x = s->col[s->cur].x;
+        a.z = s->col[s->cur].z;
+        a.c = (const T*)s->col[s->cur].c;
+        a.cap = s->col[s->cur].cap;
+        a.start = s->bk[s->cur].start;
+        a.len = s->bk[s->cur].len;
+        a.num_buckets = B;
+        a.ref_buckets = RB;
+        a.rows = s->d_rows;
+        a.bits = s->device_bits;
+        a.ref_len = d_len;
+        a.ref_start = d_start;
+        a.out_x = (uint64_t*)dev;
+        a.out_z = (uint64_t*)(dev + key_bytes);
+        a.out_c = (T*)(dev + 2 * key_bytes);
+        return a;
+    };
+    hipError_t e = hipSuccess;
+    uint64_t longest = s->max_bucket;
+    if (split) {  // the rows of each reference bucket counted, then laid out
+        e = dispatch(s, [&](auto Wc, auto Tv) { return launch_ref_counts(ctx->stream, args(Wc, Tv)); });
+        if (e == hipSuccess)
+            e = launch_bucket_offsets(ctx->stream, d_len, RB, 0, 0, 0, 0, d_start, s->d_stats + 3, s->d_tiles);
+        PP_HIP(ctx, e);
+    } else {
+        PP_HIP(ctx, launch_bucket_offsets(ctx->stream, s->bk[s->cur].len, B, 5, 0, RB, B / RB, d_start, s->d_stats + 3,
+                                          s->d_tiles, s->d_stats, kStatSlots, d_len));
+        PP_HIP(ctx, launch_reduce_lens(ctx->stream, d_len, RB, s->d_stats, nullptr));
+        if ((st = read_stats(s)) != PP_OK) return st;
+        longest = s->h_stats[1];
+        if (longest > limit) return PP_OK;
+    }
+    const size_t cb = s->coeff_bytes(), bytes = 2 * key_bytes + n * cb;
+    // the sorted arrays back to back in the spare column set when they fit there, else in an allocation of their own
+    const Columns& spare = s->col[1 - s->cur];
+    unsigned char* own = nullptr;
+    if (spare.cap >= n) {
+        dev = (unsigned char*)spare.x;
+    } else {
+        if ((st = dev_alloc(ctx, (void**)&own, bytes)) != PP_OK) return st;
+        dev = own;
+    }
+    e = dispatch(s, [&](auto Wc, auto Tv) {
+        return launch_sort_export(ctx->stream, args(Wc, Tv), (uint32_t)longest);
+    });
+    const HostPart parts[3] = {{x, key_bytes}, {z, key_bytes}, {coeff, n * cb}};
+    if (e != hipSuccess) st = fail(ctx, PP_ERR_DRIVER, std::string("download: ") + hipGetErrorString(e));
+    else st = staged_d2h(ctx, parts, 3, dev);
+    if (own) (void)hipFree(own);
+    *done = st == PP_OK;
+    return st;
+}
+
 pp_status pp_sum_download(pp_sum* s, uint64_t* x, uint64_t* z, void* coeff) {
     if (s) PP_NOT_CAPTURING(s->ctx, "pp_sum_download");
     if (!s) return PP_ERR_INVALID_ARGUMENT;
@@ -2484,6 +2706,11 @@ pp_status pp_sum_download(pp_sum* s, uint64_t* x, uint64_t* z, void* coeff) {
     const uint32_t W = s->W;
     const size_t cb = s->coeff_bytes();
     const uint32_t B = 1u << s->device_bits;
+    {
+        bool done = false;
+        pp_status ds = download_sorted(s, x, z, coeff, &done);
+        if (ds != PP_OK || done) return ds;
+    }
     uint64_t *d_dense_start = nullptr, *dx = nullptr, *dz = nullptr;
     void* dc = nullptr;
     uint32_t* db = nullptr;

@@ -276,7 +276,7 @@ struct CheckArgs {
 // holds offsets_tiles(n) words.  When clear is set, clear[0 .. clear_n) is zeroed before the total is written (a
 // join's counters, without a launch of their own).
 uint32_t offsets_tiles(uint32_t out_n);
-// out_cap (modes 1-3) receives each resident segment's rows.
+// out_cap (modes 1-5) receives each segment's rows.
 hipError_t launch_bucket_offsets(hipStream_t st, const uint32_t* len, uint32_t num_buckets, uint32_t mode,
                                  uint32_t delta, uint32_t coarse_buckets, uint32_t fold, uint64_t* out_start,
                                  unsigned long long* total, uint64_t* tile_sums, unsigned long long* clear = nullptr,

@@ -16,7 +16,8 @@ namespace pp {
 // kScanTile buckets: tile sums, one workgroup scans the tile sums, then each tile scans itself).
 // mode 0: size = len[b]; mode 1: rotation output room len[b] + len[b ^ delta] (2 len[b] when delta = 0);
 // mode 2: coarsened bucket b < coarse_buckets gathers b + e * coarse_buckets for e < fold; mode 3: len[b] as a
-// resident segment (a permutation run's counts).
+// resident segment (a permutation run's counts); mode 4: len[b] and a quarter more (an upload's segments); mode 5: mode
+// 2's buckets packed densely (a download's reference buckets).
 // ---------------------------------------------------------------------------------------------------------------
 
 constexpr uint32_t kScanItems = 8;
@@ -37,8 +38,8 @@ struct OffsetsArgs {
     uint32_t clear_n;
 };
 
-// Mode 0 packs the buckets densely (the export layout); modes 1 (a join's outputs: at most both buckets of the
-// pair), 2 (coarsening) and 3 (a permutation run's destinations) allocate resident segments, rounded up to
+// Modes 0 and 5 pack the buckets densely (the export layouts); modes 1 (a join's outputs: at most both buckets of the
+// pair), 2 (coarsening), 3 (a permutation run's destinations) and 4 allocate resident segments, rounded up to
 // kSegAlign rows.
 __device__ __forceinline__ uint64_t bucket_size(const OffsetsArgs& a, uint32_t b) {
     if (a.mode == 0) return a.len[b];
@@ -47,8 +48,11 @@ __device__ __forceinline__ uint64_t bucket_size(const OffsetsArgs& a, uint32_t b
         s = a.delta ? (uint64_t)a.len[b] + a.len[b ^ a.delta] : 2ull * a.len[b];
     } else if (a.mode == 3) {
         s = a.len[b];
+    } else if (a.mode == 4) {  // room for the partners a first layer in place adds to the bucket
+        s = (uint64_t)a.len[b] + a.len[b] / 4;
     } else {
         for (uint32_t e = 0; e < a.fold; ++e) s += a.len[b + e * a.coarse_buckets];
+        if (a.mode == 5) return s;
     }
     return (s + (kSegAlign - 1)) & ~(uint64_t)(kSegAlign - 1);
 }
@@ -1497,7 +1501,7 @@ hipError_t launch_bucket_offsets(hipStream_t st, const uint32_t* len, uint32_t n
     a.clear = clear;
     a.clear_n = clear ? clear_n : 0u;
     a.len = len;
-    a.out_n = mode == 2 ? coarse_buckets : num_buckets;
+    a.out_n = mode == 2 || mode == 5 ? coarse_buckets : num_buckets;
     a.mode = mode;
     a.delta = delta;
     a.coarse_buckets = coarse_buckets;
