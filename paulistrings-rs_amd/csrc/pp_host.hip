@@ -315,6 +315,7 @@ enum ScratchSlot {
     kScrFlags,
     kScrCounts,
     kScrGathered,
+    kScrWindow,      // a windowed selection's collected keys and positions
     kScrRank,
     kScrDest,        // a permutation run's per-row output bucket
     kScrRunCounts,   // its per-bucket destination counts
@@ -362,6 +363,8 @@ struct pp_sum {
     uint64_t topn_seed = 0;        // the last selection's boundary prefix, which seeds the next one's first pass
     bool topn_seed_valid = false;
     bool topn_seed_score = false;  // the seed is a score key (the learned pass), not a |c|^2 one
+    double topn_width = 0;         // the next windowed selection's half-width around the seed (0: none yet)
+    pp::WindowCounts* d_window = nullptr;
     uint64_t phys_len = 0;
     const uint8_t* pending_flags = nullptr;
     const float* pending_score = nullptr;  // the ranking score when the selection was by score
@@ -370,8 +373,9 @@ struct pp_sum {
     uint64_t tiles_cap = 0;
     unsigned long long* d_stats = nullptr;
     unsigned long long* h_stats = nullptr;  // pinned
-    // Two pinned, device-visible slots of kStatSlots words for the counters of layers queued ahead of them (lagged
-    // lengths), allocated on first use; the device address of the same memory; the small join's sequence number.
+    // Three pinned, device-visible slots of kStatSlots words, allocated on first use: two for the counters of layers
+    // queued ahead of them (lagged lengths), one for a windowed selection's answer; the device address of the same
+    // memory; the sequence number of the slots' last writer.
     unsigned long long* h_lag = nullptr;
     unsigned long long* d_lag_host = nullptr;
     unsigned long long lag_seq = 0;
@@ -505,6 +509,33 @@ pp_status read_stats(pp_sum* s) {
     PP_HIP(ctx, hipMemcpyAsync(s->h_stats, s->d_stats, kStatSlots * sizeof(unsigned long long), hipMemcpyDeviceToHost,
                                ctx->stream));
     PP_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    return PP_OK;
+}
+
+pp_status ensure_lag_slots(pp_sum* s) {
+    if (s->h_lag) return PP_OK;
+    if (hipHostMalloc((void**)&s->h_lag, 3 * kStatSlots * sizeof(unsigned long long),
+                      hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
+        (void)hipGetLastError();
+        s->h_lag = nullptr;
+        return fail(s->ctx, PP_ERR_OUT_OF_MEMORY, "pinned host allocation");
+    }
+    std::memset(s->h_lag, 0, 3 * kStatSlots * sizeof(unsigned long long));
+    PP_HIP(s->ctx, hipHostGetDevicePointer((void**)&s->d_lag_host, s->h_lag, 0));
+    return PP_OK;
+}
+
+// Wait on the host until a queued kernel has written `seq` to word 4 of its pinned slot, and after a long wait for the
+// stream itself (which reports a failed launch).
+pp_status wait_for_slot(pp_context* ctx, volatile const unsigned long long* h, unsigned long long seq,
+                        const char* never) {
+    const auto t0 = std::chrono::steady_clock::now();
+    while (h[4] != seq)
+        if (std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(200)) {
+            PP_HIP(ctx, hipStreamSynchronize(ctx->stream));
+            if (h[4] != seq) return fail(ctx, PP_ERR_DRIVER, never);
+            break;
+        }
     return PP_OK;
 }
 
@@ -2420,6 +2451,7 @@ pp_status pp_sum_free(pp_sum* s) {
     if (s->h_lag) (void)hipHostFree(s->h_lag);
     if (s->d_lag_counters) (void)hipFree(s->d_lag_counters);
     if (s->d_topn) (void)hipFree(s->d_topn);
+    if (s->d_window) (void)hipFree(s->d_window);
     if (s->d_redo) (void)hipFree(s->d_redo);
     if (s->d_score) (void)hipFree(s->d_score);
     if (s->d_hist) (void)hipFree(s->d_hist);
@@ -3089,13 +3121,7 @@ pp_status propagate_lagged(pp_sum* s, const RunPlanner& plan, const KeepProgram&
     pp_status st;
     for (hipEvent_t& e : ctx->lag_ev)
         if (!e) PP_HIP(ctx, hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    if (!s->h_lag) {
-        if (hipHostMalloc((void**)&s->h_lag, 2 * kStatSlots * sizeof(unsigned long long),
-                          hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess)
-            return fail(ctx, PP_ERR_OUT_OF_MEMORY, "pinned host allocation");
-        std::memset(s->h_lag, 0, 2 * kStatSlots * sizeof(unsigned long long));
-        PP_HIP(ctx, hipHostGetDevicePointer((void**)&s->d_lag_host, s->h_lag, 0));
-    }
+    if ((st = ensure_lag_slots(s)) != PP_OK) return st;
     if (!s->d_lag_counters &&
         (st = dev_alloc(ctx, (void**)&s->d_lag_counters, 8 * sizeof(unsigned long long))) != PP_OK)
         return st;
@@ -3131,17 +3157,9 @@ pp_status propagate_lagged(pp_sum* s, const RunPlanner& plan, const KeepProgram&
     auto read_oldest = [&]() -> pp_status {
         const uint32_t k = head;
         volatile const unsigned long long* h = s->h_lag + kStatSlots * k;
-        if (queued_seq[k]) {
-            // the next launch (a small join, or the publication at a drain) writes the slot, then the sequence
-            // number: wait for it on the host, and after a long wait for the stream itself (which reports a failed
-            // launch)
-            const auto t0 = std::chrono::steady_clock::now();
-            while (h[4] != queued_seq[k])
-                if (std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(200)) {
-                    PP_HIP(ctx, hipStreamSynchronize(ctx->stream));
-                    if (h[4] != queued_seq[k]) return fail(ctx, PP_ERR_DRIVER, "small join: counters never arrived");
-                    break;
-                }
+        if (queued_seq[k]) {  // the next launch (a small join, or the publication at a drain) writes the slot
+            const pp_status ws = wait_for_slot(ctx, h, queued_seq[k], "small join: counters never arrived");
+            if (ws != PP_OK) return ws;
         } else {
             PP_HIP(ctx, hipEventSynchronize(ctx->lag_ev[k]));
         }

@@ -102,6 +102,68 @@ struct TopnTieArgs {
     uint32_t buckets_per_block;  // at most kHistBucketsMax
 };
 
+// The windowed selection: a selection at a TopN cap falls near the one before, so one pass over the keys counts those at
+// or above a window around the last boundary and collects those inside it, and the rank is found among the collected
+// ones alone.  A boundary outside the window (or a window too full) is reported as missed and the radix passes run.
+constexpr uint32_t kWindowBins = 128;   // equal parts of the window, counted when a second launch narrows it
+constexpr uint32_t kWindowStage = 1024; // a scanning workgroup's collected keys, held in LDS
+constexpr uint32_t kWindowRank = 256;   // keys the last workgroup ranks by counting when their digits still differ
+constexpr uint32_t kWindowList = 2048;  // and at most (a run of equal keys cannot be told apart by digits)
+constexpr uint32_t kWindowTies = 1024;  // equal keys it puts into canonical order
+enum WindowStatus : uint32_t { kWindowMissed = 1, kWindowDone = 2, kWindowCrowded = 3 };
+
+// Workgroup w of the scan adds to part w % kWindowParts of the counters (a line of their own each) and collects into that
+// part of the arrays, and to copy w % kWindowCopies of the bins: atomics on one line follow one another every ~12 ns
+// whatever word they hit, so 2048 workgroups on one line are 25 us per counter.
+constexpr uint32_t kWindowParts = 32;
+constexpr uint32_t kWindowCopies = 128;
+
+struct WindowCounts {  // zero before the scan; the last launch clears it
+    struct alignas(128) Part {
+        unsigned long long above_finite;  // keys at or above the window, and in the high word keys that are no NaN
+        unsigned long long count;         // keys inside (collected up to the part's room)
+        unsigned long long overflow;      // a workgroup collected more than it holds
+    } part[kWindowParts];
+    unsigned long long narrowed;        // keys of the boundary's bin (the second launch)
+    unsigned long long narrowed_above;  // keys above that bin
+    uint32_t bins[kWindowCopies][kWindowBins];
+};
+
+template <int W, typename T>
+struct WindowArgs {
+    const uint64_t* x;
+    const uint64_t* z;
+    const T* c;
+    const float* score;  // as in TopnHistArgs
+    uint64_t cap;
+    const uint64_t* start;
+    const uint32_t* len;
+    uint32_t num_buckets;
+    uint32_t buckets_per_block;
+    const uint64_t* rows;
+    int32_t ref_bits;
+    uint64_t n;        // terms to keep
+    uint64_t lo, hi;   // the window's keys: lo <= u < hi
+    int32_t bin_shift; // (u - lo) >> bin_shift < kWindowBins
+    uint32_t narrow;   // the second launch runs
+    WindowCounts* counts;
+    uint64_t* key;     // collected keys and their positions, kWindowParts parts of `room`; then the narrowed ones
+    uint64_t* pos;
+    uint64_t* key2;
+    uint64_t* pos2;
+    uint64_t room;
+    uint8_t* flags;    // per column position: written at equal keys when only some of them stay
+    TopnState* state;
+    // pinned: [0] WindowStatus, [1] boundary key, [2] the fullest part's keys (~0 when a workgroup held too many),
+    // [3] finite keys, [5] 1 when flags are needed, [6] the boundary's bin when the window was too full but counted it
+    // (kWindowCrowded), then [4] = seq
+    unsigned long long* host;
+    unsigned long long seq;
+};
+// Two launches, or three with a.narrow.
+template <int W, typename T>
+hipError_t launch_topn_window(hipStream_t st, const WindowArgs<W, T>& a);
+
 template <int W, typename T>
 struct TopnRetainArgs {
     uint64_t* x;

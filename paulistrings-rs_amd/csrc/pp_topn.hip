@@ -144,12 +144,13 @@ __device__ __forceinline__ uint32_t list_rows(const uint64_t* start, const uint3
     return total;
 }
 
-// Column positions of list rows g0 + q * kBlock (q < 4) that exist; j is the caller's bucket cursor (rows only move
+// Column positions of list rows g0 + q * kBlock (q < N) that exist; j is the caller's bucket cursor (rows only move
 // forward, so it does too).
+template <int N>
 __device__ __forceinline__ void list_positions(const RowList& l, uint32_t total, uint32_t g0, uint32_t& j,
-                                               uint64_t (&pos)[4], bool (&in)[4]) {
+                                               uint64_t (&pos)[N], bool (&in)[N]) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
+    for (int q = 0; q < N; ++q) {
         const uint32_t g = g0 + (uint32_t)q * kBlock;
         in[q] = g < total;
         if (in[q]) {
@@ -451,6 +452,396 @@ __global__ void __launch_bounds__(kBlock) k_topn_flags_batch(const TopnFlagItem*
     for (uint64_t j = threadIdx.x; j < it.ties; j += kBlock) it.flags[it.pos[j]] = j < it.kept ? 1 : 0;
 }
 
+// ---- the windowed selection ---------------------------------------------------------------------------------
+
+// The keys of a workgroup's buckets against the window: those at or above it and those that are numbers are counted,
+// those inside collected.  The coefficients' (or scores') bytes, and above 10^7 keys the merging of the bins' counts,
+// bound it: 8 us at 2^20 f64 terms and 48 at 2^24 (72 with twice the bins, 164 with one line of counters).  With the
+// narrowing and the finish a selection is 26 and 84 us of kernels and one wait of the host, where the radix passes, the
+// gather of the boundary bin and their selects were 50-60 and 170 with two or three synchronizations.
+template <int W, typename T>
+__global__ void __launch_bounds__(kBlock) k_window_scan(const WindowArgs<W, T> a) {
+    __shared__ RowList list;
+    __shared__ uint64_t su[kWindowStage], sp[kWindowStage];
+    __shared__ uint32_t bins[kWindowBins];
+    __shared__ uint32_t collected, totals[2];
+    __shared__ unsigned long long base;
+    if (threadIdx.x < 2) totals[threadIdx.x] = 0u;
+    if (threadIdx.x == 2) collected = 0u;
+    if (threadIdx.x < kWindowBins) bins[threadIdx.x] = 0u;
+    const uint32_t b_lo = blockIdx.x * a.buckets_per_block;
+    const uint32_t nb = min(a.num_buckets, b_lo + a.buckets_per_block) - b_lo;  // <= kHistBucketsMax
+    const uint32_t total = list_rows(a.start, a.len, b_lo, nb, list);
+    uint32_t above = 0, finite = 0, j = 0;
+    for (uint32_t g0 = threadIdx.x; g0 < total; g0 += 8 * kBlock) {
+        uint64_t pos[8];
+        bool in[8];
+        list_positions(list, total, g0, j, pos, in);
+        uint64_t u[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q)
+            if (in[q]) u[q] = rank_bits<T>(a.c, a.score, pos[q]);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            if (!in[q] || (!a.score && is_nan_bits(u[q]))) continue;
+            ++finite;
+            if (u[q] >= a.hi) {
+                ++above;
+            } else if (u[q] >= a.lo) {
+                const uint32_t slot = atomicAdd(&collected, 1u);
+                if (slot < kWindowStage) {
+                    su[slot] = u[q];
+                    sp[slot] = pos[q];
+                }
+                if (a.narrow) atomicAdd(&bins[(uint32_t)((u[q] - a.lo) >> a.bin_shift)], 1u);
+            }
+        }
+    }
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) {
+        above += (uint32_t)__shfl_xor((int)above, d, 64);
+        finite += (uint32_t)__shfl_xor((int)finite, d, 64);
+    }
+    if (lane_id() == 0) {
+        atomicAdd(&totals[0], above);
+        atomicAdd(&totals[1], finite);
+    }
+    __syncthreads();
+    const uint32_t part = blockIdx.x % kWindowParts;
+    if (threadIdx.x == 0) {
+        WindowCounts::Part& p = a.counts->part[part];
+        base = collected ? atomicAdd(&p.count, (unsigned long long)collected) : 0ull;
+        if (totals[1]) atomicAdd(&p.above_finite, (unsigned long long)totals[0] | ((unsigned long long)totals[1] << 32));
+        if (collected > kWindowStage) atomicOr(&p.overflow, 1ull);
+    }
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < min(collected, kWindowStage); i += kBlock)
+        if (base + i < a.room) {
+            a.key[part * a.room + base + i] = su[i];
+            a.pos[part * a.room + base + i] = sp[i];
+        }
+    if (a.narrow && threadIdx.x < kWindowBins && bins[threadIdx.x])
+        atomicAdd(&a.counts->bins[blockIdx.x % kWindowCopies][threadIdx.x], bins[threadIdx.x]);
+}
+
+// The scan's counters of all parts, and the collected keys as one list: entry i of it lies at at(i).  Every thread of
+// the workgroup calls read (one barrier); nothing is kept from a part with more keys than room.
+struct WindowTotals {
+    uint64_t first[kWindowParts + 1];
+    uint64_t above, finite, fullest;
+
+    __device__ __forceinline__ void read(const WindowCounts& w) {  // into LDS
+        if (threadIdx.x < 64) {
+            const uint32_t l = threadIdx.x & (kWindowParts - 1);
+            const WindowCounts::Part p = w.part[l];
+            uint64_t n = p.count, up = p.above_finite & 0xFFFFFFFFull, f = p.above_finite >> 32;
+            uint64_t most = p.overflow ? ~0ull : n;
+#pragma unroll
+            for (int d = 1; d < (int)kWindowParts; d <<= 1) {
+                const uint64_t o = __shfl_up(n, d, kWindowParts);
+                if (l >= (uint32_t)d) n += o;
+                up += __shfl_xor(up, d, kWindowParts);
+                f += __shfl_xor(f, d, kWindowParts);
+                const uint64_t m = __shfl_xor(most, d, kWindowParts);
+                most = m > most ? m : most;
+            }
+            if (threadIdx.x < kWindowParts) first[l + 1] = n;
+            if (threadIdx.x == 0) {
+                first[0] = 0;
+                above = up;
+                finite = f;
+                fullest = most;
+            }
+        }
+        __syncthreads();
+    }
+    // whether the n-th key is inside the window, and every key inside collected
+    __device__ __forceinline__ bool inside(uint64_t n) const { return above < n && above + first[kWindowParts] >= n; }
+    __device__ __forceinline__ bool holds(uint64_t n, uint64_t room) const { return fullest <= room && inside(n); }
+    __device__ __forceinline__ uint64_t at(uint64_t i, uint64_t room) const {
+        uint32_t p = 0;
+#pragma unroll
+        for (uint32_t half = kWindowParts / 2; half > 0; half >>= 1)
+            if (first[p + half] <= i) p += half;
+        return p * room + (i - first[p]);
+    }
+};
+
+// The bin (of BINS in ascending order, hist[bin]) that holds the k-th key from the top, the keys above it and its own,
+// by a workgroup of BLOCK threads; k is at least 1 and at most the bins' total.  Every thread gets the answer.
+template <uint32_t BINS, uint32_t BLOCK>
+__device__ __forceinline__ void window_bin(const uint32_t* hist, uint64_t k, uint64_t* part, uint64_t (&answer)[3]) {
+    constexpr uint32_t PER = (BINS + BLOCK - 1) / BLOCK;  // the threads past the last bin hold none
+    static_assert(PER * BLOCK == BINS || PER == 1, "bins split evenly over the workgroup");
+    uint64_t mine = 0;
+#pragma unroll
+    for (uint32_t q = 0; q < PER; ++q)
+        if (threadIdx.x * PER + q < BINS) mine += hist[threadIdx.x * PER + q];
+    uint64_t suffix = mine;  // this lane's bins and the higher lanes' of its wave
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint64_t o = __shfl_down(suffix, d, 64);
+        if (lane_id() + (uint32_t)d < 64u) suffix += o;
+    }
+    if (lane_id() == 0) part[wave_id()] = suffix;
+    __syncthreads();
+    uint64_t above = suffix - mine;
+    for (uint32_t w = wave_id() + 1; w < BLOCK / 64; ++w) above += part[w];
+    if (above < k && above + mine >= k) {
+        for (uint32_t q = PER; q-- > 0;) {
+            const uint64_t h = hist[threadIdx.x * PER + q];
+            if (above + h >= k) {
+                part[BLOCK / 64] = threadIdx.x * PER + q;
+                part[BLOCK / 64 + 1] = above;
+                part[BLOCK / 64 + 2] = h;
+                break;
+            }
+            above += h;
+        }
+    }
+    __syncthreads();
+    for (int i = 0; i < 3; ++i) answer[i] = part[BLOCK / 64 + i];
+    __syncthreads();
+}
+
+// The copies of the scan's bins summed into hist (zero before), by a workgroup of BLOCK threads.
+template <uint32_t BLOCK>
+__device__ __forceinline__ void window_bins_sum(const WindowCounts& w, uint32_t* hist) {
+    static_assert(BLOCK % kWindowBins == 0, "a group of threads per bin");
+    uint32_t sum = 0;
+#pragma unroll 8
+    for (uint32_t c = threadIdx.x / kWindowBins; c < kWindowCopies; c += BLOCK / kWindowBins)
+        sum += w.bins[c][threadIdx.x % kWindowBins];
+    atomicAdd(&hist[threadIdx.x % kWindowBins], sum);
+    __syncthreads();
+}
+
+// The collected keys of the boundary's bin, for a sum whose window holds too many for one workgroup.
+template <int W, typename T>
+__global__ void __launch_bounds__(kBlock) k_window_narrow(const WindowArgs<W, T> a) {
+    __shared__ uint64_t part[kWaves + 3];
+    __shared__ uint32_t hist[kWindowBins];
+    __shared__ uint64_t su[kWindowStage], sp[kWindowStage];
+    __shared__ uint32_t collected;
+    __shared__ unsigned long long base;
+    __shared__ WindowTotals t;
+    WindowCounts& w = *a.counts;
+    if (threadIdx.x < kWindowBins) hist[threadIdx.x] = 0u;
+    if (threadIdx.x == 0) collected = 0u;
+    t.read(w);  // complete at this launch's start
+    if (!t.holds(a.n, a.room)) return;  // uniform
+    window_bins_sum<kBlock>(w, hist);
+    uint64_t bin[3];
+    window_bin<kWindowBins, kBlock>(hist, a.n - t.above, part, bin);
+    if (blockIdx.x == 0 && threadIdx.x == 0) w.narrowed_above = t.above + bin[1];
+    const uint64_t m = t.first[kWindowParts], stride = (uint64_t)gridDim.x * kBlock;
+    for (uint64_t i0 = (uint64_t)blockIdx.x * kBlock; i0 < m; i0 += stride) {  // uniform
+        const uint64_t i = i0 + threadIdx.x;
+        if (i < m) {
+            const uint64_t at = t.at(i, a.room), u = a.key[at];
+            if (((u - a.lo) >> a.bin_shift) == bin[0]) {
+                const uint32_t slot = atomicAdd(&collected, 1u);
+                su[slot] = u;
+                sp[slot] = a.pos[at];
+            }
+        }
+        __syncthreads();
+        const uint32_t held = collected;
+        if (held > kWindowStage - kBlock || i0 + stride >= m) {  // uniform: the next step's keys may not fit, or the end
+            if (threadIdx.x == 0) base = held ? atomicAdd(&w.narrowed, (unsigned long long)held) : 0ull;
+            __syncthreads();
+            for (uint32_t q = threadIdx.x; q < held; q += kBlock) {
+                a.key2[base + q] = su[q];
+                a.pos2[base + q] = sp[q];
+            }
+            __syncthreads();
+            if (threadIdx.x == 0) collected = 0u;
+        }
+        __syncthreads();
+    }
+}
+
+// The n-th key among the collected (or narrowed) ones, by one workgroup: 11-bit digits of the window until at most
+// kWindowRank keys are left or they are equal, those ranked by counting, and the keys equal to the boundary put into canonical order when
+// only some of them stay.  Then the state the next layer reads, the answer to the host, and the counts cleared.
+constexpr uint32_t kFinishBlock = 1024;
+template <int W, typename T>
+__global__ void __launch_bounds__(kFinishBlock) k_window_finish(const WindowArgs<W, T> a) {
+    constexpr uint32_t kDigits = 2048;
+    __shared__ uint32_t hist[kDigits];
+    __shared__ uint64_t part[kFinishBlock / 64 + 3];
+    __shared__ uint64_t su[kWindowList], sp[kWindowList];
+    __shared__ uint64_t tx[W][kWindowTies], tz[W][kWindowTies], tp[kWindowTies];
+    __shared__ uint32_t tb[kWindowTies];
+    __shared__ uint32_t held, ties;
+    __shared__ uint64_t found[3];  // the boundary key, the list's keys above it, the keys equal to it
+    __shared__ WindowTotals t;
+    const uint32_t tid = threadIdx.x;
+    WindowCounts& w = *a.counts;
+    t.read(w);
+    const bool keep_all = t.finite <= a.n;
+    bool done = !keep_all && t.holds(a.n, a.room);  // uniform
+    uint64_t boundary = 0, stay = 0;
+    uint32_t equal = 0;
+    if (done) {
+        const uint64_t m = a.narrow ? w.narrowed : t.first[kWindowParts];
+        const uint64_t* const key = a.narrow ? a.key2 : a.key;
+        const uint64_t* const pos = a.narrow ? a.pos2 : a.pos;
+        auto at = [&](uint64_t i) { return a.narrow ? i : t.at(i, a.room); };
+        uint64_t k = a.n - (a.narrow ? w.narrowed_above : t.above);  // 1 <= k <= m
+        uint64_t base = a.lo, left = m;
+        int shift = 64;  // the keys sought lie in [base, base + 2^shift)
+        if (m > kWindowRank) {
+            shift = 64 - __builtin_clzll(a.hi - a.lo);
+            do {
+                const int sh = max(shift - 11, 0);
+                for (uint32_t i = tid; i < kDigits; i += kFinishBlock) hist[i] = 0u;
+                __syncthreads();
+                for (uint64_t i0 = tid; i0 < m; i0 += 4 * kFinishBlock) {  // four loads in flight per thread
+                    uint64_t r[4];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        r[q] = i0 + q * kFinishBlock < m ? key[at(i0 + q * kFinishBlock)] - base : ~0ull;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)  // a smaller key wraps far past the range
+                        if ((r[q] >> shift) == 0) atomicAdd(&hist[r[q] >> sh], 1u);
+                }
+                __syncthreads();
+                uint64_t bin[3];
+                window_bin<kDigits, kFinishBlock>(hist, k, part, bin);
+                base += bin[0] << sh;
+                k -= bin[1];
+                left = bin[2];
+                shift = sh;
+            } while (left > kWindowRank && shift > 0);
+        }
+        done = left <= kWindowList;  // else more equal keys than the list holds
+        if (done) {
+            if (tid == 0) {
+                held = 0u;
+                ties = 0u;
+            }
+            __syncthreads();
+            for (uint64_t i0 = tid; i0 < m; i0 += 4 * kFinishBlock) {
+                uint64_t u[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (i0 + q * kFinishBlock < m) u[q] = key[at(i0 + q * kFinishBlock)];
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (i0 + q * kFinishBlock < m && (shift == 64 || ((u[q] - base) >> shift) == 0)) {
+                        const uint32_t slot = atomicAdd(&held, 1u);
+                        su[slot] = u[q];
+                        sp[slot] = pos[at(i0 + q * kFinishBlock)];
+                    }
+            }
+            __syncthreads();
+            const uint32_t n = held;  // = left
+            for (uint32_t i = tid; i < n; i += kFinishBlock) {
+                const uint64_t u = su[i];
+                uint32_t greater = 0, same = 0;
+                for (uint32_t q = 0; q < n; ++q) {
+                    greater += su[q] > u;
+                    same += su[q] == u;
+                }
+                if (greater < k && greater + same >= k) {  // every row equal to the boundary writes the same
+                    found[0] = u;
+                    found[1] = greater;
+                    found[2] = same;
+                }
+            }
+            __syncthreads();
+            boundary = found[0];
+            stay = k - found[1];
+            equal = (uint32_t)found[2];
+            if (stay < equal) {
+                done = equal <= kWindowTies;
+                if (done) {
+                    for (uint32_t i = tid; i < n; i += kFinishBlock) {
+                        if (su[i] != boundary) continue;
+                        const uint32_t e = atomicAdd(&ties, 1u);
+                        const Key<W> kk = load_key<W>(a.x, a.z, a.cap, sp[i]);
+#pragma unroll
+                        for (int v = 0; v < W; ++v) {
+                            tx[v][e] = kk.x[v];
+                            tz[v][e] = kk.z[v];
+                        }
+                        tb[e] = bucket_of<W>(kk, a.rows, a.ref_bits);
+                        tp[e] = sp[i];
+                    }
+                    __syncthreads();
+                    for (uint32_t i = tid; i < equal; i += kFinishBlock) {
+                        uint32_t before = 0;
+                        for (uint32_t q = 0; q < equal; ++q) {
+                            int order = tb[q] < tb[i] ? -1 : tb[q] > tb[i] ? 1 : 0;
+#pragma unroll
+                            for (int v = 0; v < W; ++v)
+                                if (order == 0) order = tx[v][q] < tx[v][i] ? -1 : tx[v][q] > tx[v][i] ? 1 : 0;
+#pragma unroll
+                            for (int v = 0; v < W; ++v)
+                                if (order == 0) order = tz[v][q] < tz[v][i] ? -1 : tz[v][q] > tz[v][i] ? 1 : 0;
+                            before += order < 0;
+                        }
+                        a.flags[tp[i]] = before < stay ? 1 : 0;
+                    }
+                }
+            }
+        }
+    }
+    const bool crowded = !done && !keep_all && a.narrow && t.fullest > a.room && t.inside(a.n);  // uniform
+    uint64_t bin[3] = {0, 0, 0};
+    if (crowded) {
+        if (tid < kWindowBins) hist[tid] = 0u;
+        __syncthreads();
+        window_bins_sum<kFinishBlock>(w, hist);
+        window_bin<kWindowBins, kFinishBlock>(hist, a.n - t.above, part, bin);
+    }
+    __syncthreads();  // the counts are no longer read
+    if (a.narrow)
+        for (uint32_t i = tid; i < kWindowCopies * kWindowBins / 4; i += kFinishBlock)
+            reinterpret_cast<uint4*>(&w.bins[0][0])[i] = make_uint4(0u, 0u, 0u, 0u);
+    if (tid < kWindowParts) {
+        w.part[tid].above_finite = 0;
+        w.part[tid].count = 0;
+        w.part[tid].overflow = 0;
+    }
+    if (tid == 0) {
+        w.narrowed = 0;
+        w.narrowed_above = 0;
+        if (done || keep_all) {
+            TopnState& s = *a.state;
+            s.prefix = boundary;
+            s.mask = ~0ull;
+            s.k = stay;
+            s.above = a.n - stay;
+            s.finite = t.finite;
+            s.ties = equal;
+            s.keep_all_finite = keep_all ? 1 : 0;
+        }
+        volatile unsigned long long* h = a.host;  // fine-grained host memory: the stores bypass the L2
+        h[0] = done || keep_all ? kWindowDone : crowded ? kWindowCrowded : kWindowMissed;
+        h[1] = keep_all ? 0ull : boundary;
+        h[2] = t.fullest;
+        h[3] = t.finite;
+        h[5] = done && stay < equal ? 1 : 0;
+        h[6] = bin[0];
+        __builtin_amdgcn_s_waitcnt(0);  // the slot's words land before its sequence number
+        h[4] = a.seq;
+    }
+}
+
+template <int W, typename T>
+hipError_t launch_topn_window(hipStream_t st, const WindowArgs<W, T>& a) {
+    if (a.buckets_per_block == 0 || a.buckets_per_block > kHistBucketsMax || a.hi <= a.lo || a.n == 0 ||
+        a.hi - a.lo >= (1ull << 62) || a.bin_shift < 0 || a.bin_shift > 63 || ((a.hi - a.lo - 1) >> a.bin_shift) >= kWindowBins)
+        return hipErrorInvalidValue;
+    const uint32_t blocks = (a.num_buckets + a.buckets_per_block - 1) / a.buckets_per_block;
+    hipLaunchKernelGGL((k_window_scan<W, T>), dim3(blocks), dim3(kBlock), 0, st, a);
+    if (a.narrow) hipLaunchKernelGGL((k_window_narrow<W, T>), dim3(256), dim3(kBlock), 0, st, a);
+    hipLaunchKernelGGL((k_window_finish<W, T>), dim3(1), dim3(kFinishBlock), 0, st, a);
+    return hipGetLastError();
+}
+
 // ---- ApproxTopN ---------------------------------------------------------------------------------------------
 
 // octave(norm_sqr) = norm_sqr.to_bits() >> 52 (builtin.rs:276-279).  A NaN of either sign counts in octave 2047,
@@ -687,6 +1078,7 @@ template hipError_t launch_topn_hist_seeded<float>(hipStream_t, const TopnHistAr
 template hipError_t launch_octave_hist<double>(hipStream_t, const OctaveHistArgs<double>&, uint32_t);
 template hipError_t launch_octave_hist<float>(hipStream_t, const OctaveHistArgs<float>&, uint32_t);
 #define PP_TOPN_INSTANTIATE(W, T)                                                                       \
+    template hipError_t launch_topn_window<W, T>(hipStream_t, const WindowArgs<W, T>&);                 \
     template hipError_t launch_topn_gather_ties<W, T>(hipStream_t, const TopnTieArgs<W, T>&, uint32_t); \
     template hipError_t launch_topn_gather_batch<W, T>(hipStream_t, const TopnTieArgs<W, T>*, const uint32_t*, \
                                                        uint32_t, uint32_t);                               \
