@@ -1356,10 +1356,16 @@ pp_status layer_in_place(pp_sum* s, const Prepared& p, const KeepProgram& keep) 
     uint32_t lcap = delta ? 2u * s->max_bucket : s->max_bucket;
     lcap = std::max<uint32_t>(64, (lcap + 63) & ~63u);
     if (lcap > kMaxPairRows) lcap = kMaxPairRows;
-    // a generator anticommutes with a fraction of a bucket: 256 staged rows leave room for six workgroups per CU
-    const uint32_t scap = std::min<uint32_t>(ctx->tuning.stage_rows ? join_stage_rows(ctx->tuning.stage_rows, lcap)
-                                                                     : 256u,
-                                             lcap);
+    // a generator anticommutes with a fraction of a bucket: the first launch stages at most a row per thread
+    const uint32_t scap = std::min<uint32_t>({ctx->tuning.stage_rows ? join_stage_rows(ctx->tuning.stage_rows, lcap)
+                                                                     : (uint32_t)kBlock,
+                                             (uint32_t)kBlock, lcap});
+    // of every row the first launch reads the words the generator's commutation test asks for, or all of them when the
+    // keep program counts weights
+    uint32_t need = 0;
+    for (uint32_t w = 0; w < s->W; ++w) need |= (p.gz[w] ? 1u : 0u) << (2 * w) | (p.gx[w] ? 2u : 0u) << (2 * w);
+    for (int i = 0; i < keep.n; ++i)
+        if (keep.op[i] == KEEP_WEIGHT) need = ~0u;
     auto table_bits_for = [](uint32_t rows) {
         uint32_t b = 1;
         while ((1u << b) < 2u * rows) ++b;
@@ -1417,6 +1423,7 @@ pp_status layer_in_place(pp_sum* s, const Prepared& p, const KeepProgram& keep) 
             a.redo_count = s->d_stats + 4;
             a.redo_mode = redo_mode;
             a.count_totals = count_in_join ? 1u : 0u;
+            a.need = need;
             a.compact = in_place_compaction() ? 1u : 0u;
             if (s->pending_topn) {  // the layer reads its input through the selection
                 a.filter = s->d_topn;

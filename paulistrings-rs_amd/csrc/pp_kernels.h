@@ -101,6 +101,7 @@ struct InplaceArgs {
     unsigned long long* redo_count;
     uint32_t redo_mode;
     uint32_t count_totals;
+    uint32_t need;     // key words phase A reads of every row: bit 2w x[w], bit 2w + 1 z[w]
     uint32_t compact;  // a side left with more holes than new rows closes them in place (else the pair moves)
     // a TopN selection the layer reads its input through (the filtered launch): rows it drops are holes
     const TopnState* filter;

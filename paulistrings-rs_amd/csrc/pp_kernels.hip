@@ -714,16 +714,17 @@ size_t inplace_lds_bytes(uint32_t scap, uint32_t tcap_bits) {
            2 * (size_t)kInplaceHoles * 2;
 }
 
-// A side's holes as a bitmap of its rows (kInplaceHoles bits) with the holes before each word (pre[w], pre[32] all):
-// the k-th hole in ascending order, and the holes below row p, each in a few steps.
+// A side's holes as a bitmap of its rows (WORDS words) with the holes before each word (pre[w], pre[WORDS] all): the
+// k-th hole in ascending order, and the holes below row p, each in a few steps.
 constexpr uint32_t kHoleWords = kInplaceHoles / 32;
 __device__ __forceinline__ uint32_t holes_below(const uint32_t* bits, const uint16_t* pre, uint32_t p) {
     const uint32_t w = p >> 5, b = p & 31u;
     return pre[w] + (b ? (uint32_t)__popc(bits[w] & ((1u << b) - 1u)) : 0u);
 }
 
+template <uint32_t WORDS>
 __device__ __forceinline__ uint32_t kth_hole(const uint32_t* bits, const uint16_t* pre, uint32_t k) {
-    uint32_t lo = 0, hi = kHoleWords;  // the word w with pre[w] <= k < pre[w + 1]
+    uint32_t lo = 0, hi = WORDS;  // the word w with pre[w] <= k < pre[w + 1]
     while (hi - lo > 1) {
         const uint32_t mid = (lo + hi) >> 1;
         if (pre[mid] <= k) lo = mid;
@@ -743,7 +744,294 @@ __device__ __forceinline__ uint32_t kth_hole(const uint32_t* bits, const uint16_
     return lo * 32u + pos;
 }
 
-template <int W, typename T, bool REDO, bool FILTER>
+// The first launch: a workgroup per pair, one staged row per thread.  Most rows commute with the generator, and a row
+// that commutes and stays is not written, so phase A reads of every row only the words the anticommutation test (and the
+// keep program, when it counts weights) asks for and the coefficient; the pair's flags become ballots whose counts meet
+// in LDS at one barrier.  Phase A2 then reads the whole keys of the anticommuting rows, a row per thread, all lanes busy.
+// A thread keeps its staged row, decision and new coefficients in registers; LDS holds what partners look up (key,
+// coefficient, table) and the holes: 15 KiB, eight workgroups a compute unit where the LDS of the redo launch allows six
+// at 256 rows.  Order within the pair decides every position, so a layer leaves the same layout on every run.
+constexpr uint32_t kPairHoles = 512;  // rows of a side at most: settling refines a bucket past half a pair's rows
+template <int W, typename T, bool FILTER>
+__global__ void __launch_bounds__(kBlock) k_rotation_pair(const InplaceArgs<W, T> a) {
+    constexpr uint32_t kWords = kPairHoles / 32;
+    constexpr uint32_t kChunks = kPairRowsMax / kBlock;
+    constexpr uint32_t kTableBits = 9;  // twice the staged rows
+    static_assert((1u << kTableBits) == 2 * kBlock, "table load at most 1/2");
+    __shared__ uint64_t Lx[W][kBlock], Lz[W][kBlock];
+    __shared__ T Lc[kBlock];
+    __shared__ uint32_t table[1u << kTableBits];
+    __shared__ uint16_t Lrow[kBlock];
+    __shared__ uint16_t holes[2][kPairHoles];
+    __shared__ uint32_t hbits[2][kWords];
+    __shared__ uint16_t hpre[2][kWords + 1];
+    __shared__ uint64_t counts[kChunks * kWaves];
+    __shared__ uint32_t scan_scratch[4 * kWaves];
+    const uint32_t tid = threadIdx.x;
+    const bool pair = a.delta != 0;
+    const uint32_t p = blockIdx.x;
+    uint32_t b0, b1;
+    if (pair) {
+        const uint32_t lo = p & ((1u << a.hb) - 1u);
+        b0 = ((p >> a.hb) << (a.hb + 1u)) | lo;
+        b1 = b0 ^ a.delta;
+    } else {
+        b0 = b1 = p;
+    }
+    const uint32_t n0 = a.len[b0], n1 = pair ? a.len[b1] : 0u;
+    const uint64_t s0 = a.start[b0], s1 = a.start[b1];
+    const uint32_t cap0 = a.bcap[b0], cap1 = a.bcap[b1];
+    const uint32_t n = n0 + n1;
+    // leave the pair untouched for the redo launch; its move may take `rows` rows
+    auto queue = [&](uint32_t rows) {
+        if (tid == 0) {
+            a.redo[atomicAdd(a.redo_count, 1ull)] = p;
+            atomicAdd(&a.stats[7], (unsigned long long)rows);
+        }
+    };
+    if (n0 > kPairHoles || n1 > kPairHoles) {  // uniform
+        queue(2u * moved_segment_rows(n));
+        return;
+    }
+    Key<W> g;
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+        g.x[w] = a.gx[w];
+        g.z[w] = a.gz[w];
+    }
+    const uint32_t supp = support_words<W>(g);
+    TopnState fs{};
+    if constexpr (FILTER) fs = *a.filter;
+    auto selected = [&](uint64_t i, T c) -> bool {
+        if constexpr (!FILTER) {
+            return true;
+        } else {
+            const uint64_t u = a.filter_score ? score_bits(a.filter_score[i]) : magnitude_bits<T>(c);
+            return topn_keeps(fs, u, !a.filter_score && is_nan_bits(u), a.filter_flags, i);
+        }
+    };
+    auto column_row = [&](uint32_t r) -> uint64_t { return r >= n0 ? s1 + (r - n0) : s0 + r; };
+    // ---- phase A: each row's flags, every chunk's loads in flight; no global write ----
+    uint64_t hole_mask[kChunks], anti_mask[kChunks];
+    {
+        Key<W> k[kChunks];
+        T c[kChunks];
+#pragma unroll
+        for (uint32_t q = 0; q < kChunks; ++q) {
+            const uint32_t r = q * kBlock + tid;
+            if (r < n) {
+                const uint64_t row = column_row(r);
+#pragma unroll
+                for (int w = 0; w < W; ++w) {  // uniform tests
+                    k[q].x[w] = (a.need >> (2 * w)) & 1u ? a.x[w * a.cap + row] : 0ull;
+                    k[q].z[w] = (a.need >> (2 * w + 1)) & 1u ? a.z[w * a.cap + row] : 0ull;
+                }
+                c[q] = a.c[row];
+            }
+        }
+#pragma unroll
+        for (uint32_t q = 0; q < kChunks; ++q) {
+            const uint32_t base = q * kBlock, r = base + tid;
+            hole_mask[q] = anti_mask[q] = 0;
+            if (base >= n) continue;  // uniform
+            bool anti = false, hole = false;
+            if (r < n) {
+                const bool valid = selected(column_row(r), c[q]);
+                anti = valid && anticommutes_on<W>(k[q], g, supp);
+                hole = !anti && !(valid && survives<W, T>(a.keep, k[q], c[q]));
+            }
+            const uint64_t hm = __ballot(hole), am = __ballot(anti);
+            hole_mask[q] = hm;
+            anti_mask[q] = am;
+            if (lane_id() == 0) {
+                const uint32_t first = base + wave_id() * 64u;  // rows [first, first + split) are side 0's
+                const uint32_t split = first >= n0 ? 0u : min(n0 - first, 64u);
+                const uint64_t side0 = split == 64u ? ~0ull : (1ull << split) - 1ull;
+                counts[q * kWaves + wave_id()] = (uint64_t)__popcll(hm & side0) |
+                                                        ((uint64_t)__popcll(hm & ~side0) << 16) |
+                                                        ((uint64_t)__popcll(am) << 32);
+            }
+        }
+    }
+    for (uint32_t i = tid; i < (1u << kTableBits); i += kBlock) table[i] = 0u;
+    if (tid < 2 * kWords) (&hbits[0][0])[tid] = 0u;
+    __syncthreads();
+    const uint32_t entries = ((n + kBlock - 1) / kBlock) * kWaves;
+    uint64_t total = 0;
+    for (uint32_t e = 0; e < entries; ++e) total += counts[e];
+    uint32_t hc0 = (uint32_t)total & 0xFFFFu, hc1 = (uint32_t)(total >> 16) & 0xFFFFu;
+    const uint32_t nl = (uint32_t)(total >> 32);
+    if (nl > a.scap) {  // uniform: a.scap is at most kBlock
+        queue(2u * moved_segment_rows(n));  // a side's rows after the layer are at most the pair's
+        return;
+    }
+    {
+        uint64_t before = 0;
+        uint32_t e = 0;
+#pragma unroll
+        for (uint32_t q = 0; q < kChunks; ++q) {
+            if (q * kBlock >= n) break;  // uniform
+            for (; e < q * kWaves + wave_id(); ++e) before += counts[e];
+            const uint32_t r = q * kBlock + tid;
+            const uint64_t bit = 1ull << lane_id(), lt = bit - 1ull;
+            if (anti_mask[q] & bit)
+                Lrow[(uint32_t)(before >> 32) + (uint32_t)__popcll(anti_mask[q] & lt)] = (uint16_t)r;
+            if (hole_mask[q] & bit) {
+                const uint32_t first = r - lane_id();
+                const uint32_t split = first >= n0 ? 0u : min(n0 - first, 64u);
+                const uint64_t side0 = split == 64u ? ~0ull : (1ull << split) - 1ull;
+                const bool j = r >= n0;
+                const uint32_t idx = j ? r - n0 : r;
+                const uint32_t at = (uint32_t)(j ? before >> 16 : before) & 0xFFFFu;
+                holes[j][at + (uint32_t)__popcll(hole_mask[q] & (j ? ~side0 : side0) & lt)] = (uint16_t)idx;
+                if (a.compact) atomicOr(&hbits[j][idx >> 5], 1u << (idx & 31u));
+            }
+        }
+    }
+    __syncthreads();
+    // ---- phase A2: the staged rows' keys ----
+    const bool valid = tid < nl;
+    Key<W> kk{};
+    T cc = T(0);
+    uint32_t jj = 0, idx = 0, fold = 0;
+    if (valid) {
+        const uint32_t r = Lrow[tid];
+        jj = r >= n0 ? 1u : 0u;
+        idx = jj ? r - n0 : r;
+        const uint64_t row = column_row(r);
+        kk = load_key<W>(a.x, a.z, a.cap, row);
+        cc = a.c[row];
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            Lx[w][tid] = kk.x[w];
+            Lz[w][tid] = kk.z[w];
+        }
+        Lc[tid] = cc;
+        fold = key_fold<W>(kk);
+        const uint32_t h = fold_mix(fold);
+        const uint32_t entry = (h << 16) | (tid + 1u);
+        uint32_t sl = h >> (32u - kTableBits);
+        while (atomicCAS(&table[sl], 0u, entry) != 0u) sl = (sl + 1u) & ((1u << kTableBits) - 1u);
+    }
+    __syncthreads();
+    // ---- phase B: the staged row's decision; own drops extend the holes ----
+    T own = T(0), fresh = T(0);
+    Key<W> q{};
+    bool keep_own = false, keep_new = false;
+    if (valid) {
+        q = key_xor<W>(kk, g);
+        const uint32_t h = fold_mix(fold ^ key_fold<W>(g));
+        const uint32_t tag = h << 16;
+        uint32_t sl = h >> (32u - kTableBits);
+        int found = -1;
+        for (;;) {
+            const uint32_t e = table[sl];
+            if (e == 0u) break;
+            if ((e & 0xFFFF0000u) == tag) {
+                const uint32_t ix = (e & 0xFFFFu) - 1u;
+                bool eq = true;
+#pragma unroll
+                for (int w = 0; w < W; ++w) eq = eq && (Lx[w][ix] == q.x[w]) && (Lz[w][ix] == q.z[w]);
+                if (eq) {
+                    found = (int)ix;
+                    break;
+                }
+            }
+            sl = (sl + 1u) & ((1u << kTableBits) - 1u);
+        }
+        const T a1 = partner_amplitude_on<W, T>(found >= 0 ? q : kk, g, supp, a.gphase, a.sin_t);
+        own = a.clifford ? T(0) : cc * a.cos_t;
+        if (found >= 0) own = own + Lc[found] * a1;
+        keep_own = survives<W, T>(a.keep, kk, own);
+        if (found < 0) {
+            fresh = cc * a1;
+            keep_new = survives<W, T>(a.keep, q, fresh);
+        }
+    }
+    const uint32_t jn = pair ? (jj ^ 1u) : jj;
+    const bool drop = valid && !keep_own;
+    bool f[4] = {drop && jj == 0, drop && jj == 1, keep_new && jn == 0, keep_new && jn == 1};
+    uint32_t off[4], tot[4];
+    block_flag_scan<4>(f, off, tot, scan_scratch);
+    if (drop) {
+        holes[jj][jj ? hc1 + off[1] : hc0 + off[0]] = (uint16_t)idx;
+        if (a.compact) atomicOr(&hbits[jj][idx >> 5], 1u << (idx & 31u));
+    }
+    const uint32_t rank = jn ? off[3] : off[2];
+    hc0 += tot[0];
+    hc1 += tot[1];
+    const uint32_t nc0 = tot[2], nc1 = tot[3];
+    const uint32_t fin0 = n0 - hc0 + nc0, fin1 = n1 - hc1 + nc1;
+    const bool fits = fin0 <= cap0 && (!pair || fin1 <= cap1) &&
+                      (a.compact || (hc0 <= nc0 && (!pair || hc1 <= nc1)));
+    if (!fits) {
+        queue(moved_segment_rows(fin0) + (pair ? moved_segment_rows(fin1) : 0u));
+        return;
+    }
+    __syncthreads();  // every hole in LDS
+    // ---- phase C, as in the redo launch ----
+    const bool shrink0 = hc0 > nc0, shrink1 = pair && hc1 > nc1;
+    if (shrink0 || shrink1) {  // uniform: the holes before each word of the bitmap
+        if (tid < 2) {
+            uint32_t acc = 0;
+            for (uint32_t w = 0; w < kWords; ++w) {
+                hpre[tid][w] = (uint16_t)acc;
+                acc += (uint32_t)__popc(hbits[tid][w]);
+            }
+            hpre[tid][kWords] = (uint16_t)acc;
+        }
+        __syncthreads();
+    }
+    if (keep_own) {
+        const uint32_t fin = jj ? fin1 : fin0;
+        const uint64_t sj = jj ? s1 : s0;
+        if ((jj ? shrink1 : shrink0) && idx >= fin) {  // a staying row above the final length moves down
+            const uint32_t above = (idx - fin) - (holes_below(hbits[jj], hpre[jj], idx) -
+                                                  holes_below(hbits[jj], hpre[jj], fin));
+            const uint64_t pos = sj + kth_hole<kWords>(hbits[jj], hpre[jj], (jj ? nc1 : nc0) + above);
+            store_key<W>(a.x, a.z, a.cap, pos, kk);
+            store_coeff<T>(a.c, pos, own);
+        } else {
+            a.c[sj + idx] = own;
+        }
+    }
+    if (keep_new) {
+        const uint32_t hcn = jn ? hc1 : hc0;
+        const uint32_t slot = (jn ? shrink1 : shrink0) ? kth_hole<kWords>(hbits[jn], hpre[jn], rank)
+                              : rank < hcn             ? holes[jn][rank]
+                                                       : (jn ? n1 : n0) + (rank - hcn);
+        const uint64_t pos = (jn ? s1 : s0) + slot;
+        store_key<W>(a.x, a.z, a.cap, pos, q);
+        store_coeff<T>(a.c, pos, fresh);
+    }
+    for (int side = 0; side < (pair ? 2 : 1); ++side) {
+        if (!(side ? shrink1 : shrink0)) continue;  // uniform
+        const uint32_t fin = side ? fin1 : fin0, nn = side ? n1 : n0;
+        const uint64_t sj = side ? s1 : s0;
+        for (uint32_t at = fin + tid; at < nn; at += kBlock) {
+            if ((hbits[side][at >> 5] >> (at & 31u)) & 1u) continue;
+            const Key<W> k = load_key<W>(a.x, a.z, a.cap, sj + at);
+            if (anticommutes_on<W>(k, g, supp)) continue;  // a staged row: moved above
+            const T c = a.c[sj + at];
+            const uint32_t above = (at - fin) - (holes_below(hbits[side], hpre[side], at) -
+                                                 holes_below(hbits[side], hpre[side], fin));
+            const uint32_t to = kth_hole<kWords>(hbits[side], hpre[side], (side ? nc1 : nc0) + above);
+            store_key<W>(a.x, a.z, a.cap, sj + to, k);
+            store_coeff<T>(a.c, sj + to, c);
+        }
+    }
+    if (tid == 0) {
+        a.len[b0] = fin0;
+        if (pair) a.len[b1] = fin1;
+        if (a.count_totals) {
+            atomicAdd(&a.stats[0], (unsigned long long)(fin0 + fin1));
+            atomicMax(&a.stats[1], (unsigned long long)max(fin0, fin1));
+        }
+    }
+}
+
+// The redo launch: the queued pairs, staging up to the largest.
+template <int W, typename T, bool FILTER>
 __global__ void __launch_bounds__(kBlock) k_rotation_inplace(const InplaceArgs<W, T> a) {
     extern __shared__ __align__(16) unsigned char lds[];
     __shared__ uint32_t scan_scratch[4 * kWaves];
@@ -764,7 +1052,7 @@ __global__ void __launch_bounds__(kBlock) k_rotation_inplace(const InplaceArgs<W
     uint8_t* const Lm = reinterpret_cast<uint8_t*>(holes + 2 * kInplaceHoles);
     uint8_t* const Lflag = Lm + S;
 
-    const uint32_t count = REDO ? (uint32_t)*a.redo_count : a.num_cosets;
+    const uint32_t count = (uint32_t)*a.redo_count;
     const bool pair = a.delta != 0;
     Key<W> g;
 #pragma unroll
@@ -786,7 +1074,7 @@ __global__ void __launch_bounds__(kBlock) k_rotation_inplace(const InplaceArgs<W
         }
     };
     for (uint32_t t = blockIdx.x; t < count; t += gridDim.x) {  // uniform
-        const uint32_t p = REDO ? a.redo[t] : t;
+        const uint32_t p = a.redo[t];
         uint32_t b0, b1;
         if (pair) {
             const uint32_t lo = p & ((1u << a.hb) - 1u);
@@ -866,15 +1154,7 @@ __global__ void __launch_bounds__(kBlock) k_rotation_inplace(const InplaceArgs<W
             nl += tot[2] + tot[3];
         }
         if (overflow) {
-            if (threadIdx.x == 0) {
-                if (REDO) {
-                    atomicOr(&a.stats[2], 1ull);  // the redo launch stages the largest pair: never expected
-                } else {
-                    a.redo[atomicAdd(a.redo_count, 1ull)] = p;
-                    // a side's rows after the layer are at most the pair's
-                    atomicAdd(&a.stats[7], (unsigned long long)(2u * moved_segment_rows(n)));
-                }
-            }
+            if (threadIdx.x == 0) atomicOr(&a.stats[2], 1ull);  // it stages the largest pair: never expected
             continue;
         }
         __syncthreads();  // staging, table and phase A's holes complete
@@ -949,13 +1229,6 @@ __global__ void __launch_bounds__(kBlock) k_rotation_inplace(const InplaceArgs<W
         const bool fits = fin0 <= cap0 && (!pair || fin1 <= cap1) &&
                           (compactable || (hc0 <= nc0 && (!pair || hc1 <= nc1)));
         __syncthreads();  // every decision and hole in LDS
-        if (!fits && !REDO) {
-            if (threadIdx.x == 0) {
-                a.redo[atomicAdd(a.redo_count, 1ull)] = p;
-                atomicAdd(&a.stats[7], (unsigned long long)(moved_segment_rows(fin0) + (pair ? moved_segment_rows(fin1) : 0u)));
-            }
-            continue;
-        }
         if (fits) {
             // ---- phase C in place: kept own coefficients, new rows into the holes and then after the rows; a
             // side left with holes (more holes than new rows) takes its new rows into its lowest holes and moves the
@@ -982,7 +1255,7 @@ __global__ void __launch_bounds__(kBlock) k_rotation_inplace(const InplaceArgs<W
                         // its rank among the rows that stay above the final length, after the new rows
                         const uint32_t above = (at - fin) - (holes_below(hbits[jj], hpre[jj], at) -
                                                              holes_below(hbits[jj], hpre[jj], fin));
-                        const uint32_t to = kth_hole(hbits[jj], hpre[jj], (jj ? nc1 : nc0) + above);
+                        const uint32_t to = kth_hole<kHoleWords>(hbits[jj], hpre[jj], (jj ? nc1 : nc0) + above);
                         const uint64_t pos = (jj ? s1 : s0) + to;
                         Key<W> kk;
 #pragma unroll
@@ -1000,7 +1273,7 @@ __global__ void __launch_bounds__(kBlock) k_rotation_inplace(const InplaceArgs<W
                     const uint32_t jn = pair ? (jj ^ 1u) : jj;
                     const uint32_t rk = Lrank[i];
                     const uint32_t hcn = jn ? hc1 : hc0;
-                    const uint32_t slot = (jn ? shrink1 : shrink0) ? kth_hole(hbits[jn], hpre[jn], rk)
+                    const uint32_t slot = (jn ? shrink1 : shrink0) ? kth_hole<kHoleWords>(hbits[jn], hpre[jn], rk)
                                           : rk < hcn ? holes[jn * kInplaceHoles + rk]
                                                      : (jn ? n1 : n0) + (rk - hcn);
                     const uint64_t pos = (jn ? s1 : s0) + slot;
@@ -1027,7 +1300,7 @@ __global__ void __launch_bounds__(kBlock) k_rotation_inplace(const InplaceArgs<W
                     const T c = a.c[sj + at];
                     const uint32_t above = (at - fin) - (holes_below(hbits[jj], hpre[jj], at) -
                                                          holes_below(hbits[jj], hpre[jj], fin));
-                    const uint32_t to = kth_hole(hbits[jj], hpre[jj], (jj ? nc1 : nc0) + above);
+                    const uint32_t to = kth_hole<kHoleWords>(hbits[jj], hpre[jj], (jj ? nc1 : nc0) + above);
                     store_key<W>(a.x, a.z, a.cap, sj + to, k);
                     store_coeff<T>(a.c, sj + to, c);
                 }
@@ -1601,16 +1874,17 @@ hipError_t launch_publish_counters(hipStream_t st, unsigned long long* counters,
 template <int W, typename T>
 hipError_t launch_rotation_inplace(hipStream_t st, const InplaceArgs<W, T>& a) {
     if (a.num_cosets == 0) return hipSuccess;
-    if (a.scap > kPairRowsMax || a.tcap_bits > 11) return hipErrorInvalidValue;
-    const size_t lds = inplace_lds_bytes<W, T>(a.scap, a.tcap_bits);
     const bool filter = a.filter != nullptr;
     if (!a.redo_mode) {
+        if (a.scap > kBlock) return hipErrorInvalidValue;
         if (filter)
-            hipLaunchKernelGGL((k_rotation_inplace<W, T, false, true>), dim3(a.num_cosets), dim3(kBlock), lds, st, a);
+            hipLaunchKernelGGL((k_rotation_pair<W, T, true>), dim3(a.num_cosets), dim3(kBlock), 0, st, a);
         else
-            hipLaunchKernelGGL((k_rotation_inplace<W, T, false, false>), dim3(a.num_cosets), dim3(kBlock), lds, st, a);
+            hipLaunchKernelGGL((k_rotation_pair<W, T, false>), dim3(a.num_cosets), dim3(kBlock), 0, st, a);
         return hipGetLastError();
     }
+    if (a.scap > kPairRowsMax || a.tcap_bits > 11) return hipErrorInvalidValue;
+    const size_t lds = inplace_lds_bytes<W, T>(a.scap, a.tcap_bits);
     static int cus = 0;
     if (cus == 0) {
         int dev = 0;
@@ -1620,14 +1894,14 @@ hipError_t launch_rotation_inplace(hipStream_t st, const InplaceArgs<W, T>& a) {
     }
     int per = 0;
     const hipError_t oe = filter ? hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                                       &per, k_rotation_inplace<W, T, true, true>, kBlock, lds)
+                                       &per, k_rotation_inplace<W, T, true>, kBlock, lds)
                                  : hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                                       &per, k_rotation_inplace<W, T, true, false>, kBlock, lds);
+                                       &per, k_rotation_inplace<W, T, false>, kBlock, lds);
     if (oe != hipSuccess || per <= 0) per = 1;
     if (filter)
-        hipLaunchKernelGGL((k_rotation_inplace<W, T, true, true>), dim3(cus * per), dim3(kBlock), lds, st, a);
+        hipLaunchKernelGGL((k_rotation_inplace<W, T, true>), dim3(cus * per), dim3(kBlock), lds, st, a);
     else
-        hipLaunchKernelGGL((k_rotation_inplace<W, T, true, false>), dim3(cus * per), dim3(kBlock), lds, st, a);
+        hipLaunchKernelGGL((k_rotation_inplace<W, T, false>), dim3(cus * per), dim3(kBlock), lds, st, a);
     return hipGetLastError();
 }
 
