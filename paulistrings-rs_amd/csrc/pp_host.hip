@@ -283,6 +283,10 @@ struct pp_context {
     void* stage[2] = {nullptr, nullptr};   // pinned host chunks of the bulk transfers, allocated on first use
     hipEvent_t stage_ev[2] = {nullptr, nullptr};
     void* class_pinned = nullptr;  // a class pass's program on its way up and its counters on their way down
+    // The sums' pinned slots, carved from blocks of kSlotBlock that stay with the context: a pinned allocation of its own
+    // costs a sum 0.1 ms, and giving it back 0.2-0.4 ms.
+    std::vector<void*> slot_blocks;
+    std::vector<unsigned long long*> free_slots;
     hipEvent_t lag_ev[2] = {nullptr, nullptr};  // the counters of a layer queued ahead of them have arrived
 };
 
@@ -364,7 +368,7 @@ struct pp_sum {
     bool topn_seed_valid = false;
     bool topn_seed_score = false;  // the seed is a score key (the learned pass), not a |c|^2 one
     double topn_width = 0;         // the next windowed selection's half-width around the seed (0: none yet)
-    pp::WindowCounts* d_window = nullptr;
+    bool window_ready = false;     // d_window is zero between selections
     uint64_t phys_len = 0;
     const uint8_t* pending_flags = nullptr;
     const float* pending_score = nullptr;  // the ranking score when the selection was by score
@@ -373,15 +377,17 @@ struct pp_sum {
     uint64_t tiles_cap = 0;
     unsigned long long* d_stats = nullptr;
     unsigned long long* h_stats = nullptr;  // pinned
-    // Three pinned, device-visible slots of kStatSlots words, allocated on first use: two for the counters of layers
-    // queued ahead of them (lagged lengths), one for a windowed selection's answer; the device address of the same
-    // memory; the sequence number of the slots' last writer.
+    // Three more slots of kStatSlots words in h_stats' block, which kernels write: two for the counters of layers queued
+    // ahead of them (lagged lengths), one for a windowed selection's or a read-out's answer; the device address of the
+    // same memory; the sequence number of the slots' last writer.
     unsigned long long* h_lag = nullptr;
     unsigned long long* d_lag_host = nullptr;
     unsigned long long lag_seq = 0;
     unsigned long long* d_lag_counters = nullptr;  // the small joins' counters: two sets of 4, by ring slot
     pp::TopnState* d_topn = nullptr;
     unsigned long long* d_hist = nullptr;
+    pp::WindowCounts* d_window = nullptr;
+    unsigned char* d_fixed = nullptr;  // the allocation of d_stats, d_lag_counters, d_rows, d_topn, d_hist and d_window
     uint32_t* d_redo = nullptr;  // pairs a join could not stage, for its redo launch
     uint64_t redo_cap = 0;
     float* d_score = nullptr;  // the learned pass's score per column position
@@ -512,16 +518,42 @@ pp_status read_stats(pp_sum* s) {
     return PP_OK;
 }
 
-pp_status ensure_lag_slots(pp_sum* s) {
-    if (s->h_lag) return PP_OK;
-    if (hipHostMalloc((void**)&s->h_lag, 3 * kStatSlots * sizeof(unsigned long long),
-                      hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
-        (void)hipGetLastError();
-        s->h_lag = nullptr;
-        return fail(s->ctx, PP_ERR_OUT_OF_MEMORY, "pinned host allocation");
+constexpr size_t kSumSlotWords = 4 * kStatSlots;  // a sum's pinned words: h_stats, then the three slots of h_lag
+constexpr size_t kSlotBlock = (size_t)1 << 14;    // 64 sums' worth
+
+// A new sum's fixed device memory (one allocation: counters, read-out partials, hash rows, selection state, histograms
+// and window counts) and its pinned slots.
+pp_status alloc_fixed(pp_sum* s) {
+    pp_context* ctx = s->ctx;
+    if (ctx->free_slots.empty()) {
+        void* block = nullptr;
+        if (hipHostMalloc(&block, kSlotBlock, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
+            (void)hipGetLastError();
+            return fail(ctx, PP_ERR_OUT_OF_MEMORY, "pinned host allocation");
+        }
+        ctx->slot_blocks.push_back(block);
+        for (size_t w = 0; w + kSumSlotWords <= kSlotBlock / 8; w += kSumSlotWords)
+            ctx->free_slots.push_back((unsigned long long*)block + w);
     }
-    std::memset(s->h_lag, 0, 3 * kStatSlots * sizeof(unsigned long long));
-    PP_HIP(s->ctx, hipHostGetDevicePointer((void**)&s->d_lag_host, s->h_lag, 0));
+    s->h_stats = ctx->free_slots.back();
+    ctx->free_slots.pop_back();
+    std::memset(s->h_stats, 0, kSumSlotWords * sizeof(unsigned long long));
+    void* dev = nullptr;
+    PP_HIP(ctx, hipHostGetDevicePointer(&dev, s->h_stats, 0));
+    s->h_lag = s->h_stats + kStatSlots;
+    s->d_lag_host = (unsigned long long*)dev + kStatSlots;
+    auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
+    const size_t stats = (kStatSlots + kReadoutGroups + 8) * 8, rows = s->rows.size() * 8;
+    const size_t o_rows = up(stats), o_topn = o_rows + up(rows), o_hist = o_topn + up(sizeof(TopnState));
+    const size_t o_window = o_hist + up(kSeededHistWords * 8);
+    pp_status st = dev_alloc(ctx, (void**)&s->d_fixed, o_window + sizeof(WindowCounts));
+    if (st != PP_OK) return st;
+    s->d_stats = (unsigned long long*)s->d_fixed;
+    s->d_lag_counters = s->d_stats + kStatSlots + kReadoutGroups;
+    s->d_rows = (uint64_t*)(s->d_fixed + o_rows);
+    s->d_topn = (TopnState*)(s->d_fixed + o_topn);
+    s->d_hist = (unsigned long long*)(s->d_fixed + o_hist);
+    s->d_window = (WindowCounts*)(s->d_fixed + o_window);
     return PP_OK;
 }
 
@@ -2177,6 +2209,7 @@ void pp_context_destroy(pp_context* ctx) {
         if (ctx->stage_ev[k]) (void)hipEventDestroy(ctx->stage_ev[k]);
     }
     if (ctx->class_pinned) (void)hipHostFree(ctx->class_pinned);
+    for (void* b : ctx->slot_blocks) (void)hipHostFree(b);
     for (hipEvent_t e : ctx->lag_ev)
         if (e) (void)hipEventDestroy(e);
     delete ctx;
@@ -2336,10 +2369,7 @@ pp_status pp_sum_upload(pp_context* ctx, uint32_t num_qubits, uint32_t width, pp
         return st;
     };
     pp_status st;
-    if ((st = dev_alloc(ctx, (void**)&s->d_rows, s->rows.size() * 8)) != PP_OK) return bail(st);
-    if ((st = dev_alloc(ctx, (void**)&s->d_stats, kStatSlots * sizeof(unsigned long long))) != PP_OK) return bail(st);
-    if (hipHostMalloc((void**)&s->h_stats, kStatSlots * sizeof(unsigned long long), hipHostMallocDefault) != hipSuccess)
-        return bail(fail(ctx, PP_ERR_OUT_OF_MEMORY, "pinned host allocation"));
+    if ((st = alloc_fixed(s)) != PP_OK) return bail(st);
     if (hipMemcpy(s->d_rows, s->rows.data(), s->rows.size() * 8, hipMemcpyHostToDevice) != hipSuccess)
         return bail(fail(ctx, PP_ERR_DRIVER, "hash rows upload"));
 
@@ -2452,16 +2482,10 @@ pp_status pp_sum_free(pp_sum* s) {
         free_columns(s->col[i]);
         free_buckets(s->bk[i]);
     }
-    if (s->d_rows) (void)hipFree(s->d_rows);
-    if (s->d_stats) (void)hipFree(s->d_stats);
-    if (s->h_stats) (void)hipHostFree(s->h_stats);
-    if (s->h_lag) (void)hipHostFree(s->h_lag);
-    if (s->d_lag_counters) (void)hipFree(s->d_lag_counters);
-    if (s->d_topn) (void)hipFree(s->d_topn);
-    if (s->d_window) (void)hipFree(s->d_window);
+    if (s->d_fixed) (void)hipFree(s->d_fixed);
+    if (s->h_stats) s->ctx->free_slots.push_back(s->h_stats);
     if (s->d_redo) (void)hipFree(s->d_redo);
     if (s->d_score) (void)hipFree(s->d_score);
-    if (s->d_hist) (void)hipFree(s->d_hist);
     if (s->d_tiles) (void)hipFree(s->d_tiles);
     for (void* p : s->scratch)
         if (p) (void)hipFree(p);
@@ -2496,10 +2520,7 @@ pp_status pp_sum_clone(const pp_sum* src_c, pp_sum** out) {
         return st;
     };
     pp_status st;
-    if ((st = dev_alloc(ctx, (void**)&s->d_rows, s->rows.size() * 8)) != PP_OK) return bail(st);
-    if ((st = dev_alloc(ctx, (void**)&s->d_stats, kStatSlots * sizeof(unsigned long long))) != PP_OK) return bail(st);
-    if (hipHostMalloc((void**)&s->h_stats, kStatSlots * sizeof(unsigned long long), hipHostMallocDefault) != hipSuccess)
-        return bail(fail(ctx, PP_ERR_OUT_OF_MEMORY, "pinned host allocation"));
+    if ((st = alloc_fixed(s)) != PP_OK) return bail(st);
     const Columns& sc = src->col[src->cur];
     const BucketArrays& sb = src->bk[src->cur];
     if ((st = ensure_columns(s, 0, sc.cap)) != PP_OK) return bail(st);
@@ -3128,10 +3149,6 @@ pp_status propagate_lagged(pp_sum* s, const RunPlanner& plan, const KeepProgram&
     pp_status st;
     for (hipEvent_t& e : ctx->lag_ev)
         if (!e) PP_HIP(ctx, hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    if ((st = ensure_lag_slots(s)) != PP_OK) return st;
-    if (!s->d_lag_counters &&
-        (st = dev_alloc(ctx, (void**)&s->d_lag_counters, 8 * sizeof(unsigned long long))) != PP_OK)
-        return st;
     // zero from here on, each set cleared when its counters are published (and here, in case a propagation that
     // failed left one unpublished)
     PP_HIP(ctx, launch_fill_u64(ctx->stream, s->d_lag_counters, 8, 0ull));
@@ -3362,11 +3379,7 @@ pp_status pp_expectation_product(pp_sum* s, const uint64_t* axis_x, const uint64
         if (rs != PP_OK) return rs;
     }
     const uint32_t B = 1u << s->device_bits;
-    const uint32_t per = 64;
-    const uint32_t blocks = (B + per - 1) / per;
-    double* d_partial = nullptr;
-    pp_status st;
-    if ((st = dev_alloc(ctx, (void**)&d_partial, blocks * 8)) != PP_OK) return st;
+    const unsigned long long seq = ++s->lag_seq;
     hipError_t e = dispatch(s, [&](auto Wc, auto Tv) {
         constexpr int W = decltype(Wc)::value;
         using T = decltype(Tv);
@@ -3378,23 +3391,25 @@ pp_status pp_expectation_product(pp_sum* s, const uint64_t* axis_x, const uint64
         a.start = s->bk[s->cur].start;
         a.len = s->bk[s->cur].len;
         a.num_buckets = B;
-        a.buckets_per_block = per;
+        a.buckets_per_block = std::max<uint32_t>(1, B / kReadoutGroups);
         for (int w = 0; w < W; ++w) {
+            const uint64_t live = live_mask(s->num_qubits, w);
             a.axis_x[w] = axis_x[w];
             a.axis_z[w] = axis_z[w];
             a.negative[w] = negative[w];
+            if (w == 0) a.sieve = (~axis_x[0] & live) ? 1u : (~axis_z[0] & live) ? 2u : 0u;
         }
-        a.partial = d_partial;
-        return launch_expectation<W, T>(ctx->stream, a, blocks);
+        a.partial = (double*)(s->d_stats + kStatSlots);
+        a.host = s->d_lag_host + 2 * kStatSlots;
+        a.seq = seq;
+        return launch_expectation<W, T>(ctx->stream, a);
     });
-    std::vector<double> partial(blocks);
-    if (e == hipSuccess) e = hipMemcpyAsync(partial.data(), d_partial, blocks * 8, hipMemcpyDeviceToHost, ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-    (void)hipFree(d_partial);
-    if (e != hipSuccess) return fail(ctx, PP_ERR_DRIVER, std::string("expectation: ") + hipGetErrorString(e));
-    double total = 0.0;
-    for (double v : partial) total += v;
-    *out = total;
+    PP_HIP(ctx, e);
+    volatile const unsigned long long* h = s->h_lag + 2 * kStatSlots;
+    const pp_status st = wait_for_slot(ctx, h, seq, "expectation: the answer never arrived");
+    if (st != PP_OK) return st;
+    const unsigned long long bits = h[0];
+    std::memcpy(out, &bits, 8);
     return PP_OK;
 }
 

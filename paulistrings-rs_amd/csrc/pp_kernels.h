@@ -226,8 +226,12 @@ struct ExpectationArgs {
     uint64_t axis_x[W];
     uint64_t axis_z[W];
     uint64_t negative[W];
-    double* partial;
+    uint32_t sieve;   // what of word 0 rules most terms out: 1 an x bit off the axis, 2 a z bit, 0 the two together
+    double* partial;  // a sum per workgroup, at most kReadoutGroups
+    unsigned long long* host;  // pinned: [0] the total's bits, then [4] = seq
+    unsigned long long seq;
 };
+constexpr uint32_t kReadoutGroups = 2048;
 
 template <int W, typename T>
 struct ExportArgs {
@@ -324,7 +328,7 @@ hipError_t launch_refine(hipStream_t st, const RefineArgs<W, T>& a);
 template <int W, typename T>
 hipError_t launch_coarsen(hipStream_t st, const CoarsenArgs<W, T>& a);
 template <int W, typename T>
-hipError_t launch_expectation(hipStream_t st, const ExpectationArgs<W, T>& a, uint32_t blocks);
+hipError_t launch_expectation(hipStream_t st, const ExpectationArgs<W, T>& a);
 template <int W, typename T>
 hipError_t launch_export(hipStream_t st, const ExportArgs<W, T>& a, uint32_t num_buckets);
 template <int W, typename T>
