@@ -18,6 +18,7 @@ constexpr int kMlpTile = 64;  // terms per workgroup pass
 constexpr int kOffW1 = 0, kOffB1 = kOffW1 + kMlpInPad * kMlpHid, kOffW2 = kOffB1 + kMlpHid,
               kOffB2 = kOffW2 + kMlpHid * kMlpHid, kOffW3 = kOffB2 + kMlpHid, kOffB3 = kOffW3 + kMlpHid,
               kMlpParams = kOffB3 + 1;
+constexpr int kMlpPartial = (kMlpParams + 3) & ~3;  // a tile's partial gradient, every one 16-byte aligned
 
 struct MlpDev {
     const float* params;   // fp32 master, kMlpParams
@@ -41,12 +42,23 @@ struct MlpBatch {
 hipError_t launch_mlp_refresh(hipStream_t st, const float* params, uint16_t* w1t, uint16_t* w2t, uint16_t* w2);
 hipError_t launch_mlp_predict(hipStream_t st, const MlpDev& m, const MlpBatch& b, float* out);
 // The gradient of the batch's mean squared error into grads (kMlpParams floats) and the sum of its squared errors
-// into loss[0], through per-tile partials (partial: partial_tiles x kMlpParams floats, loss_part: partial_tiles
+// into loss[0], through per-tile partials (partial: partial_tiles x kMlpPartial floats, loss_part: partial_tiles
 // doubles, at least one tile per kMlpTile rows) summed in a fixed order.
 hipError_t launch_mlp_grad(hipStream_t st, const MlpDev& m, const MlpBatch& b, float* partial, double* loss_part,
                            uint64_t partial_tiles, float* grads, double* loss);
-hipError_t launch_mlp_adam(hipStream_t st, float* params, float* adam_m, float* adam_v, const float* grads,
-                           float lr, float beta1, float beta2, float eps, int step);
+// One training step in two launches: the tiles' gradients, then their sums, Adam and the bf16 copies; the batch's sum of
+// squared errors into loss[0].
+struct MlpTrain {
+    float* params;
+    float* adam_m;
+    float* adam_v;
+    uint16_t* w1t;
+    uint16_t* w2t;
+    uint16_t* w2;
+};
+hipError_t launch_mlp_train_step(hipStream_t st, const MlpDev& m, const MlpBatch& b, const MlpTrain& t, float* partial,
+                                 double* loss_part, uint64_t partial_tiles, double* loss, float lr, float beta1,
+                                 float beta2, float eps, int step);
 
 // The score of every term of a resident one-word sum, ln|c| + the network's output (the predicted ln of the term's
 // read-out factor |<psi| P propagated |psi>|), so the predicted ln|contribution|; written at the term's column

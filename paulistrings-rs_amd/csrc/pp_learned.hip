@@ -176,12 +176,10 @@ __device__ __forceinline__ void mlp_layer1(const FwdWeights& fw, FwdLds& s) {
                 pack_bf16x4(relu(acc[i][j][0]), relu(acc[i][j][1]), relu(acc[i][j][2]), relu(acc[i][j][3]));
 }
 
-// Layer 2 of the tile in s.a1 (K = 128) and this wave's share of the output into ypart[w]; h2 (fp32 relu(z2),
-// [row][hidden]) is written when not null.
-__device__ __forceinline__ void mlp_layer2(const FwdWeights& fw, const FwdLds& s, float* h2,
-                                           float (*ypart)[kMlpTile]) {
+// Layer 2 of the tile in s.a1 (K = 128) and this wave's share of the output into ypart[w].
+__device__ __forceinline__ void mlp_layer2(const FwdWeights& fw, const FwdLds& s, float (*ypart)[kMlpTile]) {
     const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int lr = l & 15, lk = (l >> 4) * 8, lq = 4 * (l >> 4);
+    const int lr = l & 15, lk = (l >> 4) * 8;
     f32x4 acc[kMlpTile / 16][2];
 #pragma unroll
     for (int i = 0; i < kMlpTile / 16; ++i)
@@ -206,15 +204,8 @@ __device__ __forceinline__ void mlp_layer2(const FwdWeights& fw, const FwdLds& s
         for (int j = 0; j < 2; ++j) {
             const float4 w3v = lane_units(s.w3, j);
             const float w3q[4] = {w3v.x, w3v.y, w3v.z, w3v.w};
-            float h[4];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                h[q] = relu(acc[i][j][q]);
-                part = __builtin_fmaf(h[q], w3q[q], part);
-            }
-            if (h2)
-                *reinterpret_cast<float4*>(h2 + (16 * i + lr) * kMlpHid + 32 * w + 16 * j + lq) =
-                    make_float4(h[0], h[1], h[2], h[3]);
+            for (int q = 0; q < 4; ++q) part = __builtin_fmaf(relu(acc[i][j][q]), w3q[q], part);
         }
         part += __shfl_xor(part, 16, 64);
         part += __shfl_xor(part, 32, 64);
@@ -230,11 +221,11 @@ __device__ __forceinline__ float mlp_output(const FwdWeights& fw, const float (*
     return v + fw.b3;
 }
 
-// Layers 1 and 2 and the output for the tile in s.a0, into s.y; h2 as in mlp_layer2.
-__device__ __forceinline__ void mlp_forward_tile(const FwdWeights& fw, FwdLds& s, float* h2) {
+// Layers 1 and 2 and the output for the tile in s.a0, into s.y.
+__device__ __forceinline__ void mlp_forward_tile(const FwdWeights& fw, FwdLds& s) {
     mlp_layer1(fw, s);
     __syncthreads();
-    mlp_layer2(fw, s, h2, s.ypart[0]);
+    mlp_layer2(fw, s, s.ypart[0]);
     __syncthreads();
     if (threadIdx.x < kMlpTile) s.y[threadIdx.x] = mlp_output(fw, s.ypart[0], threadIdx.x);
     __syncthreads();
@@ -265,149 +256,253 @@ __global__ void __launch_bounds__(256) k_mlp_predict(const MlpDev m, const MlpBa
     term_features(m, valid ? b.x[i] : 0, valid ? b.z[i] : 0, valid ? b.c[i] : 1.0, valid ? b.remaining[i] : 0.f,
                   valid, part, s.a0 + row * kLd0, nullptr);
     __syncthreads();
-    mlp_forward_tile(fw, s, nullptr);
+    mlp_forward_tile(fw, s);
     if (threadIdx.x < kMlpTile && base + threadIdx.x < b.count) out[base + threadIdx.x] = s.y[threadIdx.x];
 }
 
-struct GradLds {
-    FwdLds f;
-    uint16_t a0t[kMlpInPad * kMlpTile];  // [64 inputs][64 rows]
-    uint16_t a1t[kMlpHid * kMlpTile];    // [128 hidden][64 rows]
-    uint16_t dz2[kMlpTile * kMlpHid];    // bf16 dz2 [rows][hidden]
-    uint16_t dzt[kMlpHid * kMlpTile];    // bf16 dz2, later dz1, transposed [hidden][rows]
-    float h[kMlpTile * kMlpHid];         // fp32 h2, then dz2, then dz1
+// ---- the backward pass ---------------------------------------------------------------------------------------------
+//
+// A workgroup of sixteen waves takes a tile of 64 samples: a training batch is a few such tiles, far fewer than compute
+// units, so a step's time is one tile's chain of phases.  Wave (w, i) = (wave & 3, wave >> 2) owns hidden units
+// 32 w .. 32 w + 31 of sample tile i in both forward layers and keeps its second layer's outputs in registers until the
+// error is known; the weight-gradient products are split sixteen ways.  Every sum runs in the order it has with one
+// wave per 32 hidden units, so the gradients have the same bits.
+
+constexpr int kGradBlock = 1024, kGradWaves = kGradBlock / 64;
+constexpr int kLdT = kMlpTile + 8;   // row stride (bf16) of the transposed tiles: a row per unit, a column per sample
+constexpr int kLdH = kMlpHid + 4;    // row stride (fp32) of h
+
+struct alignas(16) GradLds {
+    uint16_t a0[kMlpTile * kLd0];  // features [row][input]
+    uint16_t a0t[kMlpInPad * kLdT];
+    uint16_t a1[kMlpTile * kLd1];  // relu(z1) [row][hidden]
+    uint16_t a1t[kMlpHid * kLdT];
+    uint16_t dz2[kMlpTile * kLd1];  // bf16 dz2 [row][hidden]
+    uint16_t dzt[kMlpHid * kLdT];   // bf16 dz2, later dz1, transposed
+    float h[kMlpTile * kLdH];       // fp32 h2, then dz2, then dz1
+    float ypart[kWaves][kMlpTile];
+    float b1[kMlpHid], b2[kMlpHid], w3[kMlpHid];
     float dy[kMlpTile];
-    double e2[kMlpTile];                 // each row's squared error
+    double e2[kMlpTile];  // each row's squared error
 };
 
-// Column sums over the tile's 64 rows of an fp32 [64][128] matrix, stored to g[0 .. 128).
+// Column sums over the tile's 64 rows of h, in row order, stored to g[0 .. 128).
 __device__ __forceinline__ void store_column_sums(const float* h, float* g) {
     if (threadIdx.x < kMlpHid) {
         float s = 0.f;
-        for (int r = 0; r < kMlpTile; ++r) s += h[r * kMlpHid + threadIdx.x];
+#pragma unroll 16
+        for (int r = 0; r < kMlpTile; ++r) s += h[r * kLdH + threadIdx.x];
         g[threadIdx.x] = s;
     }
 }
 
-// Workgroup t writes the gradient of its 64 rows to partial[t * kMlpParams ...] (every parameter but W1's padding
-// rows, each by one thread) and their squared error to loss_part[t]; k_mlp_reduce sums the tiles in tile order, so
-// that a gradient, and the training built on it, is the same on every run.
-__global__ void __launch_bounds__(256) k_mlp_grad(const MlpDev m, const MlpBatch b, float* __restrict__ partial,
-                                                  double* __restrict__ loss_part) {
+// Workgroup t writes the gradient of its 64 rows to partial[t * kMlpPartial ...] (every parameter but W1's padding
+// rows, each by one thread) and their squared error to loss_part[t]; k_mlp_reduce or k_mlp_step sums the tiles in tile
+// order, so that a gradient, and the training built on it, is the same on every run.  A chain of eight barriers bounds
+// it: 17 us a step of eight tiles, 30 with four waves, whose transposes hit one LDS bank.
+__global__ void __launch_bounds__(kGradBlock) k_mlp_grad(const MlpDev m, const MlpBatch b, float* __restrict__ partial,
+                                                         double* __restrict__ loss_part) {
     __shared__ GradLds s;
-    float* const grads = partial + (uint64_t)blockIdx.x * kMlpParams;
-    const FwdWeights fw = load_fwd_weights(m, s.f);
-    const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+    float* const grads = partial + (uint64_t)blockIdx.x * kMlpPartial;
+    const int tid = threadIdx.x, l = tid & 63, wave = tid >> 6;
+    const int w = wave & 3, ti = wave >> 2;
+    const int lr = l & 15, lk = (l >> 4) * 8, lq = 4 * (l >> 4);
     const uint64_t base = (uint64_t)blockIdx.x * kMlpTile;
-    {
-        const int row = threadIdx.x & 63, part = threadIdx.x >> 6;
-        const uint64_t i = base + row;
+    // this wave's weights, in flight through the features
+    bf16x8 w1[2][kMlpInPad / 32], w2[2][kMlpHid / 32];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int row = 32 * w + 16 * j + lr;
+#pragma unroll
+        for (int ks = 0; ks < kMlpInPad / 32; ++ks) w1[j][ks] = load_frag(m.w1t + row * kMlpInPad + 32 * ks + lk);
+#pragma unroll
+        for (int ks = 0; ks < kMlpHid / 32; ++ks) w2[j][ks] = load_frag(m.w2t + row * kMlpHid + 32 * ks + lk);
+    }
+    const float b3 = m.params[kOffB3];
+    if (tid < 256) {
+        const int part = tid >> 6;
+        const uint64_t i = base + l;
         const bool valid = i < b.count;
         term_features(m, valid ? b.x[i] : 0, valid ? b.z[i] : 0, valid ? b.c[i] : 1.0, valid ? b.remaining[i] : 0.f,
-                      valid, part, s.f.a0 + row * kLd0, nullptr);
+                      valid, part, s.a0 + l * kLd0, nullptr);
+    } else if (tid < 256 + kMlpHid) {
+        s.b1[tid - 256] = m.params[kOffB1 + tid - 256];
+        s.b2[tid - 256] = m.params[kOffB2 + tid - 256];
+        s.w3[tid - 256] = m.params[kOffW3 + tid - 256];
     }
     __syncthreads();
-    mlp_forward_tile(fw, s.f, s.h);
+    {  // a0 transposed: a lane per row, four inputs a wave
+        const uint2 v = *reinterpret_cast<const uint2*>(s.a0 + l * kLd0 + 4 * wave);
+        s.a0t[(4 * wave + 0) * kLdT + l] = (uint16_t)v.x;
+        s.a0t[(4 * wave + 1) * kLdT + l] = (uint16_t)(v.x >> 16);
+        s.a0t[(4 * wave + 2) * kLdT + l] = (uint16_t)v.y;
+        s.a0t[(4 * wave + 3) * kLdT + l] = (uint16_t)(v.y >> 16);
+    }
+    // layer 1, its outputs in both layouts
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const float4 bias = *reinterpret_cast<const float4*>(s.b1 + 32 * w + 16 * j + lq);
+        f32x4 acc = f32x4{bias.x, bias.y, bias.z, bias.w};
+#pragma unroll
+        for (int ks = 0; ks < kMlpInPad / 32; ++ks)
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w1[j][ks], load_frag(s.a0 + (16 * ti + lr) * kLd0 + 32 * ks + lk),
+                                                          acc, 0, 0, 0);
+        const uint2 p = pack_bf16x4(relu(acc[0]), relu(acc[1]), relu(acc[2]), relu(acc[3]));
+        const int unit = 32 * w + 16 * j + lq, row = 16 * ti + lr;
+        *reinterpret_cast<uint2*>(s.a1 + row * kLd1 + unit) = p;
+        s.a1t[(unit + 0) * kLdT + row] = (uint16_t)p.x;
+        s.a1t[(unit + 1) * kLdT + row] = (uint16_t)(p.x >> 16);
+        s.a1t[(unit + 2) * kLdT + row] = (uint16_t)p.y;
+        s.a1t[(unit + 3) * kLdT + row] = (uint16_t)(p.y >> 16);
+    }
+    __syncthreads();
+    // layer 2 and this wave's share of the output
+    float h2[2][4];
+    {
+        float part = 0.f;
+        f32x4 acc[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const float4 bias = *reinterpret_cast<const float4*>(s.b2 + 32 * w + 16 * j + lq);
+            acc[j] = f32x4{bias.x, bias.y, bias.z, bias.w};
+        }
+#pragma unroll
+        for (int ks = 0; ks < kMlpHid / 32; ++ks) {
+            const bf16x8 a = load_frag(s.a1 + (16 * ti + lr) * kLd1 + 32 * ks + lk);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w2[j][ks], a, acc[j], 0, 0, 0);
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int unit = 32 * w + 16 * j + lq;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                h2[j][q] = relu(acc[j][q]);
+                part = __builtin_fmaf(h2[j][q], s.w3[unit + q], part);
+            }
+            *reinterpret_cast<float4*>(s.h + (16 * ti + lr) * kLdH + unit) =
+                make_float4(h2[j][0], h2[j][1], h2[j][2], h2[j][3]);
+        }
+        part += __shfl_xor(part, 16, 64);
+        part += __shfl_xor(part, 32, 64);
+        s.ypart[w][16 * ti + lr] = part;  // the four lanes of a term hold the same sum
+    }
+    __syncthreads();
     // dy and the loss
-    if (threadIdx.x < kMlpTile) {
-        const uint64_t i = base + threadIdx.x;
+    if (tid < kMlpTile) {
+        const uint64_t i = base + tid;
         float d = 0.f;
         double e2 = 0.0;
         if (i < b.count) {
-            const float e = s.f.y[threadIdx.x] - b.label[i];
+            float y = s.ypart[0][tid];
+#pragma unroll
+            for (int ww = 1; ww < kWaves; ++ww) y += s.ypart[ww][tid];
+            const float e = (y + b3) - b.label[i];
             d = 2.f * e / (float)b.count;
             e2 = (double)e * (double)e;
         }
-        s.dy[threadIdx.x] = d;
-        s.e2[threadIdx.x] = e2;
-    }
-    // transposes of a0 and a1 for the weight-gradient GEMMs
-    for (int i = threadIdx.x; i < kMlpTile * kMlpInPad; i += 256) {
-        const int r = i / kMlpInPad, k = i % kMlpInPad;
-        s.a0t[k * kMlpTile + r] = s.f.a0[r * kLd0 + k];
-    }
-    for (int i = threadIdx.x; i < kMlpTile * kMlpHid; i += 256) {
-        const int r = i / kMlpHid, k = i % kMlpHid;
-        s.a1t[k * kMlpTile + r] = s.f.a1[r * kLd1 + k];
+        s.dy[tid] = d;
+        s.e2[tid] = e2;
     }
     __syncthreads();
     // w3, b3 gradients; dz2 = dy w3 (h2 > 0)
-    const float* w3 = m.params + kOffW3;
-    if (threadIdx.x < kMlpHid) {
+    if (tid < kMlpHid) {
         float g = 0.f;
-        for (int r = 0; r < kMlpTile; ++r) g += s.h[r * kMlpHid + threadIdx.x] * s.dy[r];
-        grads[kOffW3 + threadIdx.x] = g;
-    } else if (threadIdx.x == kMlpHid) {
+#pragma unroll 16
+        for (int r = 0; r < kMlpTile; ++r) g += s.h[r * kLdH + tid] * s.dy[r];
+        grads[kOffW3 + tid] = g;
+    } else if (tid == 2 * kMlpHid) {
         float g = 0.f;
         for (int r = 0; r < kMlpTile; ++r) g += s.dy[r];
         grads[kOffB3] = g;
-    } else if (threadIdx.x == kMlpHid + 1) {
-        double l = 0.0;
-        for (int r = 0; r < kMlpTile; ++r) l += s.e2[r];
-        loss_part[blockIdx.x] = l;
+    } else if (tid == 3 * kMlpHid) {
+        double sum = 0.0;
+        for (int r = 0; r < kMlpTile; ++r) sum += s.e2[r];
+        loss_part[blockIdx.x] = sum;
     }
-    __syncthreads();
-    for (int i = threadIdx.x; i < kMlpTile * kMlpHid; i += 256) {
-        const int r = i / kMlpHid, j = i % kMlpHid;
-        const float d = s.h[i] > 0.f ? s.dy[r] * w3[j] : 0.f;
-        s.h[i] = d;
-        const uint16_t bd = bf16_bits(d);
-        s.dz2[i] = bd;
-        s.dzt[j * kMlpTile + r] = bd;
+    float d2[2][4];
+    const float dyr = s.dy[16 * ti + lr];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int unit = 32 * w + 16 * j + lq, row = 16 * ti + lr;
+        uint16_t bd[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            d2[j][q] = h2[j][q] > 0.f ? dyr * s.w3[unit + q] : 0.f;
+            bd[q] = bf16_bits(d2[j][q]);
+            s.dzt[(unit + q) * kLdT + row] = bd[q];
+        }
+        *reinterpret_cast<uint2*>(s.dz2 + row * kLd1 + unit) =
+            make_uint2((uint32_t)bd[0] | ((uint32_t)bd[1] << 16), (uint32_t)bd[2] | ((uint32_t)bd[3] << 16));
     }
+    __syncthreads();  // h2 is read
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+        *reinterpret_cast<float4*>(s.h + (16 * ti + lr) * kLdH + 32 * w + 16 * j + lq) =
+            make_float4(d2[j][0], d2[j][1], d2[j][2], d2[j][3]);
     __syncthreads();
     store_column_sums(s.h, grads + kOffB2);
     // dW2[i][o] = sum_m a1[m][i] dz2[m][o]: D[o][i] = dz2t[o][.] . a1t[i][.], 64 tiles of 16x16, K = 64 rows
-    for (int t = w; t < 64; t += 4) {
+    for (int t = wave; t < 64; t += kGradWaves) {
         const int ot = t >> 3, it = t & 7;
         f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int ks = 0; ks < kMlpTile / 32; ++ks)
-            acc = mfma_16x16x32(s.dzt + (16 * ot) * kMlpTile + 32 * ks, kMlpTile, s.a1t + (16 * it) * kMlpTile + 32 * ks,
-                                kMlpTile, acc);
-        const int i = 16 * it + (l & 15);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int o = 16 * ot + 4 * (l >> 4) + q;
-            grads[kOffW2 + i * kMlpHid + o] = acc[q];
-        }
+            acc = mfma_16x16x32(s.dzt + (16 * ot) * kLdT + 32 * ks, kLdT, s.a1t + (16 * it) * kLdT + 32 * ks, kLdT, acc);
+        *reinterpret_cast<float4*>(grads + kOffW2 + (16 * it + lr) * kMlpHid + 16 * ot + lq) =
+            make_float4(acc[0], acc[1], acc[2], acc[3]);
     }
-    __syncthreads();
-    // dh1[m][i] = sum_o dz2[m][o] W2[i][o]; dz1 = dh1 (a1 > 0)
-    for (int it = 0; it < kMlpHid / 16; ++it) {
+    // dh1[m][i] = sum_o dz2[m][o] W2[i][o]; dz1 = dh1 (a1 > 0): row tile w, hidden tiles ti and ti + 4
+    float d1[2][4];
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+        const int it = ti + 4 * half;
         f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int ks = 0; ks < kMlpHid / 32; ++ks)
-            acc = mfma_16x16x32(s.dz2 + (16 * w) * kMlpHid + 32 * ks, kMlpHid, m.w2 + (16 * it) * kMlpHid + 32 * ks,
-                                kMlpHid, acc);
-        const int i = 16 * it + (l & 15);
+            acc = mfma_16x16x32(s.dz2 + (16 * w) * kLd1 + 32 * ks, kLd1, m.w2 + (16 * it) * kMlpHid + 32 * ks, kMlpHid, acc);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            d1[half][q] = bf16_float(s.a1[(16 * w + lq + q) * kLd1 + 16 * it + lr]) > 0.f ? acc[q] : 0.f;
+    }
+    __syncthreads();  // dz2 and its transpose are read
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+        const int i = 16 * (ti + 4 * half) + lr, row = 16 * w + lq;
+        uint16_t bd[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const int r = 16 * w + 4 * (l >> 4) + q;
-            const float d = bf16_float(s.f.a1[r * kLd1 + i]) > 0.f ? acc[q] : 0.f;
-            s.h[r * kMlpHid + i] = d;
-            s.dzt[i * kMlpTile + r] = bf16_bits(d);
+            s.h[(row + q) * kLdH + i] = d1[half][q];
+            bd[q] = bf16_bits(d1[half][q]);
         }
+        *reinterpret_cast<uint2*>(s.dzt + i * kLdT + row) =
+            make_uint2((uint32_t)bd[0] | ((uint32_t)bd[1] << 16), (uint32_t)bd[2] | ((uint32_t)bd[3] << 16));
     }
     __syncthreads();
     store_column_sums(s.h, grads + kOffB1);
     // dW1[k][o] = sum_m a0[m][k] dz1[m][o]: D[o][k] = dz1t[o][.] . a0t[k][.], 8 x 4 tiles (inputs >= 35 skipped)
-    for (int t = w; t < 32; t += 4) {
+    for (int t = wave; t < 32; t += kGradWaves) {
         const int ot = t >> 2, kt = t & 3;
         f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int ks = 0; ks < kMlpTile / 32; ++ks)
-            acc = mfma_16x16x32(s.dzt + (16 * ot) * kMlpTile + 32 * ks, kMlpTile, s.a0t + (16 * kt) * kMlpTile + 32 * ks,
-                                kMlpTile, acc);
-        const int k = 16 * kt + (l & 15);
-        if (k < kMlpIn) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int o = 16 * ot + 4 * (l >> 4) + q;
-                grads[kOffW1 + k * kMlpHid + o] = acc[q];
-            }
-        }
+            acc = mfma_16x16x32(s.dzt + (16 * ot) * kLdT + 32 * ks, kLdT, s.a0t + (16 * kt) * kLdT + 32 * ks, kLdT, acc);
+        const int k = 16 * kt + lr;
+        if (k < kMlpIn)
+            *reinterpret_cast<float4*>(grads + kOffW1 + k * kMlpHid + 16 * ot + lq) =
+                make_float4(acc[0], acc[1], acc[2], acc[3]);
     }
+}
+
+// Whether parameter i is one of W1's padding rows, which stay zero.
+__device__ __forceinline__ bool mlp_padding(int i) { return i >= kOffW1 + kMlpIn * kMlpHid && i < kOffB1; }
+
+// Parameter i's gradient: the tiles' partial ones summed in tile order.
+__device__ __forceinline__ float mlp_tile_sum(const float* partial, uint32_t tiles, int i) {
+    float g = 0.f;
+#pragma unroll 8
+    for (uint32_t t = 0; t < tiles; ++t) g += partial[(uint64_t)t * kMlpPartial + i];
+    return g;
 }
 
 // grads[i] = the tiles' partial gradients summed in tile order (W1's padding rows zero); loss[0] likewise.
@@ -421,24 +516,38 @@ __global__ void __launch_bounds__(256) k_mlp_reduce(const float* __restrict__ pa
         loss[0] = l;
     }
     if (i >= kMlpParams) return;
-    float g = 0.f;
-    if (!(i >= kOffW1 + kMlpIn * kMlpHid && i < kOffB1))
-        for (uint32_t t = 0; t < tiles; ++t) g += partial[(uint64_t)t * kMlpParams + i];
-    grads[i] = g;
+    grads[i] = mlp_padding(i) ? 0.f : mlp_tile_sum(partial, tiles, i);
 }
 
-__global__ void __launch_bounds__(256) k_mlp_adam(float* __restrict__ p, float* __restrict__ am,
-                                                  float* __restrict__ av, const float* __restrict__ g, float lr,
-                                                  float beta1, float beta2, float eps, float c1, float c2) {
+// A training step after its tiles: each parameter's gradient summed, its Adam update, and its bf16 copies, in one
+// launch (three launches and 11 us before); the step's squared error to loss[0].
+__global__ void __launch_bounds__(256) k_mlp_step(const float* __restrict__ partial, uint32_t tiles,
+                                                  const double* __restrict__ loss_part, double* __restrict__ loss,
+                                                  const MlpTrain t, float lr, float beta1, float beta2, float eps,
+                                                  float c1, float c2) {
     const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= kMlpParams) return;
-    if (i >= kOffW1 + kMlpIn * kMlpHid && i < kOffB1) return;  // W1's padding rows stay zero
-    const float gi = g[i];
-    const float mi = beta1 * am[i] + (1.f - beta1) * gi;
-    const float vi = beta2 * av[i] + (1.f - beta2) * gi * gi;
-    am[i] = mi;
-    av[i] = vi;
-    p[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+    if (i == 0) {
+        double l = 0.0;
+        for (uint32_t k = 0; k < tiles; ++k) l += loss_part[k];
+        loss[0] = l;
+    }
+    if (i >= kMlpParams || mlp_padding(i)) return;
+    const float gi = mlp_tile_sum(partial, tiles, i);
+    const float mi = beta1 * t.adam_m[i] + (1.f - beta1) * gi;
+    const float vi = beta2 * t.adam_v[i] + (1.f - beta2) * gi * gi;
+    t.adam_m[i] = mi;
+    t.adam_v[i] = vi;
+    float p = t.params[i];
+    p -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+    t.params[i] = p;
+    if (i < kOffB1) {
+        t.w1t[(i % kMlpHid) * kMlpInPad + i / kMlpHid] = bf16_bits(p);
+    } else if (i >= kOffW2 && i < kOffB2) {
+        const int k = (i - kOffW2) / kMlpHid, n = (i - kOffW2) % kMlpHid;
+        const uint16_t v = bf16_bits(p);
+        t.w2t[n * kMlpHid + k] = v;
+        t.w2[k * kMlpHid + n] = v;
+    }
 }
 
 // The first nonempty bucket at or after b among this workgroup's (b, b + gridDim.x, ...); num_buckets when none.
@@ -509,7 +618,7 @@ k_mlp_score(const MlpDev m, const ScoreArgs<T> a) {
             a.score[prev] = mlp_output(fw, s.ypart[parity ^ 1], r) + lnc[parity ^ 1][r];
         mlp_layer1(fw, s);
         __syncthreads();
-        mlp_layer2(fw, s, nullptr, s.ypart[parity]);
+        mlp_layer2(fw, s, s.ypart[parity]);
         prev = start + t0 + r;
         prev_valid = valid;
         if (!more) break;
@@ -544,17 +653,21 @@ hipError_t launch_mlp_grad(hipStream_t st, const MlpDev& m, const MlpBatch& b, f
     const uint64_t tiles = (b.count + kMlpTile - 1) / kMlpTile;
     if (tiles > partial_tiles) return hipErrorInvalidValue;
     if (tiles)
-        hipLaunchKernelGGL(k_mlp_grad, dim3((uint32_t)tiles), dim3(256), 0, st, m, b, partial, loss_part);
+        hipLaunchKernelGGL(k_mlp_grad, dim3((uint32_t)tiles), dim3(kGradBlock), 0, st, m, b, partial, loss_part);
     hipLaunchKernelGGL(k_mlp_reduce, dim3((kMlpParams + 255) / 256), dim3(256), 0, st, partial, (uint32_t)tiles,
                        grads, loss_part, loss);
     return hipGetLastError();
 }
 
-hipError_t launch_mlp_adam(hipStream_t st, float* params, float* adam_m, float* adam_v, const float* grads, float lr,
-                           float beta1, float beta2, float eps, int step) {
+hipError_t launch_mlp_train_step(hipStream_t st, const MlpDev& m, const MlpBatch& b, const MlpTrain& t, float* partial,
+                                 double* loss_part, uint64_t partial_tiles, double* loss, float lr, float beta1,
+                                 float beta2, float eps, int step) {
+    const uint64_t tiles = (b.count + kMlpTile - 1) / kMlpTile;
+    if (tiles == 0 || tiles > partial_tiles) return hipErrorInvalidValue;
     const float c1 = 1.f - powf(beta1, (float)step), c2 = 1.f - powf(beta2, (float)step);
-    hipLaunchKernelGGL(k_mlp_adam, dim3((kMlpParams + 255) / 256), dim3(256), 0, st, params, adam_m, adam_v, grads,
-                       lr, beta1, beta2, eps, c1, c2);
+    hipLaunchKernelGGL(k_mlp_grad, dim3((uint32_t)tiles), dim3(kGradBlock), 0, st, m, b, partial, loss_part);
+    hipLaunchKernelGGL(k_mlp_step, dim3((kMlpParams + 255) / 256), dim3(256), 0, st, partial, (uint32_t)tiles, loss_part,
+                       loss, t, lr, beta1, beta2, eps, c1, c2);
     return hipGetLastError();
 }
 

@@ -188,3 +188,32 @@ def test_propagate_learned_matches_a_layer_by_layer_emulation(clifford_block):
                                                                got.coefficients_array())}
     want_terms = {(int(a), int(b)): float(v) for a, b, v in zip(x[:, 0], z[:, 0], c)}
     assert got_terms == want_terms  # same keys, coefficients equal as doubles
+
+
+@pytest.mark.parametrize("n,batch", [(1, 64), (63, 64), (64, 64), (65, 64), (200, 128), (1000, 1000), (1500, 1024)])
+def test_training_steps_are_the_gradients_and_adam(n, batch):
+    """A training step (its tiles' gradients, their sum, Adam and the bf16 copies in two launches) against the same step
+    taken from pp_model_gradient on the host in float32 numpy, over one epoch of whole and partial batches: full and
+    partial tiles.  Both round every operation to float32 once, so the parameters agree to a few of its last bits per
+    step; the next step's gradients are those of the device's own parameters."""
+    announce(f"mlp training steps n={n} batch={batch}")
+    rng = np.random.default_rng(n)
+    m = PL.Model(L.lattice_groups(8, 8), depth_scale=40.0, seed=11)
+    x, z, c, rem = samples(rng, n)
+    labels = (-0.3 * np.arange(n) / n + 0.1 * rng.standard_normal(n)).astype(np.float32)
+    # a one-batch epoch visits every sample, so its order does not matter to the gradient beyond rounding
+    seen = min(n, batch)
+    x, z, c, rem, labels = x[:seen], z[:seen], c[:seen], rem[:seen], labels[:seen]
+    before = m.get_params()
+    grad, loss = m.gradient(x, z, c, rem, labels)
+    got = m.train(x, z, c, rem, labels, epochs=1, batch=batch, lr=1e-3, seed=3)
+    after = m.get_params()
+    assert abs(got - loss) <= 1e-5 * max(1.0, loss)
+    # the first Adam step from zero moments moves each parameter by lr g / (|g| + eps'), at most lr
+    g = grad.astype(np.float64)
+    step = 1e-3 * g / (np.abs(g) + 1e-8)
+    moved = before.astype(np.float64) - after
+    # the batch order changes a gradient by its rounding only; where that rounding matters to the step, g is near eps
+    tol = 2e-6 + 1e-3 * np.minimum(1.0, 1e-5 * np.abs(g).max() / (np.abs(g) + 1e-8))
+    assert (np.abs(moved - step) <= tol).all(), float(np.abs(moved - step).max())
+    m.free()
