@@ -369,6 +369,7 @@ struct pp_sum {
     bool topn_seed_score = false;  // the seed is a score key (the learned pass), not a |c|^2 one
     double topn_width = 0;         // the next windowed selection's half-width around the seed (0: none yet)
     bool window_ready = false;     // d_window is zero between selections
+    bool octave_ready = false;     // d_octave's counts are zero between cuts
     uint64_t phys_len = 0;
     const uint8_t* pending_flags = nullptr;
     const float* pending_score = nullptr;  // the ranking score when the selection was by score
@@ -387,7 +388,8 @@ struct pp_sum {
     pp::TopnState* d_topn = nullptr;
     unsigned long long* d_hist = nullptr;
     pp::WindowCounts* d_window = nullptr;
-    unsigned char* d_fixed = nullptr;  // the allocation of d_stats, d_lag_counters, d_rows, d_topn, d_hist and d_window
+    pp::OctaveCounts* d_octave = nullptr;
+    unsigned char* d_fixed = nullptr;  // the allocation of d_stats, d_lag_counters, d_rows, d_topn, d_hist, d_window and d_octave
     uint32_t* d_redo = nullptr;  // pairs a join could not stage, for its redo launch
     uint64_t redo_cap = 0;
     float* d_score = nullptr;  // the learned pass's score per column position
@@ -545,8 +547,8 @@ pp_status alloc_fixed(pp_sum* s) {
     auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
     const size_t stats = (kStatSlots + kReadoutGroups + 8) * 8, rows = s->rows.size() * 8;
     const size_t o_rows = up(stats), o_topn = o_rows + up(rows), o_hist = o_topn + up(sizeof(TopnState));
-    const size_t o_window = o_hist + up(kSeededHistWords * 8);
-    pp_status st = dev_alloc(ctx, (void**)&s->d_fixed, o_window + sizeof(WindowCounts));
+    const size_t o_window = o_hist + up(kSeededHistWords * 8), o_octave = o_window + up(sizeof(WindowCounts));
+    pp_status st = dev_alloc(ctx, (void**)&s->d_fixed, o_octave + sizeof(OctaveCounts));
     if (st != PP_OK) return st;
     s->d_stats = (unsigned long long*)s->d_fixed;
     s->d_lag_counters = s->d_stats + kStatSlots + kReadoutGroups;
@@ -554,6 +556,7 @@ pp_status alloc_fixed(pp_sum* s) {
     s->d_topn = (TopnState*)(s->d_fixed + o_topn);
     s->d_hist = (unsigned long long*)(s->d_fixed + o_hist);
     s->d_window = (WindowCounts*)(s->d_fixed + o_window);
+    s->d_octave = (OctaveCounts*)(s->d_fixed + o_octave);
     return PP_OK;
 }
 
@@ -1960,7 +1963,7 @@ bool batch_topn_enabled() {
 }
 pp_status topn_device(pp_sum* s, uint64_t n, const float* score = nullptr,
                       bool defer = false);  // pp_topn_impl.inc
-pp_status approx_topn_device(pp_sum* s, uint64_t n);  // pp_topn_impl.inc
+pp_status approx_topn_device(pp_sum* s, uint64_t n, bool defer = false);  // pp_topn_impl.inc
 
 pp_status check_channels(pp_sum* s, const pp_channel* channels, uint64_t n_channels) {
     for (uint64_t i = 0; i < n_channels; ++i)
@@ -3363,9 +3366,9 @@ pp_status pp_truncate_approx_topn(pp_sum* s, uint64_t n) {
 
 pp_status RunPlanner::finish_run(pp_sum* s, bool defer) const {
     if (!finalizes) return PP_OK;
-    if (policy->has_topn == 2) return pp_truncate_approx_topn(s, policy->topn);
-    if (!defer) return pp_truncate_topn(s, policy->topn);
+    if (!defer) return policy->has_topn == 2 ? pp_truncate_approx_topn(s, policy->topn) : pp_truncate_topn(s, policy->topn);
     if (s->len <= policy->topn) return PP_OK;
+    if (policy->has_topn == 2) return approx_topn_device(s, policy->topn, true);
     return topn_device(s, policy->topn, nullptr, true);
 }
 

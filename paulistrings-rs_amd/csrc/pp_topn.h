@@ -263,6 +263,44 @@ struct OctaveCutArgs {
     uint64_t out_cap;
 };
 
+// The cut on the device, for a layout whose reference buckets gather whole device buckets: the octave counts and the
+// boundary octave, its terms per device bucket, the reference bucket where the quota runs out with its first terms in
+// canonical order, and a flag for every boundary term.  It leaves a TopnState whose decided bits are the octave, so a
+// layer can read its input through it.
+constexpr uint32_t kOctaveCopies = 8;
+constexpr uint32_t kCutRows = 2048;  // boundary terms of the split bucket the last workgroup orders
+struct OctaveCounts {  // zero before the scan; the edge launch clears it
+    uint32_t hist[kOctaveCopies][kOctaveBins];
+    uint32_t nan[kOctaveCopies * 32];  // one line each
+    // the edge's answer
+    uint32_t bin;
+    unsigned long long quota;  // boundary terms to keep
+    unsigned long long above;  // terms above the boundary octave that are no NaN
+};
+
+template <int W, typename T>
+struct OctaveSelectArgs {
+    const uint64_t* x;
+    const uint64_t* z;
+    const T* c;
+    uint64_t cap;
+    const uint64_t* start;
+    const uint32_t* len;
+    uint32_t num_buckets;
+    uint32_t ref_buckets;  // at most num_buckets
+    uint32_t buckets_per_block;
+    uint64_t n;  // terms to keep
+    OctaveCounts* counts;
+    uint32_t* boundary;  // per device bucket: terms of the boundary octave
+    uint32_t* split;     // [0] the reference bucket where the quota runs out (ref_buckets: nowhere)
+    uint8_t* flags;
+    TopnState* state;
+    unsigned long long* host;  // pinned: [0] 1 cut, 2 the split bucket holds more than kCutRows; [1] terms that stay;
+    unsigned long long seq;    // then [4] = seq
+};
+template <int W, typename T>
+hipError_t launch_octave_select(hipStream_t st, const OctaveSelectArgs<W, T>& a);
+
 template <typename T>
 hipError_t launch_octave_hist(hipStream_t st, const OctaveHistArgs<T>& a, uint32_t blocks);
 template <int W, typename T>

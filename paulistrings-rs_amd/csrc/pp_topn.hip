@@ -872,6 +872,246 @@ __device__ __forceinline__ int octave_side(uint64_t u, uint32_t bin) {
     return o > bin ? 1 : (o == bin ? 0 : -1);
 }
 
+// ---- the cut on the device: five launches and one wait of the host
+
+// Octave counts, a copy of the LDS histogram per wave (a wave's keys share a few octaves).
+template <int W, typename T>
+__global__ void __launch_bounds__(kBlock) k_octave_scan(const OctaveSelectArgs<W, T> a) {
+    __shared__ uint32_t h[kWaves][kOctaveBins];
+    __shared__ RowList list;
+    __shared__ uint32_t nan;
+    for (uint32_t i = threadIdx.x; i < kWaves * kOctaveBins; i += kBlock) (&h[0][0])[i] = 0u;
+    if (threadIdx.x == 0) nan = 0u;
+    const uint32_t b_lo = blockIdx.x * a.buckets_per_block;
+    const uint32_t nb = min(a.num_buckets, b_lo + a.buckets_per_block) - b_lo;  // <= kHistBucketsMax
+    const uint32_t total = list_rows(a.start, a.len, b_lo, nb, list);
+    uint32_t j = 0;
+    for (uint32_t g0 = threadIdx.x; g0 < total; g0 += 8 * kBlock) {
+        uint64_t pos[8];
+        bool in[8];
+        list_positions(list, total, g0, j, pos, in);
+        T c[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q)
+            if (in[q]) c[q] = a.c[pos[q]];
+#pragma unroll
+        for (int q = 0; q < 8; ++q)
+            if (in[q]) {
+                const uint64_t u = magnitude_bits<T>(c[q]);
+                atomicAdd(&h[wave_id()][octave_of(u)], 1u);
+                if (is_nan_bits(u)) atomicAdd(&nan, 1u);
+            }
+    }
+    __syncthreads();
+    const uint32_t copy = blockIdx.x % kOctaveCopies;
+    for (uint32_t i = threadIdx.x; i < kOctaveBins; i += kBlock) {
+        uint32_t v = 0;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) v += h[w][i];
+        if (v) atomicAdd(&a.counts->hist[copy][i], v);
+    }
+    if (threadIdx.x == 0 && nan) atomicAdd(&a.counts->nan[copy * 32], nan);
+}
+
+// octave_edge (builtin.rs:320-352): whole octaves from the top while they fit in n; the first that does not is the
+// boundary.  One workgroup, two octaves a thread.
+template <int W, typename T>
+__global__ void __launch_bounds__(kFinishBlock) k_octave_edge(const OctaveSelectArgs<W, T> a) {
+    constexpr uint32_t PER = kOctaveBins / kFinishBlock;
+    __shared__ uint64_t part[kFinishBlock / 64];
+    OctaveCounts& w = *a.counts;
+    const uint32_t tid = threadIdx.x;
+    uint64_t mine[PER], sum = 0;
+#pragma unroll
+    for (uint32_t q = 0; q < PER; ++q) {
+        mine[q] = 0;
+#pragma unroll
+        for (uint32_t c = 0; c < kOctaveCopies; ++c) mine[q] += w.hist[c][tid * PER + q];
+        sum += mine[q];
+    }
+    uint64_t suffix = sum;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint64_t o = __shfl_down(suffix, d, 64);
+        if (lane_id() + (uint32_t)d < 64u) suffix += o;
+    }
+    if (lane_id() == 0) part[wave_id()] = suffix;
+    __syncthreads();
+    uint64_t above = suffix - sum;
+    for (uint32_t v = wave_id() + 1; v < kFinishBlock / 64; ++v) above += part[v];
+    if (above <= a.n && above + sum > a.n) {  // this thread's octaves hold the boundary
+        for (uint32_t q = PER; q-- > 0;) {
+            if (above + mine[q] > a.n) {
+                uint64_t nan = 0;
+                for (uint32_t c = 0; c < kOctaveCopies; ++c) nan += w.nan[c * 32];
+                const uint32_t bin = tid * PER + q;
+                w.bin = bin;
+                w.quota = a.n - above;
+                w.above = above - (bin < kOctaveBins - 1 ? nan : 0ull);  // NaNs count in the last octave, and go
+                break;
+            }
+            above += mine[q];
+        }
+    }
+    __syncthreads();
+    for (uint32_t i = tid; i < kOctaveCopies * kOctaveBins; i += kFinishBlock) (&w.hist[0][0])[i] = 0u;
+    if (tid < kOctaveCopies) w.nan[tid * 32] = 0u;
+}
+
+// A wave per device bucket: its terms of the boundary octave counted (FLAGS false), or flagged by whether the quota
+// reaches their reference bucket (FLAGS true; the split bucket's are flagged already).
+template <int W, typename T, bool FLAGS>
+__global__ void __launch_bounds__(kBlock) k_octave_bucket(const OctaveSelectArgs<W, T> a) {
+    const uint32_t b = blockIdx.x * kWaves + wave_id();
+    if (b >= a.num_buckets) return;  // the whole wave
+    const uint32_t bin = a.counts->bin;
+    const uint32_t n = a.len[b];
+    const uint64_t s = a.start[b];
+    uint8_t flag = 0;
+    if constexpr (FLAGS) {
+        const uint32_t rb = b & (a.ref_buckets - 1u), split = a.split[0];
+        if (rb == split) return;
+        flag = rb < split ? 1 : 0;
+    }
+    uint32_t count = 0;
+    for (uint32_t r0 = lane_id(); r0 < n; r0 += 4 * 64) {
+        T c[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (r0 + q * 64 < n) c[q] = a.c[s + r0 + q * 64];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            if (r0 + q * 64 >= n || octave_side(magnitude_bits<T>(c[q]), bin) != 0) continue;
+            if constexpr (FLAGS) a.flags[s + r0 + q * 64] = flag;
+            else ++count;
+        }
+    }
+    if constexpr (!FLAGS) {
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) count += (uint32_t)__shfl_xor((int)count, d, 64);
+        if (lane_id() == 0) a.boundary[b] = count;
+    }
+}
+
+// QuotaSplit::new (builtin.rs:160-197): the reference bucket where the quota runs out, and its first terms in
+// lexicographic order ranked by counting.  One workgroup; each thread owns a run of reference buckets.
+template <int W, typename T>
+__global__ void __launch_bounds__(kFinishBlock) k_octave_split(const OctaveSelectArgs<W, T> a) {
+    __shared__ uint64_t part[kFinishBlock / 64];
+    __shared__ uint64_t kx[W][kCutRows], kz[W][kCutRows], kp[kCutRows];
+    __shared__ uint32_t held, split;
+    __shared__ uint64_t left;
+    const OctaveCounts& w = *a.counts;
+    const uint32_t tid = threadIdx.x, parts = a.num_buckets / a.ref_buckets;
+    if (tid == 0) {
+        held = 0u;
+        split = a.ref_buckets;
+        left = 0;
+    }
+    const uint32_t per = (a.ref_buckets + kFinishBlock - 1) / kFinishBlock;
+    const uint32_t lo = min(tid * per, a.ref_buckets), hi = min(lo + per, a.ref_buckets);
+    auto ref_count = [&](uint32_t rb) {
+        uint32_t v = 0;
+#pragma unroll 4
+        for (uint32_t e = 0; e < parts; ++e) v += a.boundary[rb + e * a.ref_buckets];
+        return v;
+    };
+    uint64_t mine = 0;
+    for (uint32_t e = 0; e < parts; ++e) {
+#pragma unroll 4
+        for (uint32_t rb = lo; rb < hi; ++rb) mine += a.boundary[rb + e * a.ref_buckets];
+    }
+    uint64_t inc = mine;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint64_t o = __shfl_up(inc, d, 64);
+        if (lane_id() >= (uint32_t)d) inc += o;
+    }
+    if (lane_id() == 63) part[wave_id()] = inc;
+    __syncthreads();
+    uint64_t seen = inc - mine, total = 0;
+    for (uint32_t v = 0; v < kFinishBlock / 64; ++v) {
+        seen += v < wave_id() ? part[v] : 0ull;
+        total += part[v];
+    }
+    const uint64_t quota = w.quota;
+    if (seen <= quota && seen + mine > quota)  // this thread's buckets hold the split
+        for (uint32_t rb = lo; rb < hi; ++rb) {
+            const uint32_t v = ref_count(rb);
+            if (seen + v > quota) {
+                split = rb;
+                left = quota - seen;
+                break;
+            }
+            seen += v;
+        }
+    __syncthreads();
+    const uint32_t sb = split;
+    const uint64_t remaining = left;
+    if (sb < a.ref_buckets) {
+        for (uint32_t e = 0; e < parts; ++e) {
+            const uint32_t b = sb + e * a.ref_buckets;
+            const uint32_t n = a.len[b];
+            const uint64_t s = a.start[b];
+            for (uint32_t r = tid; r < n; r += kFinishBlock) {
+                if (octave_side(magnitude_bits<T>(a.c[s + r]), w.bin) != 0) continue;
+                const uint32_t slot = atomicAdd(&held, 1u);
+                if (slot >= kCutRows) continue;
+                const Key<W> k = load_key<W>(a.x, a.z, a.cap, s + r);
+#pragma unroll
+                for (int v = 0; v < W; ++v) {
+                    kx[v][slot] = k.x[v];
+                    kz[v][slot] = k.z[v];
+                }
+                kp[slot] = s + r;
+            }
+        }
+        __syncthreads();
+        const uint32_t m = min(held, kCutRows);
+        for (uint32_t i = tid; i < m; i += kFinishBlock) {
+            uint32_t before = 0;
+            for (uint32_t q = 0; q < m; ++q) {
+                int order = 0;
+#pragma unroll
+                for (int v = 0; v < W; ++v)
+                    if (order == 0) order = kx[v][q] < kx[v][i] ? -1 : kx[v][q] > kx[v][i] ? 1 : 0;
+#pragma unroll
+                for (int v = 0; v < W; ++v)
+                    if (order == 0) order = kz[v][q] < kz[v][i] ? -1 : kz[v][q] > kz[v][i] ? 1 : 0;
+                before += order < 0;
+            }
+            a.flags[kp[i]] = before < remaining ? 1 : 0;
+        }
+    }
+    if (tid == 0) {
+        a.split[0] = sb;
+        TopnState& st = *a.state;
+        st.prefix = (unsigned long long)w.bin << 52;
+        st.mask = 0xFFF0000000000000ull;
+        st.keep_all_finite = 0;
+        volatile unsigned long long* h = a.host;  // fine-grained host memory: the stores bypass the L2
+        h[0] = held > kCutRows ? 2 : 1;
+        h[1] = w.above + (sb < a.ref_buckets ? quota : total);
+        __builtin_amdgcn_s_waitcnt(0);  // the slot's words land before its sequence number
+        h[4] = a.seq;
+    }
+}
+
+template <int W, typename T>
+hipError_t launch_octave_select(hipStream_t st, const OctaveSelectArgs<W, T>& a) {
+    if (a.num_buckets == 0 || a.ref_buckets > a.num_buckets || a.buckets_per_block == 0 ||
+        a.buckets_per_block > kHistBucketsMax)
+        return hipErrorInvalidValue;
+    const uint32_t blocks = (a.num_buckets + a.buckets_per_block - 1) / a.buckets_per_block;
+    const uint32_t waves = (a.num_buckets + kWaves - 1) / kWaves;
+    hipLaunchKernelGGL((k_octave_scan<W, T>), dim3(blocks), dim3(kBlock), 0, st, a);
+    hipLaunchKernelGGL((k_octave_edge<W, T>), dim3(1), dim3(kFinishBlock), 0, st, a);
+    hipLaunchKernelGGL((k_octave_bucket<W, T, false>), dim3(waves), dim3(kBlock), 0, st, a);
+    hipLaunchKernelGGL((k_octave_split<W, T>), dim3(1), dim3(kFinishBlock), 0, st, a);
+    hipLaunchKernelGGL((k_octave_bucket<W, T, true>), dim3(waves), dim3(kBlock), 0, st, a);
+    return hipGetLastError();
+}
+
 template <int W, typename T>
 __global__ void __launch_bounds__(kBlock) k_octave_counts(const OctaveCutArgs<W, T> a) {
     const uint32_t b = blockIdx.x;
@@ -1078,6 +1318,7 @@ template hipError_t launch_topn_hist_seeded<float>(hipStream_t, const TopnHistAr
 template hipError_t launch_octave_hist<double>(hipStream_t, const OctaveHistArgs<double>&, uint32_t);
 template hipError_t launch_octave_hist<float>(hipStream_t, const OctaveHistArgs<float>&, uint32_t);
 #define PP_TOPN_INSTANTIATE(W, T)                                                                       \
+    template hipError_t launch_octave_select<W, T>(hipStream_t, const OctaveSelectArgs<W, T>&);         \
     template hipError_t launch_topn_window<W, T>(hipStream_t, const WindowArgs<W, T>&);                 \
     template hipError_t launch_topn_gather_ties<W, T>(hipStream_t, const TopnTieArgs<W, T>&, uint32_t); \
     template hipError_t launch_topn_gather_batch<W, T>(hipStream_t, const TopnTieArgs<W, T>*, const uint32_t*, \
