@@ -12,6 +12,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <memory>
 #include <mutex>
 #include <new>
@@ -3095,7 +3096,10 @@ namespace {
 // bounds: a rotation layer at most doubles the rows, and an output bucket draws on two input buckets, so at most
 // doubles the longest bucket.  A layer whose bounds do not fit (a pair past the largest a join stages, a column set
 // that must grow), a sum large enough for the in-place layer, or a table that is not a rotation drains the queue and
-// takes the synchronous path.  The results are the same either way: only when the host learns the counts changes.
+// takes the synchronous path.  Under a layer pass (TopN, ApproxTopN, the learned pass) a layer is queued while its bound
+// stays within the cap: the pass then does nothing after it, whatever its exact length.  The results are the same either
+// way: only when the host learns the counts changes.  A small layer costs 13 us queued and 30 when its counts are read
+// before the next.
 
 constexpr uint64_t kLagMaxRows = 1ull << 20;  // above this a layer is bandwidth-bound and its synchronization noise
 constexpr uint32_t kLagDepth = 1;             // layers whose counts may still be on their way when one is queued
@@ -3145,9 +3149,11 @@ pp_status launch_join_small(pp_sum* s, int out, const Prepared& p, const KeepPro
     return PP_OK;
 }
 
-// run_layers under a policy with no layer pass, its rotation layers queued ahead of their counts.  The planner's
-// bookkeeping (the reference's bucket count at every run start) runs as each length arrives.
-pp_status propagate_lagged(pp_sum* s, const RunPlanner& plan, const KeepProgram& keep, uint64_t* layer_len) {
+// run_layers, its small rotation layers queued ahead of their counts; finish(end) is the layer pass after the run that
+// ends at layer `end`.  The planner's bookkeeping (the reference's bucket count at every run start) runs as each length
+// arrives.
+pp_status propagate_lagged(pp_sum* s, const RunPlanner& plan, const KeepProgram& keep, uint64_t* layer_len,
+                           const std::function<pp_status(uint64_t)>& finish) {
     pp_context* ctx = s->ctx;
     pp_status st;
     for (hipEvent_t& e : ctx->lag_ev)
@@ -3214,10 +3220,14 @@ pp_status propagate_lagged(pp_sum* s, const RunPlanner& plan, const KeepProgram&
     while (i < n) {
         if (queued == 0 && i == run_end) run_end = plan.start_run(s, i);
         const Prepared p = plan.prepared(s, i);
-        bool lag = p.rotation && !p.key_preserving;
+        bool lag = p.rotation && !p.key_preserving && !s->pending_topn;
         if (lag && is_permutation_step(p) && i + 1 < n &&
             is_permutation_step(plan.prepared(s, i + 1)))
             lag = false;  // the start of a permutation run: walked in one pass
+        // the rows a layer may queue from: below the in-place layer's, and under a layer pass half its cap
+        const uint64_t small = std::min({kLagMaxRows, plan.limit / 2,
+                                         ctx->tuning.join_in_place ? in_place_min_rows() - 1 : kLagMaxRows});
+        if (queued == 0 && s->len > small) lag = false;
         if (lag && queued == 0) {
             // exact counts: the device bucketing for the layers to come, fine enough that a pair stays within the
             // join's largest stage under the doubled bound (but not so fine that the next settle coarsens it back)
@@ -3229,8 +3239,7 @@ pp_status propagate_lagged(pp_sum* s, const RunPlanner& plan, const KeepProgram&
             known_mb = s->max_bucket;
         }
         const uint64_t len_hi = known_len << queued, mb_hi = known_mb << queued;
-        lag = lag && len_hi <= kLagMaxRows && 2 * mb_hi <= kMaxPairRows &&
-              (!ctx->tuning.join_in_place || len_hi < in_place_min_rows());
+        lag = lag && len_hi <= small && 2 * mb_hi <= kMaxPairRows;
         const int out = 1 - s->cur;
         const uint32_t B = 1u << s->device_bits;
         const uint64_t need = 2 * len_hi + (uint64_t)kSegAlign * B;
@@ -3251,7 +3260,8 @@ pp_status propagate_lagged(pp_sum* s, const RunPlanner& plan, const KeepProgram&
             if (i == run_end) run_end = plan.start_run(s, i);
             const uint64_t end = run_end;
             if ((st = plan.apply_run(s, i, end, keep, layer_len ? layer_len + i : nullptr)) != PP_OK) return st;
-            if ((st = plan.finish_run(s, end < n)) != PP_OK) return st;
+            if ((st = finish(end)) != PP_OK) return st;
+            if (layer_len && plan.finalizes) layer_len[end - 1] = s->len;
             if ((st = debug_check(s)) != PP_OK) return st;
             known_len = s->len;
             known_mb = s->max_bucket;
@@ -3309,8 +3319,9 @@ pp_status pp_propagate(pp_sum* s, const pp_channel* channels, uint64_t n_channel
     if ((st = check_channels(s, channels, n_channels)) != PP_OK) return st;
     const RunPlanner plan{channels, n_channels, direction == PP_HEISENBERG, policy, target, min_buckets};
     const KeepProgram keep = lower_policy(policy);
-    if (!plan.finalizes && !class_rotation_runs() && lagged_lengths())
-        return propagate_lagged(s, plan, keep, layer_len);
+    if (!class_rotation_runs() && lagged_lengths())
+        return propagate_lagged(s, plan, keep, layer_len,
+                                [&](uint64_t end) { return plan.finish_run(s, end < n_channels); });
     uint64_t i = 0, run_end = 0;  // layer i belongs to the planner's run ending at run_end
     std::vector<Prepared> window;
     std::vector<uint64_t> lens;

@@ -188,3 +188,20 @@ def test_in_place_layer_after_a_lagged_propagation(monkeypatch):
 
     got, want = by_key(h.x_array(), h.z_array(), h.coefficients_array()), by_key(o[0], o[1], o[2])
     assert all(np.array_equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("cap", [0, 1, 700, 5_000, 40_000, 1 << 40])
+@pytest.mark.parametrize("kind", ["topn", "approx"])
+@pytest.mark.parametrize("num_qubits,n", [(40, 300), (100, 6_000)])
+def test_layer_pass_joins_and_leaves_the_queue(monkeypatch, cap, kind, num_qubits, n):
+    """Under a layer pass a small layer is queued only while it cannot pass the cap: sums that start below the cap, reach
+    it, sit at it (and fall below it again under the threshold), with permutation runs and key-preserving layers between."""
+    announce(f"lagged under {kind}({cap}) qubits={num_qubits} n={n}")
+    rng = np.random.default_rng([num_qubits, n, cap % 1000])
+    x, z, c = random_sum(rng, n, num_qubits, 0.15)
+    circ = mixed_circuit(rng, num_qubits, 60)
+    pol = truncation.coeff(0.02) & (truncation.topn(cap) if kind == "topn" else truncation.approx_topn(cap))
+    got = run(monkeypatch, True, num_qubits, x, z, c, circ, "heisenberg", pol)
+    want = run(monkeypatch, False, num_qubits, x, z, c, circ, "heisenberg", pol)
+    assert_equal_runs(got, want)
+    assert got[4][0] == want[4][0]  # the reference's bucket count
