@@ -3098,7 +3098,7 @@ namespace {
 // that must grow), a sum large enough for the in-place layer, or a table that is not a rotation drains the queue and
 // takes the synchronous path.  Under a layer pass (TopN, ApproxTopN, the learned pass) a layer is queued while its bound
 // stays within the cap: the pass then does nothing after it, whatever its exact length.  The results are the same either
-// way: only when the host learns the counts changes.  A small layer costs 13 us queued and 30 when its counts are read
+// way: only when the host learns the counts changes.  A small layer costs 12 us queued and 30 when its counts are read
 // before the next.
 
 constexpr uint64_t kLagMaxRows = 1ull << 20;  // above this a layer is bandwidth-bound and its synchronization noise
@@ -3121,8 +3121,8 @@ bool small_join_fits(const pp_sum* s, const Prepared& p) {
     return join_stage_rows(s->ctx->tuning.stage_rows, lcap) >= lcap;
 }
 
-// Queue the small join of layer p from s's current columns into column set `out`, adding into `counters` (zero);
-// its extra workgroup publishes `prev` (the counters of the small join queued just before, or null) to the pinned
+// Queue the small join of layer p from s's current columns into column set `out`, its flags into `counters` (zero);
+// its extra workgroup publishes the counts of the small join queued just before (`prev`, or null) to the pinned
 // slot whose device address is `prev_host`, followed by `prev_seq`.
 pp_status launch_join_small(pp_sum* s, int out, const Prepared& p, const KeepProgram& keep,
                             unsigned long long* counters, unsigned long long* prev, unsigned long long* prev_host,
@@ -3137,7 +3137,6 @@ pp_status launch_join_small(pp_sum* s, int out, const Prepared& p, const KeepPro
         SmallJoinArgs<W, T> a{};
         a.j = join_args<W, T>(s, s, out, p, keep, delta, lcap);
         a.j.stats = counters;
-        a.j.count_totals = 1;
         a.orows = s->bk[out].rows;
         a.num_buckets = B;
         a.prev_counters = prev;
@@ -3173,8 +3172,8 @@ pp_status propagate_lagged(pp_sum* s, const RunPlanner& plan, const KeepProgram&
     // the last small join's counters, when no small join follows it to publish them
     auto publish = [&]() -> pp_status {
         if (unpublished < 0) return PP_OK;
-        PP_HIP(ctx, launch_publish_counters(ctx->stream, counters_of(unpublished), host_of(unpublished),
-                                            queued_seq[unpublished]));
+        PP_HIP(ctx, launch_publish_counters(ctx->stream, s->bk[s->cur].len, 1u << s->device_bits,
+                                            counters_of(unpublished), host_of(unpublished), queued_seq[unpublished]));
         unpublished = -1;
         return PP_OK;
     };

@@ -53,14 +53,13 @@ struct JoinArgs {
 
 // A small layer's join in one launch (k_rotation_join_small, a layout of at most kSmallJoinBuckets buckets, one
 // workgroup per pair): every workgroup lays out its own pair's output segments from the input lengths and joins the
-// pair, adding its rows and longest bucket to j.stats[0, 1] (zero before the launch; [2] flags an overflow, and
-// workgroup 0 writes the layout's end to [3]).  One workgroup more publishes the counters of the launch before
-// (prev_counters, complete at this launch's start) to that launch's pinned host slot, then a sequence number the
-// host waits on, and clears them for the launch after this one.
+// pair; j.stats[2] (zero before the launch) flags an overflow, and workgroup 0 writes the layout's end to [3].  One
+// workgroup more publishes the counts of the launch before, whose output j reads: that layout's rows and longest
+// bucket, prev_counters[2, 3] (cleared for the launch after this one), and last the sequence number the host waits on.
 constexpr uint32_t kSmallJoinBuckets = 2048;
 template <int W, typename T>
 struct SmallJoinArgs {
-    JoinArgs<W, T> j;          // j.ostart and j.olen are written; j.count_totals set; no redo queue
+    JoinArgs<W, T> j;          // j.ostart and j.olen are written; no totals, no redo queue
     uint32_t* orows;           // each output segment's room in rows
     uint32_t num_buckets;
     unsigned long long* prev_counters;  // 4 counters of the launch before, or null
@@ -304,8 +303,8 @@ template <int W, typename T>
 hipError_t launch_rotation_join_small(hipStream_t st, const SmallJoinArgs<W, T>& a);
 // The publication of a small join's counters with no launch after it (one workgroup): as the extra workgroup of
 // k_rotation_join_small does.
-hipError_t launch_publish_counters(hipStream_t st, unsigned long long* counters, unsigned long long* host,
-                                   unsigned long long seq);
+hipError_t launch_publish_counters(hipStream_t st, const uint32_t* len, uint32_t num_buckets,
+                                   unsigned long long* counters, unsigned long long* host, unsigned long long seq);
 // One layer for each of num_items sums (device arrays: items, pair_start = exclusive prefix of their pair counts,
 // total_pairs in all): their output offsets, the joins (each item staging its largest pair, scap = lcap), and
 // their counters, also gathered into out[4 i + 0..2] = rows, longest bucket, overflow flag.

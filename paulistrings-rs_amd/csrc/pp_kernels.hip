@@ -642,19 +642,45 @@ __global__ void __launch_bounds__(BLOCK) k_rotation_join(const JoinArgs<W, T> a)
     join_items<W, T, REDO, BLOCK, FILTER>(a, blockIdx.x, gridDim.x, count, lds, scan_scratch);
 }
 
-// A small layer's counters to the host: the four words, then (once they have landed) the sequence number the host
-// waits on; then the counters are cleared for the next launch that adds into them.  Thread 0 of one workgroup.
-__device__ __forceinline__ void publish_counters(unsigned long long* counters, unsigned long long* host,
-                                                 unsigned long long seq) {
+// A finished small layer's counts to the host, by one workgroup: its rows and longest bucket, summed here over its
+// bucket lengths, its overflow flag and layout end, then (once they have landed) the sequence number the host waits
+// on; the two counter words are cleared for the next layer that uses them.  Summing here, beside the next layer's
+// joins, keeps two same-line atomics per pair (12 ns each, one after another) off the end of the layer itself: the
+// 1080 layers of a 36-qubit Trotter evolution (up to 27735 terms) take 14.15 ms, 15.0 with the atomics.
+__device__ __forceinline__ void publish_counters(const uint32_t* __restrict__ len, uint32_t num_buckets,
+                                                 unsigned long long* counters, unsigned long long* host,
+                                                 unsigned long long seq, uint32_t* part) {
+    uint32_t rows = 0, longest = 0;  // a queued layer holds at most kLagMaxRows rows
+#pragma unroll
+    for (uint32_t k = 0; k < kSmallLensPerThread; ++k) {
+        const uint32_t i = threadIdx.x + k * kBlock;
+        const uint32_t n = i < num_buckets ? len[i] : 0u;
+        rows += n;
+        longest = max(longest, n);
+    }
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) {
+        rows += (uint32_t)__shfl_down((int)rows, d, 64);
+        longest = max(longest, (uint32_t)__shfl_down((int)longest, d, 64));
+    }
+    if (lane_id() == 0) {
+        part[wave_id()] = rows;
+        part[kWaves + wave_id()] = longest;
+    }
+    __syncthreads();
+    if (threadIdx.x) return;
+    rows = longest = 0;
+    for (int w = 0; w < kWaves; ++w) {
+        rows += part[w];
+        longest = max(longest, part[kWaves + w]);
+    }
     volatile unsigned long long* c = counters;
     volatile unsigned long long* h = host;  // fine-grained host memory: the stores bypass the L2
-    const unsigned long long rows = c[0], longest = c[1], flags = c[2], end = c[3];
+    const unsigned long long flags = c[2], end = c[3];
     h[0] = rows;
     h[1] = longest;
     h[2] = flags;
     h[3] = end;
-    c[0] = 0;
-    c[1] = 0;
     c[2] = 0;
     c[3] = 0;
     __builtin_amdgcn_s_waitcnt(0);  // the slot's words land before its sequence number
@@ -665,8 +691,8 @@ __device__ __forceinline__ void publish_counters(unsigned long long* counters, u
 // (each pair's rows rounded up to kSegAlign, as the offset scan lays them out) below each of its two buckets and in
 // all, over every bucket of the layout (at most kSmallJoinBuckets, read by every workgroup while its pair's first
 // rows load), writes its buckets' starts and rooms, and joins the pair.  The workgroup after the last pair
-// publishes the launch before's counters, which that launch's end made complete: a layer's counters reach the host
-// while the next layer runs, and no workgroup waits on another's.
+// publishes the counts of the launch before, whose output this launch reads: a layer's counts reach the host while the
+// next layer runs, and no workgroup waits on another's.
 template <int W, typename T>
 __global__ void __launch_bounds__(kBlock) k_rotation_join_small(const SmallJoinArgs<W, T> a) {
     extern __shared__ __align__(16) unsigned char lds[];
@@ -674,7 +700,8 @@ __global__ void __launch_bounds__(kBlock) k_rotation_join_small(const SmallJoinA
     __shared__ uint64_t part[3][kWaves];
     const JoinArgs<W, T>& j = a.j;
     if (blockIdx.x == j.num_cosets) {  // uniform: the publishing workgroup
-        if (threadIdx.x == 0 && a.prev_counters) publish_counters(a.prev_counters, a.prev_host, a.prev_seq);
+        if (a.prev_counters)
+            publish_counters(j.len, a.num_buckets, a.prev_counters, a.prev_host, a.prev_seq, scan_scratch);
         return;
     }
     uint64_t all = 0;
@@ -683,8 +710,11 @@ __global__ void __launch_bounds__(kBlock) k_rotation_join_small(const SmallJoinA
     if (blockIdx.x == 0 && threadIdx.x == 0) j.stats[3] = all;
 }
 
-__global__ void k_publish_counters(unsigned long long* counters, unsigned long long* host, unsigned long long seq) {
-    if (threadIdx.x == 0) publish_counters(counters, host, seq);
+__global__ void __launch_bounds__(kBlock) k_publish_counters(const uint32_t* len, uint32_t num_buckets,
+                                                             unsigned long long* counters, unsigned long long* host,
+                                                             unsigned long long seq) {
+    __shared__ uint32_t part[2 * kWaves];
+    publish_counters(len, num_buckets, counters, host, seq, part);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -1898,16 +1928,17 @@ hipError_t launch_rotation_join(hipStream_t st, const JoinArgs<W, T>& a, uint32_
 
 template <int W, typename T>
 hipError_t launch_rotation_join_small(hipStream_t st, const SmallJoinArgs<W, T>& a) {
-    if (a.j.num_cosets == 0 || a.num_buckets > kSmallJoinBuckets || a.j.redo_mode || a.j.filter || !a.j.count_totals)
+    if (a.j.num_cosets == 0 || a.num_buckets > kSmallJoinBuckets || a.j.redo_mode || a.j.filter || a.j.count_totals)
         return hipErrorInvalidValue;
     const size_t lds = join_lds_bytes<W, T>(a.j.scap, a.j.tcap_bits);
     hipLaunchKernelGGL((k_rotation_join_small<W, T>), dim3(a.j.num_cosets + 1), dim3(kBlock), lds, st, a);
     return hipGetLastError();
 }
 
-hipError_t launch_publish_counters(hipStream_t st, unsigned long long* counters, unsigned long long* host,
-                                   unsigned long long seq) {
-    hipLaunchKernelGGL(k_publish_counters, dim3(1), dim3(64), 0, st, counters, host, seq);
+hipError_t launch_publish_counters(hipStream_t st, const uint32_t* len, uint32_t num_buckets,
+                                   unsigned long long* counters, unsigned long long* host, unsigned long long seq) {
+    if (num_buckets > kSmallJoinBuckets) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_publish_counters, dim3(1), dim3(kBlock), 0, st, len, num_buckets, counters, host, seq);
     return hipGetLastError();
 }
 
