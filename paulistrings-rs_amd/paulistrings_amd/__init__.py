@@ -20,7 +20,7 @@ from dataclasses import dataclass, field
 import numpy as np
 
 from . import _native, circuits, gates, truncation
-from .circuits import Circuit
+from .circuits import CHANNEL_DTYPE, Circuit
 
 __all__ = ["PauliSum", "GpuPauliSum", "Circuit", "PropagationStats", "propagated", "propagated_with_stats",
            "propagate_batch",
@@ -430,6 +430,23 @@ def propagated_with_stats(initial: PauliSum, circuit: Circuit, policy=None, dire
     return out, stats
 
 
+def _channel_rows(channels: np.ndarray) -> np.ndarray:
+    """Channels as one contiguous CHANNEL_DTYPE array, one element per entry of the first axis."""
+    if channels.dtype == CHANNEL_DTYPE and channels.ndim == 1:
+        return np.ascontiguousarray(channels)
+    out = np.zeros(len(channels), CHANNEL_DTYPE)
+    for i, row in enumerate(channels):
+        r = np.asarray(row).reshape(-1)[0]
+        for w in range(4):
+            out["gx"][i, w], out["gz"][i, w] = int(r["gx"][w]), int(r["gz"][w])
+        out["theta"][i] = float(r["theta"])
+    return out
+
+
+def _channel_ptr(rows: np.ndarray):
+    return rows.ctypes.data_as(ctypes.POINTER(_native.Channel))
+
+
 def propagate_batch(sums, circuits, policies=None, directions=None, target_bucket_len: int = 1024,
                     min_buckets: int = 128) -> None:
     """Propagate many resident sums (``GpuPauliSum``, one context, one width and coefficient type) each through its
@@ -444,14 +461,11 @@ def propagate_batch(sums, circuits, policies=None, directions=None, target_bucke
     ctx = sums[0].ctx
     policies = list(policies) if policies is not None else [None] * len(sums)
     directions = list(directions) if directions is not None else [None] * len(sums)
-    chans, offsets = [], [0]
-    for c in circuits:
-        ch = c.channels() if isinstance(c, Circuit) else np.asarray(c)
-        chans.extend(ch)
+    chans = [_channel_rows(c.channels() if isinstance(c, Circuit) else np.asarray(c)) for c in circuits]
+    offsets = [0]
+    for ch in chans:
         offsets.append(offsets[-1] + len(ch))
-    arr = (_native.Channel * max(1, len(chans)))()
-    for i, row in enumerate(chans):
-        arr[i] = GpuPauliSum._channel(row)
+    arr = np.concatenate(chans)
     offs = (ctypes.c_uint64 * len(offsets))(*offsets)
     dirs = (ctypes.c_int * len(sums))(*[_parse_direction(d) for d in directions])
     pols = (_native.Policy * len(sums))(*[truncation.lower(p) for p in policies])
@@ -460,6 +474,7 @@ def propagate_batch(sums, circuits, policies=None, directions=None, target_bucke
     _native.check(_native.lib().pp_batch_create(ctx.handle, handles, len(sums), ctypes.byref(b)), ctx.handle)
     try:
         opts = _options(target_bucket_len, min_buckets)
-        _native.check(_native.lib().pp_batch_propagate(b, arr, offs, dirs, pols, ctypes.byref(opts)), ctx.handle)
+        _native.check(_native.lib().pp_batch_propagate(b, _channel_ptr(arr), offs, dirs, pols,
+                                                       ctypes.byref(opts)), ctx.handle)
     finally:
         _native.lib().pp_batch_free(b)

@@ -151,16 +151,14 @@ def truncate_learned(sum_, model: Model, n: int, remaining: float) -> None:
 def propagate_learned(sum_, circuit: Circuit, model: Model, keep: int, filter_policy=None, direction=None,
                       target_bucket_len: int = 1024, min_buckets: int = 128) -> None:
     """``propagate`` with the learned pass keeping ``keep`` terms after every run of layers."""
-    from . import GpuPauliSum, _options, _parse_direction
+    from . import _channel_ptr, _channel_rows, _options, _parse_direction
 
-    chans = circuit.channels()
-    arr = (_native.Channel * max(1, len(chans)))()
-    for i, row in enumerate(chans):
-        arr[i] = GpuPauliSum._channel(row)
+    chans = _channel_rows(circuit.channels())
     pol = truncation.lower(filter_policy)
     opts = _options(target_bucket_len, min_buckets)
-    _native.check(_bind().pp_propagate_learned(sum_._h, arr, len(chans), _parse_direction(direction), ctypes.byref(pol),
-                                               model._h, int(keep), ctypes.byref(opts), None), sum_.ctx.handle)
+    _native.check(_bind().pp_propagate_learned(sum_._h, _channel_ptr(chans), len(chans), _parse_direction(direction),
+                                               ctypes.byref(pol), model._h, int(keep), ctypes.byref(opts), None),
+                  sum_.ctx.handle)
 
 
 def readout_labels(terms_x, terms_z, circuit_rest: Circuit, state: str, policy=None, direction: str = "heisenberg",
