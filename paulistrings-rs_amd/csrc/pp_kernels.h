@@ -307,11 +307,16 @@ hipError_t launch_publish_counters(hipStream_t st, const uint32_t* len, uint32_t
                                    unsigned long long* counters, unsigned long long* host, unsigned long long seq);
 // One layer for each of num_items sums (device arrays: items, pair_start = exclusive prefix of their pair counts,
 // total_pairs in all): their output offsets, the joins (each item staging its largest pair, scap = lcap), and
-// their counters, also gathered into out[4 i + 0..2] = rows, longest bucket, overflow flag.
+// their counters, each item's to its pinned slot: rows, longest bucket, overflow flag, and last the sequence number in
+// word 4.
+struct BatchAnswer {
+    unsigned long long* host;
+    unsigned long long seq;
+};
 template <int W, typename T>
 hipError_t launch_join_batch(hipStream_t st, const JoinArgs<W, T>* items, const uint32_t* pair_start,
-                             uint32_t num_items, uint32_t total_pairs, uint32_t scap_max, uint32_t tcap_bits_max,
-                             unsigned long long* out);
+                             const BatchAnswer* answers, uint32_t num_items, uint32_t total_pairs, uint32_t scap_max,
+                             uint32_t tcap_bits_max);
 template <int W, typename T>
 hipError_t launch_rescale(hipStream_t st, const RescaleArgs<W, T>& a, uint32_t num_buckets);
 template <int W, typename T>

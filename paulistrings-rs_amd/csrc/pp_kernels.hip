@@ -1487,7 +1487,7 @@ __global__ void __launch_bounds__(kBlock) k_offsets_batch(const JoinArgs<W, T>* 
 
 template <int W, typename T>
 __global__ void __launch_bounds__(kBlock) k_reduce_batch(const JoinArgs<W, T>* __restrict__ items,
-                                                        unsigned long long* __restrict__ out) {
+                                                        const BatchAnswer* __restrict__ answers) {
     __shared__ uint64_t wave_sums[kWaves];
     __shared__ uint32_t wave_max[kWaves];
     const JoinArgs<W, T>& a = items[blockIdx.x];
@@ -1517,9 +1517,13 @@ __global__ void __launch_bounds__(kBlock) k_reduce_batch(const JoinArgs<W, T>* _
         }
         a.stats[0] = ts;
         a.stats[1] = tm;
-        out[4 * blockIdx.x + 0] = ts;
-        out[4 * blockIdx.x + 1] = tm;
-        out[4 * blockIdx.x + 2] = a.stats[2];
+        const BatchAnswer to = answers[blockIdx.x];
+        volatile unsigned long long* h = to.host;  // fine-grained host memory: the stores bypass the L2
+        h[0] = ts;
+        h[1] = tm;
+        h[2] = a.stats[2];
+        __builtin_amdgcn_s_waitcnt(0);  // the slot's words land before its sequence number
+        h[4] = to.seq;
     }
 }
 
@@ -1979,8 +1983,8 @@ hipError_t launch_rotation_inplace(hipStream_t st, const InplaceArgs<W, T>& a) {
 
 template <int W, typename T>
 hipError_t launch_join_batch(hipStream_t st, const JoinArgs<W, T>* items, const uint32_t* pair_start,
-                             uint32_t num_items, uint32_t total_pairs, uint32_t scap_max, uint32_t tcap_bits_max,
-                             unsigned long long* out) {
+                             const BatchAnswer* answers, uint32_t num_items, uint32_t total_pairs, uint32_t scap_max,
+                             uint32_t tcap_bits_max) {
     if (num_items == 0) return hipSuccess;
     hipLaunchKernelGGL((k_offsets_batch<W, T>), dim3(num_items), dim3(kBlock), 0, st, items);
     if (total_pairs) {
@@ -1988,7 +1992,7 @@ hipError_t launch_join_batch(hipStream_t st, const JoinArgs<W, T>* items, const 
         hipLaunchKernelGGL((k_rotation_join_batch<W, T, 256>), dim3(total_pairs), dim3(256), lds, st, items,
                            pair_start, num_items);
     }
-    hipLaunchKernelGGL((k_reduce_batch<W, T>), dim3(num_items), dim3(kBlock), 0, st, items, out);
+    hipLaunchKernelGGL((k_reduce_batch<W, T>), dim3(num_items), dim3(kBlock), 0, st, items, answers);
     return hipGetLastError();
 }
 
@@ -2098,8 +2102,8 @@ hipError_t launch_check_layout(hipStream_t st, const CheckArgs<W, T>& a) {
     template size_t join_lds_bytes<W, T>(uint32_t, uint32_t);                                          \
     template hipError_t launch_rotation_join<W, T>(hipStream_t, const JoinArgs<W, T>&, uint32_t, uint32_t); \
     template hipError_t launch_rotation_join_small<W, T>(hipStream_t, const SmallJoinArgs<W, T>&);      \
-    template hipError_t launch_join_batch<W, T>(hipStream_t, const JoinArgs<W, T>*, const uint32_t*, uint32_t,     \
-                                                uint32_t, uint32_t, uint32_t, unsigned long long*);             \
+    template hipError_t launch_join_batch<W, T>(hipStream_t, const JoinArgs<W, T>*, const uint32_t*,               \
+                                                const BatchAnswer*, uint32_t, uint32_t, uint32_t, uint32_t);    \
     template hipError_t launch_rescale<W, T>(hipStream_t, const RescaleArgs<W, T>&, uint32_t);          \
     template size_t inplace_lds_bytes<W, T>(uint32_t, uint32_t);                                        \
     template hipError_t launch_rotation_inplace<W, T>(hipStream_t, const InplaceArgs<W, T>&);           \

@@ -164,6 +164,33 @@ struct WindowArgs {
 template <int W, typename T>
 hipError_t launch_topn_window(hipStream_t st, const WindowArgs<W, T>& a);
 
+// A whole selection per item in one launch, a workgroup each (from kWholeTerms on the radix passes, with workgroups over
+// all of the chip, read a sum faster than one CU does): sums of at most kWholeTerms terms in at most kWholeBuckets
+// buckets whose positions fit 32 bits (every length fits 16).  The answer is a window's (kWindowMissed: more equal keys
+// at the boundary than the list or the order holds).
+constexpr uint32_t kWholeBuckets = 2048;
+constexpr uint64_t kWholeTerms = 1ull << 17;
+template <int W, typename T>
+struct WholeArgs {
+    const uint64_t* x;
+    const uint64_t* z;
+    const T* c;
+    uint64_t cap;
+    const uint64_t* start;
+    const uint32_t* len;
+    const uint64_t* rows;
+    uint32_t num_buckets;
+    int32_t ref_bits;
+    uint64_t n;
+    uint64_t seed;  // the last boundary, or 0
+    uint8_t* flags;
+    TopnState* state;
+    unsigned long long* host;
+    unsigned long long seq;
+};
+template <int W, typename T>
+hipError_t launch_topn_whole(hipStream_t st, const WholeArgs<W, T>* items, uint32_t num_items);
+
 template <int W, typename T>
 struct TopnRetainArgs {
     uint64_t* x;

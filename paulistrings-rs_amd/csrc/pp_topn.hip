@@ -661,20 +661,102 @@ __global__ void __launch_bounds__(kBlock) k_window_narrow(const WindowArgs<W, T>
     }
 }
 
+// The k-th largest of the n listed keys (su, with their positions sp), by a workgroup of kFinishBlock threads: the
+// boundary, how many of the keys equal to it stay, and how many there are.  Only some staying, they are put into
+// canonical order and flagged; false when they are more than the order holds.  Both counts take every thread the list
+// leaves: a run of lanes per key, each over a part of the list.
+constexpr uint32_t kFinishBlock = 1024;
+template <int W>
+struct RankScratch {
+    uint64_t x[W][kWindowTies], z[W][kWindowTies], pos[kWindowTies];
+    uint32_t bucket[kWindowTies];
+    uint32_t ties;
+    uint64_t found[3];  // the boundary key, the list's keys above it, the keys equal to it
+};
+__device__ __forceinline__ uint32_t lanes_per_key(uint32_t n) {
+    uint32_t g = 1;
+    while (2 * g * n <= kFinishBlock && g < 64) g *= 2;
+    return g;
+}
+template <int W, typename Args>
+__device__ __forceinline__ bool rank_ties(const Args& a, RankScratch<W>& r, const uint64_t* su, const uint64_t* sp,
+                                          uint32_t n, uint64_t boundary, uint32_t equal, uint64_t stay) {
+    if (equal > kWindowTies) return false;
+    const uint32_t tid = threadIdx.x;
+    for (uint32_t i = tid; i < n; i += kFinishBlock) {
+        if (su[i] != boundary) continue;
+        const uint32_t e = atomicAdd(&r.ties, 1u);
+        const Key<W> kk = load_key<W>(a.x, a.z, a.cap, sp[i]);
+#pragma unroll
+        for (int v = 0; v < W; ++v) {
+            r.x[v][e] = kk.x[v];
+            r.z[v][e] = kk.z[v];
+        }
+        r.bucket[e] = bucket_of<W>(kk, a.rows, a.ref_bits);
+        r.pos[e] = sp[i];
+    }
+    __syncthreads();
+    const uint32_t g = lanes_per_key(equal), i = tid / g;
+    uint32_t before = 0;
+    if (i < equal)
+        for (uint32_t q = tid % g; q < equal; q += g) {
+            int order = r.bucket[q] < r.bucket[i] ? -1 : r.bucket[q] > r.bucket[i] ? 1 : 0;
+#pragma unroll
+            for (int v = 0; v < W; ++v)
+                if (order == 0) order = r.x[v][q] < r.x[v][i] ? -1 : r.x[v][q] > r.x[v][i] ? 1 : 0;
+#pragma unroll
+            for (int v = 0; v < W; ++v)
+                if (order == 0) order = r.z[v][q] < r.z[v][i] ? -1 : r.z[v][q] > r.z[v][i] ? 1 : 0;
+            before += order < 0;
+        }
+    for (uint32_t d = 1; d < g; d *= 2) before += (uint32_t)__shfl_xor((int)before, (int)d, 64);
+    if (i < equal && tid % g == 0) a.flags[r.pos[i]] = before < stay ? 1 : 0;
+    return true;
+}
+template <int W, typename T, typename Args>
+__device__ __forceinline__ bool rank_boundary(const Args& a, RankScratch<W>& r, const uint64_t* su, const uint64_t* sp,
+                                              uint32_t n, uint64_t k, uint64_t& boundary, uint64_t& stay,
+                                              uint32_t& equal) {
+    const uint32_t tid = threadIdx.x;
+    if (tid == 0) r.ties = 0u;
+    const uint32_t g = lanes_per_key(n);
+    for (uint32_t i0 = 0; i0 < n; i0 += kFinishBlock / g) {  // uniform
+        const uint32_t i = i0 + tid / g;
+        const uint64_t u = i < n ? su[i] : 0;
+        uint32_t greater = 0, same = 0;
+        if (i < n)
+            for (uint32_t q = tid % g; q < n; q += g) {
+                greater += su[q] > u;
+                same += su[q] == u;
+            }
+        for (uint32_t d = 1; d < g; d *= 2) {
+            greater += (uint32_t)__shfl_xor((int)greater, (int)d, 64);
+            same += (uint32_t)__shfl_xor((int)same, (int)d, 64);
+        }
+        if (i < n && greater < k && greater + same >= k) {  // every row equal to the boundary writes the same
+            r.found[0] = u;
+            r.found[1] = greater;
+            r.found[2] = same;
+        }
+    }
+    __syncthreads();
+    boundary = r.found[0];
+    stay = k - r.found[1];
+    equal = (uint32_t)r.found[2];
+    return stay == equal || rank_ties<W>(a, r, su, sp, n, boundary, equal, stay);
+}
+
 // The n-th key among the collected (or narrowed) ones, by one workgroup: 11-bit digits of the window until at most
 // kWindowRank keys are left or they are equal, those ranked by counting, and the keys equal to the boundary put into canonical order when
 // only some of them stay.  Then the state the next layer reads, the answer to the host, and the counts cleared.
-constexpr uint32_t kFinishBlock = 1024;
 template <int W, typename T>
 __global__ void __launch_bounds__(kFinishBlock) k_window_finish(const WindowArgs<W, T> a) {
     constexpr uint32_t kDigits = 2048;
     __shared__ uint32_t hist[kDigits];
     __shared__ uint64_t part[kFinishBlock / 64 + 3];
     __shared__ uint64_t su[kWindowList], sp[kWindowList];
-    __shared__ uint64_t tx[W][kWindowTies], tz[W][kWindowTies], tp[kWindowTies];
-    __shared__ uint32_t tb[kWindowTies];
-    __shared__ uint32_t held, ties;
-    __shared__ uint64_t found[3];  // the boundary key, the list's keys above it, the keys equal to it
+    __shared__ RankScratch<W> ranked;
+    __shared__ uint32_t held;
     __shared__ WindowTotals t;
     const uint32_t tid = threadIdx.x;
     WindowCounts& w = *a.counts;
@@ -717,10 +799,7 @@ __global__ void __launch_bounds__(kFinishBlock) k_window_finish(const WindowArgs
         }
         done = left <= kWindowList;  // else more equal keys than the list holds
         if (done) {
-            if (tid == 0) {
-                held = 0u;
-                ties = 0u;
-            }
+            if (tid == 0) held = 0u;
             __syncthreads();
             for (uint64_t i0 = tid; i0 < m; i0 += 4 * kFinishBlock) {
                 uint64_t u[4];
@@ -736,56 +815,7 @@ __global__ void __launch_bounds__(kFinishBlock) k_window_finish(const WindowArgs
                     }
             }
             __syncthreads();
-            const uint32_t n = held;  // = left
-            for (uint32_t i = tid; i < n; i += kFinishBlock) {
-                const uint64_t u = su[i];
-                uint32_t greater = 0, same = 0;
-                for (uint32_t q = 0; q < n; ++q) {
-                    greater += su[q] > u;
-                    same += su[q] == u;
-                }
-                if (greater < k && greater + same >= k) {  // every row equal to the boundary writes the same
-                    found[0] = u;
-                    found[1] = greater;
-                    found[2] = same;
-                }
-            }
-            __syncthreads();
-            boundary = found[0];
-            stay = k - found[1];
-            equal = (uint32_t)found[2];
-            if (stay < equal) {
-                done = equal <= kWindowTies;
-                if (done) {
-                    for (uint32_t i = tid; i < n; i += kFinishBlock) {
-                        if (su[i] != boundary) continue;
-                        const uint32_t e = atomicAdd(&ties, 1u);
-                        const Key<W> kk = load_key<W>(a.x, a.z, a.cap, sp[i]);
-#pragma unroll
-                        for (int v = 0; v < W; ++v) {
-                            tx[v][e] = kk.x[v];
-                            tz[v][e] = kk.z[v];
-                        }
-                        tb[e] = bucket_of<W>(kk, a.rows, a.ref_bits);
-                        tp[e] = sp[i];
-                    }
-                    __syncthreads();
-                    for (uint32_t i = tid; i < equal; i += kFinishBlock) {
-                        uint32_t before = 0;
-                        for (uint32_t q = 0; q < equal; ++q) {
-                            int order = tb[q] < tb[i] ? -1 : tb[q] > tb[i] ? 1 : 0;
-#pragma unroll
-                            for (int v = 0; v < W; ++v)
-                                if (order == 0) order = tx[v][q] < tx[v][i] ? -1 : tx[v][q] > tx[v][i] ? 1 : 0;
-#pragma unroll
-                            for (int v = 0; v < W; ++v)
-                                if (order == 0) order = tz[v][q] < tz[v][i] ? -1 : tz[v][q] > tz[v][i] ? 1 : 0;
-                            before += order < 0;
-                        }
-                        a.flags[tp[i]] = before < stay ? 1 : 0;
-                    }
-                }
-            }
+            done = rank_boundary<W, T>(a, ranked, su, sp, held, k, boundary, stay, equal);  // held = left
         }
     }
     const bool crowded = !done && !keep_all && a.narrow && t.fullest > a.room && t.inside(a.n);  // uniform
@@ -830,11 +860,173 @@ __global__ void __launch_bounds__(kFinishBlock) k_window_finish(const WindowArgs
     }
 }
 
+// A whole selection by one workgroup, for many sums of up to kWholeTerms terms at once: the n-th key by 11-bit digits
+// over every key of the sum, then as k_window_finish ranks.  It needs no boundary to start from.  Each wave reads four
+// buckets at a time, sixteen loads in flight per lane: the latency of the one CU's reads bounds it, and the counts of keys
+// that share a digit follow one another in the LDS.  64 sums keeping 2^15 of up to 2^16 terms: 37 us in one launch (48 with
+// the octaves as the first digit), where the start, three radix passes and their selects were 46 in seven, with a second
+// round trip for the boundary bins ordered on the host.  (The windowed selection batched the same way took 21, but with
+// angles drawn from the whole circle some sum's boundary left its window in 788 of 823 steps.)
+template <int W, typename T, typename F>
+__device__ __forceinline__ void whole_keys(const WholeArgs<W, T>& a, const uint32_t* first, const uint16_t* len, F f) {
+    constexpr uint32_t kWavesHere = kFinishBlock / 64;
+    for (uint32_t b0 = wave_id(); b0 < a.num_buckets; b0 += 4 * kWavesHere) {
+        uint32_t most = 0, from[4], n[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const uint32_t b = b0 + q * kWavesHere;
+            n[q] = b < a.num_buckets ? len[b] : 0u;
+            from[q] = n[q] ? first[b] : 0u;
+            most = max(most, n[q]);
+        }
+        for (uint32_t r0 = lane_id(); r0 - lane_id() < most; r0 += 256) {
+            T c[4][4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    if (r0 + 64 * v < n[q]) c[q][v] = a.c[from[q] + r0 + 64 * v];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    if (r0 + 64 * v < n[q]) {
+                        const uint64_t u = magnitude_bits<T>(c[q][v]);
+                        if (!is_nan_bits(u)) f(u, from[q] + r0 + 64 * v);
+                    }
+        }
+    }
+}
+
+template <int W, typename T>
+__global__ void __launch_bounds__(kFinishBlock) k_topn_whole(const WholeArgs<W, T>* __restrict__ items) {
+    constexpr uint32_t kDigits = 2048;
+    __shared__ uint32_t hist[kDigits];
+    __shared__ uint64_t part[kFinishBlock / 64 + 3];
+    __shared__ uint64_t su[kWindowList], sp[kWindowList];
+    __shared__ RankScratch<W> ranked;
+    __shared__ uint32_t first[kWholeBuckets];
+    __shared__ uint16_t len[kWholeBuckets];
+    __shared__ uint32_t held, finite_terms, above_terms;
+    const WholeArgs<W, T> a = items[blockIdx.x];
+    const uint32_t tid = threadIdx.x;
+    for (uint32_t b = tid; b < a.num_buckets; b += kFinishBlock) {
+        first[b] = (uint32_t)a.start[b];
+        len[b] = (uint16_t)a.len[b];
+    }
+    for (uint32_t i = tid; i < kDigits; i += kFinishBlock) hist[i] = 0u;
+    if (tid == 0) held = finite_terms = above_terms = 0u;
+    __syncthreads();
+    // The first digit: of eight octaves around the last boundary 256 parts each, which leaves a few keys to collect and
+    // spreads the counts over the LDS; with no boundary, or one outside them, the octaves alone.
+    const uint64_t low = a.seed ? max(a.seed >> 44, 1024ull) - 1024ull : 0ull;
+    int shift = a.seed ? 44 : 52;
+    uint32_t mine = 0, over = 0;
+    whole_keys<W, T>(a, first, len, [&](uint64_t u, uint32_t) {
+        ++mine;
+        const uint64_t r = (u >> shift) - low;
+        if (r < kDigits) atomicAdd(&hist[r], 1u);
+        else over += (u >> shift) > low;
+    });
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) {
+        mine += (uint32_t)__shfl_xor((int)mine, d, 64);
+        over += (uint32_t)__shfl_xor((int)over, d, 64);
+    }
+    if (lane_id() == 0) {
+        atomicAdd(&finite_terms, mine);
+        if (over) atomicAdd(&above_terms, over);
+    }
+    __syncthreads();
+    const uint32_t finite = finite_terms, above = above_terms;
+    const bool keep_all = finite <= a.n;  // uniform
+    bool done = keep_all;
+    uint64_t boundary = 0, stay = 0;
+    uint32_t equal = 0;
+    if (!keep_all) {
+        uint64_t k = a.n - above, base = 0, bin[3] = {0, 0, 0};
+        bool outside = above >= a.n;  // uniform, as below
+        if (!outside) {
+            if (tid == 0) part[kFinishBlock / 64 + 2] = 0;  // window_bin leaves the answer as it is when there is none
+            window_bin<kDigits, kFinishBlock>(hist, k, part, bin);
+            outside = bin[2] == 0;
+        }
+        if (outside) {
+            shift = 52;
+            k = a.n;
+            for (uint32_t i = tid; i < kDigits; i += kFinishBlock) hist[i] = 0u;
+            __syncthreads();
+            whole_keys<W, T>(a, first, len, [&](uint64_t u, uint32_t) { atomicAdd(&hist[u >> 52], 1u); });
+            __syncthreads();
+            window_bin<kDigits, kFinishBlock>(hist, k, part, bin);
+        }
+        base = (bin[0] + (outside ? 0 : low)) << shift;
+        k -= bin[1];
+        while (bin[2] > kWindowRank && shift > 0) {
+            const int sh = max(shift - 11, 0);
+            for (uint32_t i = tid; i < kDigits; i += kFinishBlock) hist[i] = 0u;
+            __syncthreads();
+            whole_keys<W, T>(a, first, len, [&](uint64_t u, uint32_t) {
+                const uint64_t r = u - base;  // a smaller key wraps far past the range
+                if ((r >> shift) == 0) atomicAdd(&hist[r >> sh], 1u);
+            });
+            __syncthreads();
+            window_bin<kDigits, kFinishBlock>(hist, k, part, bin);
+            base += bin[0] << sh;
+            k -= bin[1];
+            shift = sh;
+        }
+        done = bin[2] <= kWindowList;  // else more equal keys than the list holds
+        if (done) {
+            whole_keys<W, T>(a, first, len, [&](uint64_t u, uint32_t at) {
+                if (((u - base) >> shift) == 0) {
+                    const uint32_t slot = atomicAdd(&held, 1u);
+                    su[slot] = u;
+                    sp[slot] = at;
+                }
+            });
+            __syncthreads();
+            done = rank_boundary<W, T>(a, ranked, su, sp, held, k, boundary, stay, equal);
+        }
+    }
+    if (tid == 0) {
+        if (done) {
+            TopnState& s = *a.state;
+            s.prefix = boundary;
+            s.mask = ~0ull;
+            s.k = stay;
+            s.above = a.n - stay;
+            s.finite = finite;
+            s.ties = equal;
+            s.keep_all_finite = keep_all ? 1 : 0;
+        }
+        volatile unsigned long long* h = a.host;  // fine-grained host memory: the stores bypass the L2
+        h[0] = done ? kWindowDone : kWindowMissed;
+        h[1] = boundary;
+        h[3] = finite;
+        h[5] = done && stay < equal ? 1 : 0;
+        __builtin_amdgcn_s_waitcnt(0);  // the slot's words land before its sequence number
+        h[4] = a.seq;
+    }
+}
+
+template <int W, typename T>
+hipError_t launch_topn_whole(hipStream_t st, const WholeArgs<W, T>* items, uint32_t num_items) {
+    if (num_items == 0) return hipSuccess;
+    hipLaunchKernelGGL((k_topn_whole<W, T>), dim3(num_items), dim3(kFinishBlock), 0, st, items);
+    return hipGetLastError();
+}
+
+template <int W, typename T>
+bool window_args_valid(const WindowArgs<W, T>& a) {
+    return a.buckets_per_block != 0 && a.buckets_per_block <= kHistBucketsMax && a.hi > a.lo && a.n != 0 &&
+           a.hi - a.lo < (1ull << 62) && a.bin_shift >= 0 && a.bin_shift <= 63 &&
+           ((a.hi - a.lo - 1) >> a.bin_shift) < kWindowBins;
+}
+
 template <int W, typename T>
 hipError_t launch_topn_window(hipStream_t st, const WindowArgs<W, T>& a) {
-    if (a.buckets_per_block == 0 || a.buckets_per_block > kHistBucketsMax || a.hi <= a.lo || a.n == 0 ||
-        a.hi - a.lo >= (1ull << 62) || a.bin_shift < 0 || a.bin_shift > 63 || ((a.hi - a.lo - 1) >> a.bin_shift) >= kWindowBins)
-        return hipErrorInvalidValue;
+    if (!window_args_valid<W, T>(a)) return hipErrorInvalidValue;
     const uint32_t blocks = (a.num_buckets + a.buckets_per_block - 1) / a.buckets_per_block;
     hipLaunchKernelGGL((k_window_scan<W, T>), dim3(blocks), dim3(kBlock), 0, st, a);
     if (a.narrow) hipLaunchKernelGGL((k_window_narrow<W, T>), dim3(256), dim3(kBlock), 0, st, a);
@@ -1320,6 +1512,7 @@ template hipError_t launch_octave_hist<float>(hipStream_t, const OctaveHistArgs<
 #define PP_TOPN_INSTANTIATE(W, T)                                                                       \
     template hipError_t launch_octave_select<W, T>(hipStream_t, const OctaveSelectArgs<W, T>&);         \
     template hipError_t launch_topn_window<W, T>(hipStream_t, const WindowArgs<W, T>&);                 \
+    template hipError_t launch_topn_whole<W, T>(hipStream_t, const WholeArgs<W, T>*, uint32_t);         \
     template hipError_t launch_topn_gather_ties<W, T>(hipStream_t, const TopnTieArgs<W, T>&, uint32_t); \
     template hipError_t launch_topn_gather_batch<W, T>(hipStream_t, const TopnTieArgs<W, T>*, const uint32_t*, \
                                                        uint32_t, uint32_t);                               \

@@ -139,3 +139,44 @@ def test_batched_topn_selections_equal_one_by_one(monkeypatch):
     check_batch(inst, pol_o, pol_p)
     monkeypatch.setenv("PP_BATCH_TOPN", "0")
     check_batch(inst, pol_o, pol_p)
+
+
+@pytest.mark.parametrize("num_qubits", [50, 100])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_batched_whole_selections_equal_the_radix_passes(monkeypatch, num_qubits, dtype):
+    """Selections of sums of very different sizes, a workgroup each in one launch: caps of one
+    term, at the length, and in runs of equal magnitudes longer than a workgroup orders (which the radix
+    passes take over), on circuits of different lengths, against the radix passes alone."""
+    announce(f"batched whole selections, {num_qubits} qubits {np.dtype(dtype).name}")
+    rng = np.random.default_rng(num_qubits)
+    W = circuits.width_for(num_qubits)
+    inst, pols = [], []
+    for k, (n, cap) in enumerate([(1, 1), (3, 2), (300, 1), (300, 299), (5_000, 2_000), (60_000, 30_000), (60_000, 50_000),
+                                  (20_000, 9_000), (600_000, 400_000)]):
+        x = np.unique(rng.integers(0, 1 << 50, size=(n, W), dtype=np.uint64), axis=0)
+        z = rng.integers(0, 1 << 36, size=x.shape, dtype=np.uint64) if W == 1 else np.zeros_like(x)
+        if W == 2:
+            x[:, 1] &= np.uint64((1 << 36) - 1)
+        c = rng.standard_normal(len(x))
+        if k == 7:
+            c = np.round(c, 1) + 0.05
+        circ = Circuit(num_qubits)
+        for _ in range(8 + k):
+            q = int(rng.integers(0, num_qubits - 1))
+            circ.rzz(float(rng.uniform(0.1, 0.6)), q, q + 1).rx(float(rng.uniform(0.1, 0.6)), int(rng.integers(num_qubits)))
+        inst.append((x, z, c.astype(dtype), circ))
+        pols.append(truncation.coeff(1e-4) & truncation.topn(cap))
+
+    def run(window):
+        monkeypatch.setenv("PP_TOPN_WINDOW", window)
+        sums = [PauliSum(num_qubits, x, z, c, dtype=dtype).to_device(0) for x, z, c, _ in inst]
+        propagate_batch(sums, [i[3] for i in inst], pols, ["heisenberg"] * len(inst))
+        out = []
+        for s in sums:
+            h = s.to_host()
+            out.append((h.x_array(), h.z_array(), h.coefficients_array()))
+            s.free()
+        return out
+
+    for got, want in zip(run("1"), run("0")):
+        assert all(np.array_equal(a, b) for a, b in zip(got, want))
