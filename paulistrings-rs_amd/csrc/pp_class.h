@@ -28,14 +28,21 @@ constexpr uint32_t kClassBlock = 256;
 
 // Counter slots of a class pass.
 enum ClassStat : uint32_t {
-    kClassOutRows = 0,    // rows the apply emitted (its cursor into the output staging; may pass its capacity)
-    kClassFlags = 1,      // bit 0: a class bucket larger than the LDS set; bit 1: a layer outgrew it; bit 2: staging full
-    kClassUntouched = 2,  // untouched rows that `keep` passes
-    kClassStaged = 3,     // touched rows (the class-bucket scan's total)
-    kClassLayerRows = 4,  // [4 + l]: class rows after layer l
-    kClassLongest = 4 + kClassMaxLayers,  // the output layout's longest bucket
-    kClassStatSlots = 5 + kClassMaxLayers
+    kClassFlags = 0,      // bit 0: a class bucket larger than the LDS set; bit 1: a layer outgrew it; bit 2: staging full
+    kClassStaged = 1,     // touched rows (the class-bucket scan's total)
+    kClassLayerRows = 2,  // [2 + l]: class rows after layer l
+    kClassLongest = 2 + kClassMaxLayers,  // the output layout's longest bucket
+    kClassStats = 3 + kClassMaxLayers,
+    // Counters that many workgroups add to, on a 128-byte line each (same-line atomics follow one another every ~12 ns,
+    // whatever word they hit).  Part p of kClassParts, at kClassPart + kClassLine p: [0] the rows emitted into the output
+    // staging's part p (its cursor; may pass the part's room), [1] untouched rows that `keep` passes.
+    kClassLine = 16,
+    kClassPart = kClassLine,
+    kClassParts = 32,
+    kClassStatSlots = kClassPart + kClassLine * kClassParts
 };
+static_assert(kClassStats <= kClassPart, "the counters overlap the parts");
+constexpr uint32_t kClassCountStride = 32;  // words between two buckets' output counters: a line each
 
 // One layer: a local table (LocalPtm, channel/prepared.rs:79-86) on the support slots word/bit (pattern_of).
 struct ClassLayer {
@@ -81,12 +88,14 @@ struct ClassArgs {
     uint64_t* oz;
     T* oc;
     uint32_t* obucket;
-    uint64_t ocap;
-    uint32_t* ocount;  // [num_buckets] outputs per output bucket
+    uint64_t ocap;       // kClassParts parts of part_rows rows
+    uint64_t part_rows;
+    uint32_t* ocount;    // [num_buckets * kClassCountStride] outputs per output bucket
     unsigned long long* stats;  // ClassStat slots
-    uint32_t lcap;              // rows of one LDS set
+    uint32_t lcap;              // rows of the LDS set a layer writes
+    uint32_t icap;              // rows of the set the staging is loaded into: lcap, or fewer for a single layer
     uint32_t chunk_rows;        // staged rows one apply iteration aims for (whole class buckets)
-    uint32_t tbits;             // LDS table slots: 1 << tbits >= 2 lcap
+    uint32_t tbits;             // LDS table slots: 1 << tbits >= 2 icap
     // the output layout (the spare columns)
     uint64_t* px;
     uint64_t* pz;
@@ -97,7 +106,7 @@ struct ClassArgs {
 };
 
 template <int W, typename T>
-size_t class_lds_bytes(uint32_t lcap, uint32_t tbits, uint32_t prog_words);
+size_t class_lds_bytes(uint32_t lcap, uint32_t icap, uint32_t tbits, uint32_t prog_words);
 
 // Each launcher queues its kernel on st.
 template <int W, typename T>
@@ -109,6 +118,7 @@ hipError_t launch_class_apply(hipStream_t st, const ClassArgs<W, T>& a);  // the
 template <int W, typename T>
 hipError_t launch_class_lens(hipStream_t st, const ClassArgs<W, T>& a);  // plen = ukeep + ocount, the longest
 template <int W, typename T>
-hipError_t launch_class_place(hipStream_t st, const ClassArgs<W, T>& a, uint64_t out_rows);  // the output layout
+hipError_t launch_class_place(hipStream_t st, const ClassArgs<W, T>& a, uint64_t part_most);  // the output layout; no
+                                                                                    // part holds more than part_most
 
 }  // namespace pp

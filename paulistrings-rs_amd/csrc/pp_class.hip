@@ -5,11 +5,13 @@
 // coefficients) that trade places every layer; per layer an open-addressing table of the live set's classes under
 // that layer (the key with the layer's support cleared) and one record per class: the row of each of its (at most
 // 16) patterns.  A layer gathers every output from its sources: an output K with pattern t has, for each entry e,
-// the source of pattern t ^ delta[e] in its class, with amplitude amp[e][t ^ delta[e]]; the source that comes first
-// in entry order among those present owns K, sums its contributions in entry order (one rounded multiply and one
-// rounded add each, as a rotation's pair update or the host engine's merge), asks keep and appends it to the other
-// set.  A rotation table (identity entry first, then the generator) gives own = c cos + c_partner a1 exactly as the
-// pair join does.
+// the source of pattern t ^ delta[e] in its class, with amplitude amp[e][t ^ delta[e]].  It sums the contributions of
+// the sources present in entry order (one rounded multiply and one rounded add each, as a rotation's pair update or the
+// host engine's merge), asks keep and appends it to the other set.  A rotation table (identity entry first, then the
+// generator) gives own = c cos + c_partner a1 exactly as the pair join does.  A table of few entries gives a row's
+// outputs to one thread (the source that comes first in entry order owns an output); from kClassWideEntries on every
+// pattern of a class has a thread of its own: a general two-qubit table turns the 16 to 32 rows of a workgroup's classes
+// into up to 500 outputs of 16 sources, which would leave seven of its eight waves idle.
 
 #include "pp_class.h"
 
@@ -74,7 +76,7 @@ __global__ void __launch_bounds__(kClassBlock) k_class_route(const ClassArgs<W, 
         for (int d = 32; d > 0; d >>= 1) kept += (uint32_t)__shfl_xor((int)kept, d, 64);
         if (lane == 0) {
             a.ukeep[b] = kept;
-            if (kept) atomicAdd(&a.stats[kClassUntouched], (unsigned long long)kept);
+            if (kept) atomicAdd(&a.stats[kClassPart + kClassLine * (b % kClassParts) + 1], (unsigned long long)kept);
         }
     }
 }
@@ -82,24 +84,29 @@ __global__ void __launch_bounds__(kClassBlock) k_class_route(const ClassArgs<W, 
 // A persistent grid over the class buckets; each workgroup runs the whole program on one class bucket at a time.
 // The program's tables are copied to LDS once per workgroup.  Per layer three barriers: the table cleared; the live
 // set inserted; the outputs written.  The output counters alternate between two slots, so the next layer resets its
-// slot while the last readers of this one are still behind the third barrier.
+// slot while the last readers of this one are still behind the third barrier.  What bounds it is latency: the search,
+// the rows, the cursor and the bucket counters of a chunk follow one another.  250 007 terms through two-qubit unitaries
+// (a third of them touched, 16 outputs a class) and amplitude damping: 99 us a pass and 15 passes for 12 tables, 365 and 21
+// with one thread per row, 32 counters a line, a search of 17 dependent reads and chunks that outgrew the set.
+constexpr uint32_t kClassWideEntries = 4;
 template <int W, typename T>
 __global__ void __launch_bounds__(kClassBlock) k_class_apply(const ClassArgs<W, T> a) {
     extern __shared__ __align__(16) unsigned char class_lds[];
-    const uint32_t cap = a.lcap;
+    // set 0 holds icap rows, set 1 lcap (more than one layer: icap = lcap)
+    const uint32_t icap = a.icap;
     double* const P = reinterpret_cast<double*>(class_lds);  // every layer's amplitudes, entry-major
     uint64_t* const X0 = reinterpret_cast<uint64_t*>(P + a.prog_words);
-    uint64_t* const Z0 = X0 + (size_t)W * cap;
-    uint64_t* const X1 = Z0 + (size_t)W * cap;
-    uint64_t* const Z1 = X1 + (size_t)W * cap;
-    T* const C0 = reinterpret_cast<T*>(Z1 + (size_t)W * cap);
-    T* const C1 = C0 + cap;
-    uint32_t* const table = reinterpret_cast<uint32_t*>(C1 + cap);
+    uint64_t* const Z0 = X0 + (size_t)W * icap;
+    uint64_t* const X1 = Z0 + (size_t)W * icap;
+    uint64_t* const Z1 = X1 + (size_t)W * a.lcap;
+    T* const C0 = reinterpret_cast<T*>(Z1 + (size_t)W * a.lcap);
+    T* const C1 = C0 + icap;
+    uint32_t* const table = reinterpret_cast<uint32_t*>(C1 + a.lcap);
     // per layer, one record per class of the live set (the key with the layer's support cleared): a row holding it
     // and the row of each of its patterns (kNoRow where the class has none)
     uint32_t* const rec_rep = table + (1u << a.tbits);
-    uint16_t* const rec_mem = reinterpret_cast<uint16_t*>(rec_rep + cap);  // [cap][16]
-    uint16_t* const row_rec = rec_mem + (size_t)cap * 16;                  // [cap]
+    uint16_t* const rec_mem = reinterpret_cast<uint16_t*>(rec_rep + icap);  // [icap][16]
+    uint16_t* const row_rec = rec_mem + (size_t)icap * 16;                  // [icap]
     __shared__ uint32_t s_word[kClassMaxLayers][2];
     __shared__ uint32_t s_bit[kClassMaxLayers][2];
     __shared__ uint32_t s_mask[kClassMaxLayers];
@@ -109,12 +116,14 @@ __global__ void __launch_bounds__(kClassBlock) k_class_apply(const ClassArgs<W, 
     __shared__ uint32_t s_count[2];
     __shared__ uint32_t s_bad[2];
     __shared__ unsigned long long s_base;
+    __shared__ unsigned long long s_rows[kClassMaxLayers];  // thread 0's: the rows after each layer, all chunks
     const uint32_t tid = threadIdx.x;
     const uint32_t nl = a.n_layers;
 
     if (tid == 0) {
         uint32_t off = 0;
         for (uint32_t l = 0; l < nl; ++l) {
+            s_rows[l] = 0;
             s_off[l] = off;
             off += a.layers[l].n_entries * 16u;
         }
@@ -141,15 +150,17 @@ __global__ void __launch_bounds__(kClassBlock) k_class_apply(const ClassArgs<W, 
     const uint64_t chunks = (staged + R - 1) / R;
     __shared__ unsigned long long s_range[2];
     for (uint64_t q = blockIdx.x; q < chunks; q += gridDim.x) {
-        if (tid < 2) {  // the first class bucket starting at or after q R (or (q + 1) R), as a row of the staging
-            const uint64_t at = (q + tid) * R;
+        if (wave_id() < 2) {  // the first class bucket starting at or after q R (or (q + 1) R), as a row of the staging
+            const uint64_t at = (q + wave_id()) * R;
             uint32_t lo = 0, hi = a.num_classes;
-            while (lo < hi) {
-                const uint32_t mid = (lo + hi) >> 1;
-                if (a.cstart[mid] < at) lo = mid + 1;
-                else hi = mid;
+            while (lo < hi) {  // 64 probes a step; the first c of them lie before it
+                const uint32_t step = (hi - lo + 63u) / 64u, p = lo + lane_id() * step;
+                const uint32_t c = (uint32_t)__popcll(__ballot(p < hi && a.cstart[p] < at));
+                const uint32_t next = min(hi, lo + c * step);
+                if (c) lo += (c - 1u) * step + 1u;
+                hi = next;
             }
-            s_range[tid] = lo < a.num_classes ? a.cstart[lo] : staged;
+            if (lane_id() == 0) s_range[wave_id()] = lo < a.num_classes ? a.cstart[lo] : staged;
         }
         __syncthreads();
         const uint64_t base = s_range[0];
@@ -157,12 +168,12 @@ __global__ void __launch_bounds__(kClassBlock) k_class_apply(const ClassArgs<W, 
         __syncthreads();  // read before the next chunk's search writes them
         const uint32_t n0 = (uint32_t)(end - base);
         if (n0 == 0u) continue;  // uniform
-        if (n0 > cap) {
+        if (n0 > icap) {
             if (tid == 0) atomicOr(&a.stats[kClassFlags], 1ull);
             continue;
         }
         for (uint32_t i = tid; i < n0; i += kClassBlock) {
-            store_key<W>(X0, Z0, cap, i, load_key<W>(a.sx, a.sz, a.scap, base + i));
+            store_key<W>(X0, Z0, icap, i, load_key<W>(a.sx, a.sz, a.scap, base + i));
             C0[i] = a.sc[base + i];
         }
         uint32_t n = n0;
@@ -172,6 +183,7 @@ __global__ void __launch_bounds__(kClassBlock) k_class_apply(const ClassArgs<W, 
             const uint64_t* IX = in0 ? X0 : X1;
             const uint64_t* IZ = in0 ? Z0 : Z1;
             const T* IC = in0 ? C0 : C1;
+            const uint32_t cap = in0 ? icap : a.lcap, out_cap = in0 ? a.lcap : icap;
             uint64_t* OX = in0 ? X1 : X0;
             uint64_t* OZ = in0 ? Z1 : Z0;
             T* OC = in0 ? C1 : C0;
@@ -228,7 +240,38 @@ __global__ void __launch_bounds__(kClassBlock) k_class_apply(const ClassArgs<W, 
                 row_rec[i] = (uint16_t)r;
             }
             __syncthreads();
-            for (uint32_t i = tid; i < n; i += kClassBlock) {
+            auto append = [&](const Key<W>& K, T w) {
+                const uint32_t j = atomicAdd(&s_count[slot], 1u);
+                if (j < out_cap) {
+                    store_key<W>(OX, OZ, out_cap, j, K);
+                    OC[j] = w;
+                } else {
+                    s_bad[slot] = 1u;
+                }
+            };
+            const bool wide = ne >= kClassWideEntries;  // uniform
+            const uint32_t dim = s_mask[l] + 1u;        // patterns: 16, 4 or 1
+            for (uint32_t it = tid; wide && it < n * dim; it += kClassBlock) {
+                const uint32_t i = it / dim, t = it % dim;
+                if (row_rec[i] != i) continue;  // the row that holds its class's record
+                const Key<W> k = load_key<W>(IX, IZ, cap, i);
+                const uint16_t* const mem = rec_mem + (size_t)i * 16;
+                T w = T(0);
+                bool any = false;
+                for (uint32_t f = 0; f < ne; ++f) {
+                    const uint32_t src = t ^ D[f];
+                    const double af = A[f * 16u + src];
+                    const uint32_t j = mem[src];
+                    if (af == 0.0 || j == 0xFFFFu) continue;
+                    const T v = IC[j] * (T)af;
+                    w = any ? w + v : v;
+                    any = true;
+                }
+                Key<W> K = k;
+                xor_local_delta<W>(K, t ^ pattern_of<W>(k, s_word[l], s_bit[l], s_mask[l]), s_word[l], s_bit[l]);
+                if (any && survives<W, T>(a.keep, K, w)) append(K, w);
+            }
+            for (uint32_t i = tid; !wide && i < n; i += kClassBlock) {
                 const Key<W> k = load_key<W>(IX, IZ, cap, i);
                 const T c = IC[i];
                 const uint32_t s = pattern_of<W>(k, s_word[l], s_bit[l], s_mask[l]);
@@ -269,14 +312,7 @@ __global__ void __launch_bounds__(kClassBlock) k_class_apply(const ClassArgs<W, 
                         w = any ? w + v : v;
                         any = true;
                     }
-                    if (!owner || !survives<W, T>(a.keep, K, w)) continue;
-                    const uint32_t j = atomicAdd(&s_count[slot], 1u);
-                    if (j < cap) {
-                        store_key<W>(OX, OZ, cap, j, K);
-                        OC[j] = w;
-                    } else {
-                        s_bad[slot] = 1u;
-                    }
+                    if (owner && survives<W, T>(a.keep, K, w)) append(K, w);
                 }
             }
             __syncthreads();
@@ -284,7 +320,7 @@ __global__ void __launch_bounds__(kClassBlock) k_class_apply(const ClassArgs<W, 
             bad = s_bad[slot] != 0u;
             if (bad) break;  // uniform
             in0 = !in0;
-            if (tid == 0) atomicAdd(&a.stats[kClassLayerRows + l], (unsigned long long)n);
+            if (tid == 0) s_rows[l] += n;
         }
         if (bad) {
             if (tid == 0) atomicOr(&a.stats[kClassFlags], 2ull);
@@ -294,23 +330,25 @@ __global__ void __launch_bounds__(kClassBlock) k_class_apply(const ClassArgs<W, 
         const uint64_t* FX = in0 ? X0 : X1;
         const uint64_t* FZ = in0 ? Z0 : Z1;
         const T* FC = in0 ? C0 : C1;
-        if (tid == 0) s_base = atomicAdd(&a.stats[kClassOutRows], (unsigned long long)n);
+        const uint32_t part = blockIdx.x % kClassParts;
+        if (tid == 0) s_base = atomicAdd(&a.stats[kClassPart + kClassLine * part], (unsigned long long)n);
         __syncthreads();
-        const uint64_t o0 = s_base;
-        if (o0 + n <= a.ocap) {
+        const uint64_t o0 = part * a.part_rows + s_base;
+        if (s_base + n <= a.part_rows) {
             for (uint32_t i = tid; i < n; i += kClassBlock) {
-                const Key<W> K = load_key<W>(FX, FZ, cap, i);
+                const Key<W> K = load_key<W>(FX, FZ, in0 ? icap : a.lcap, i);
                 const uint32_t ob = bucket_of<W>(K, a.rows, a.bits);
                 store_key<W>(a.ox, a.oz, a.ocap, o0 + i, K);
                 a.oc[o0 + i] = FC[i];
                 a.obucket[o0 + i] = ob;
-                atomicAdd(&a.ocount[ob], 1u);
+                atomicAdd(&a.ocount[ob * kClassCountStride], 1u);
             }
         } else if (tid == 0) {
             atomicOr(&a.stats[kClassFlags], 4ull);
         }
         __syncthreads();  // the sets are read before the next class bucket loads over them
     }
+    if (tid < nl && s_rows[tid]) atomicAdd(&a.stats[kClassLayerRows + tid], s_rows[tid]);
 }
 
 __global__ void __launch_bounds__(256) k_class_lens(const uint32_t* __restrict__ ukeep, const uint32_t* __restrict__ ocount,
@@ -319,7 +357,7 @@ __global__ void __launch_bounds__(256) k_class_lens(const uint32_t* __restrict__
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     uint32_t v = 0;
     if (i < n) {
-        v = ukeep[i] + ocount[i];
+        v = ukeep[i] + ocount[i * kClassCountStride];
         plen[i] = v;
     }
 #pragma unroll
@@ -329,15 +367,19 @@ __global__ void __launch_bounds__(256) k_class_lens(const uint32_t* __restrict__
 
 // The output layout in one launch: the first `place_blocks` workgroups put each bucket's untouched strings that keep
 // passes, in their order, at the front of its segment (a wave per bucket); the others put one class output each
-// behind its bucket's untouched strings (each bucket's count counts down to zero).
+// behind its bucket's untouched strings (each bucket's count counts down to zero).  The counters' atomics bounded it while
+// 32 buckets shared a line: 249 us for 1.3 million outputs, 66 with a line each.
 template <int W, typename T>
 __global__ void __launch_bounds__(kClassBlock) k_class_place(const ClassArgs<W, T> a, uint32_t place_blocks,
-                                                             uint64_t out_rows) {
+                                                             uint32_t part_blocks) {
     if (blockIdx.x >= place_blocks) {
-        const uint64_t i = (uint64_t)(blockIdx.x - place_blocks) * kClassBlock + threadIdx.x;
-        if (i >= out_rows) return;
+        const uint32_t g = blockIdx.x - place_blocks, part = g / part_blocks;
+        const uint64_t r = (uint64_t)(g % part_blocks) * kClassBlock + threadIdx.x;
+        if (r >= a.stats[kClassPart + kClassLine * part]) return;
+        const uint64_t i = part * a.part_rows + r;
         const uint32_t ob = a.obucket[i];
-        const uint64_t pos = a.pstart[ob] + a.ukeep[ob] + (uint64_t)(atomicSub(&a.ocount[ob], 1u) - 1u);
+        const uint32_t before = atomicSub(&a.ocount[ob * kClassCountStride], 1u) - 1u;
+        const uint64_t pos = a.pstart[ob] + a.ukeep[ob] + (uint64_t)before;
         store_key<W>(a.px, a.pz, a.pcap, pos, load_key<W>(a.ox, a.oz, a.ocap, i));
         a.pc[pos] = a.oc[i];
         return;
@@ -373,9 +415,9 @@ inline uint32_t wave_grid(uint32_t buckets) { return (buckets + kClassBlock / 64
 }  // namespace
 
 template <int W, typename T>
-size_t class_lds_bytes(uint32_t lcap, uint32_t tbits, uint32_t prog_words) {
-    return (size_t)prog_words * 8 + (size_t)2 * lcap * (2 * W * sizeof(uint64_t) + sizeof(T)) + ((size_t)4 << tbits) +
-           (size_t)lcap * (4 + 32 + 2);
+size_t class_lds_bytes(uint32_t lcap, uint32_t icap, uint32_t tbits, uint32_t prog_words) {
+    return (size_t)prog_words * 8 + ((size_t)lcap + icap) * (2 * W * sizeof(uint64_t) + sizeof(T)) +
+           ((size_t)4 << tbits) + (size_t)icap * (4 + 32 + 2);
 }
 
 template <int W, typename T>
@@ -398,13 +440,14 @@ template <int W, typename T>
 hipError_t launch_class_apply(hipStream_t st, const ClassArgs<W, T>& a) {
     if (a.num_classes == 0) return hipSuccess;
     if (!a.layers || !a.rows || !a.cstart || !a.sx || !a.ox || !a.obucket || !a.ocount || !a.stats ||
-        a.chunk_rows == 0)
+        a.chunk_rows == 0 || a.part_rows * kClassParts > a.ocap)
         return hipErrorInvalidValue;
-    if (a.tbits < 2 || a.tbits > 14 || ((size_t)1 << a.tbits) < 2 * (size_t)a.lcap || a.lcap > 0xFFFFu)
+    if (a.tbits < 2 || a.tbits > 14 || ((size_t)1 << a.tbits) < 2 * (size_t)a.icap || a.lcap > 0xFFFFu ||
+        a.icap > a.lcap || a.icap % 4 != 0 || a.lcap % 4 != 0 || (a.n_layers > 1 && a.icap != a.lcap))
         return hipErrorInvalidValue;
     if (a.prog_words > kClassMaxLayers * kClassMaxEntries * 16 || a.n_layers > kClassMaxLayers)
         return hipErrorInvalidValue;
-    const size_t lds = class_lds_bytes<W, T>(a.lcap, a.tbits, a.prog_words);
+    const size_t lds = class_lds_bytes<W, T>(a.lcap, a.icap, a.tbits, a.prog_words);
     static int cus = 0;
     if (cus == 0) {
         int dev = 0;
@@ -412,8 +455,8 @@ hipError_t launch_class_apply(hipStream_t st, const ClassArgs<W, T>& a) {
             hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
             cus = 256;
     }
-    static int resident[15][5] = {};  // by tbits (which fixes lcap) and the program's size in 4 KiB
-    int& per = resident[a.tbits][std::min<uint32_t>(a.prog_words / 512u, 4u)];
+    static int resident[15][2][5] = {};  // by tbits (which fixes icap), lcap and the program's size in 4 KiB
+    int& per = resident[a.tbits][a.lcap > 512 ? 1 : 0][std::min<uint32_t>(a.prog_words / 512u, 4u)];
     if (per == 0 &&
         (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_class_apply<W, T>, kClassBlock, lds) != hipSuccess ||
          per <= 0))
@@ -433,19 +476,21 @@ hipError_t launch_class_lens(hipStream_t st, const ClassArgs<W, T>& a) {
 }
 
 template <int W, typename T>
-hipError_t launch_class_place(hipStream_t st, const ClassArgs<W, T>& a, uint64_t out_rows) {
-    if (!a.ukeep || !a.ocount || !a.pstart || !a.px || (out_rows && !a.obucket)) return hipErrorInvalidValue;
+hipError_t launch_class_place(hipStream_t st, const ClassArgs<W, T>& a, uint64_t part_most) {
+    if (!a.ukeep || !a.ocount || !a.pstart || !a.px || !a.stats || (part_most && !a.obucket) || part_most > a.part_rows)
+        return hipErrorInvalidValue;
     const uint32_t place_blocks = wave_grid(a.num_buckets);
-    const uint64_t blocks = place_blocks + (out_rows + kClassBlock - 1) / kClassBlock;
+    const uint64_t part_blocks = (part_most + kClassBlock - 1) / kClassBlock;
+    const uint64_t blocks = place_blocks + part_blocks * kClassParts;
     if (blocks == 0) return hipSuccess;
     if (blocks > 0x7FFFFFFFull) return hipErrorInvalidValue;
     hipLaunchKernelGGL((k_class_place<W, T>), dim3((uint32_t)blocks), dim3(kClassBlock), 0, st, a, place_blocks,
-                       out_rows);
+                       (uint32_t)std::max<uint64_t>(part_blocks, 1));
     return hipGetLastError();
 }
 
 #define PP_CLASS_INSTANTIATE(W, T)                                                              \
-    template size_t class_lds_bytes<W, T>(uint32_t, uint32_t, uint32_t);                                  \
+    template size_t class_lds_bytes<W, T>(uint32_t, uint32_t, uint32_t, uint32_t);                              \
     template hipError_t launch_class_route<W, T>(hipStream_t, const ClassArgs<W, T>&);          \
     template hipError_t launch_class_gather<W, T>(hipStream_t, const ClassArgs<W, T>&);         \
     template hipError_t launch_class_apply<W, T>(hipStream_t, const ClassArgs<W, T>&);          \

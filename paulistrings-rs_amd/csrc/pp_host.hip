@@ -1772,34 +1772,55 @@ pp_status class_pass(pp_sum* s, const Prepared* layers, uint32_t n, const KeepPr
         return st;
     // class buckets of about 16 rows of the input, packed into chunks of a quarter of the LDS set; on an overflow
     // smaller chunks and finer class buckets, then a larger set
-    int cbits = 0;
-    while (cbits < 22 && ((uint64_t)16 << cbits) < len_in) ++cbits;
     uint64_t growth = 1;  // the program's worst fanout, capped: a chunk of lcap / growth rows fits its outputs
     for (uint32_t l = 0; l < n && growth < 16; ++l) growth *= std::max<uint32_t>(layers[l].fanout, 1u);
-    uint32_t lcap = 512, tbits = 10, chunk = (uint32_t)std::max<uint64_t>(16, 512 / std::min<uint64_t>(growth, 16));
-    uint64_t ocap = std::max<uint64_t>({2 * len_in, (uint64_t)4096, s->class_out_hint});
+    // a chunk runs up to one class bucket past its rows: where its outputs fill the set, smaller chunks of smaller buckets
+    // (at fanout 16, 32 rows of buckets of 16 outgrew the set in 9 of 12 tables, and the pass ran again)
+    const bool fills = growth >= 8;
+    int cbits = 0;
+    while (cbits < 22 && ((uint64_t)(fills ? 4 : 16) << cbits) < len_in) ++cbits;
+    // a single layer's input needs no room for its outputs: six workgroups share a CU in place of three (148 -> 99 us)
+    uint32_t lcap = 512, icap = n == 1 && fills ? 128 : 512, tbits = icap == 128 ? 8 : 10;
+    uint32_t chunk = (uint32_t)std::max<uint64_t>(16, (fills ? 256 : 512) / std::min<uint64_t>(growth, 16));
+    // the staging's parts hold a few chunks' outputs more than their share
+    const uint64_t ocap_least = 2 * len_in + kClassParts * 1024ull;
+    uint64_t ocap = std::max({ocap_least, s->class_out_hint, std::min<uint64_t>(growth, 16) / 4 * len_in});
     uint64_t *ox = nullptr, *oz = nullptr;
     void* oc = nullptr;
     uint32_t* ob = nullptr;
     unsigned long long* d_cst = nullptr;
     uint32_t* d_ocount = nullptr;
     int attempt = 0;
+    uint64_t untouched = 0, out_rows = 0, part_most = 0;  // counts of the pass; the fullest part of the staging
+    bool counted = false;                                 // ocap is a need, not an estimate
     for (;;) {
         const uint32_t C = 1u << cbits;
+        ocap = (ocap + kClassParts - 1) / kClassParts * kClassParts;
         // the counters, the outputs per bucket and the rows per class bucket: one block, one clear
         unsigned char* d_counts = nullptr;
         uint64_t* d_cstart = nullptr;
-        const size_t count_bytes = kClassStatSlots * 8 + (size_t)B * 4 + (size_t)C * 4;
+        const size_t ocount_bytes = (size_t)B * kClassCountStride * 4;
+        const size_t count_bytes = kClassStatSlots * 8 + ocount_bytes + (size_t)C * 4;
         if ((st = slot_scratch(s, kScrClassCount, count_bytes, &d_counts)) != PP_OK ||
             (st = slot_scratch(s, kScrClassStart, (size_t)C * 8, &d_cstart)) != PP_OK ||
             (st = slot_scratch(s, kScrClassOX, (size_t)s->W * ocap * 8, &ox)) != PP_OK ||
             (st = slot_scratch(s, kScrClassOZ, (size_t)s->W * ocap * 8, &oz)) != PP_OK ||
             (st = slot_scratch(s, kScrClassOC, ocap * cb, &oc)) != PP_OK ||
-            (st = slot_scratch(s, kScrClassOB, ocap * 4, &ob)) != PP_OK || (st = ensure_tiles(s, C)) != PP_OK)
-            return st;
+            (st = slot_scratch(s, kScrClassOB, ocap * 4, &ob)) != PP_OK || (st = ensure_tiles(s, C)) != PP_OK) {
+            if (st != PP_ERR_OUT_OF_MEMORY || counted || ocap <= ocap_least + kClassParts) return st;
+            // the estimate does not fit: give back what it took, and as many rows as the outputs turn out to be
+            for (ScratchSlot slot : {kScrClassOX, kScrClassOZ, kScrClassOC, kScrClassOB}) {
+                if (s->scratch[slot]) (void)hipFree(s->scratch[slot]);
+                s->scratch[slot] = nullptr;
+                s->scratch_cap[slot] = 0;
+            }
+            s->class_out_hint = 0;
+            ocap = ocap_least;
+            continue;
+        }
         d_cst = reinterpret_cast<unsigned long long*>(d_counts);
         d_ocount = reinterpret_cast<uint32_t*>(d_counts + kClassStatSlots * 8);
-        uint32_t* const d_ccount = d_ocount + B;
+        uint32_t* const d_ccount = d_ocount + ocount_bytes / 4;
         PP_HIP(ctx, hipMemsetAsync(d_counts, 0, count_bytes, ctx->stream));
         hipError_t e = dispatch(s, [&](auto Wc, auto Tv) {
             constexpr int W = decltype(Wc)::value;
@@ -1833,9 +1854,11 @@ pp_status class_pass(pp_sum* s, const Prepared* layers, uint32_t n, const KeepPr
             a.oc = (T*)oc;
             a.obucket = ob;
             a.ocap = ocap;
+            a.part_rows = ocap / kClassParts;
             a.ocount = d_ocount;
             a.stats = d_cst;
             a.lcap = lcap;
+            a.icap = icap;
             a.tbits = tbits;
             a.chunk_rows = chunk;
             hipError_t r = launch_class_route<W, T>(ctx->stream, a);
@@ -1850,15 +1873,25 @@ pp_status class_pass(pp_sum* s, const Prepared* layers, uint32_t n, const KeepPr
         PP_HIP(ctx, hipMemcpyAsync(h, d_cst, kClassStatSlots * 8, hipMemcpyDeviceToHost, ctx->stream));
         PP_HIP(ctx, hipStreamSynchronize(ctx->stream));
         const unsigned long long flags = h[kClassFlags];
+        untouched = out_rows = part_most = 0;
+        for (uint32_t p = 0; p < kClassParts; ++p) {
+            const unsigned long long* const q = h + kClassPart + kClassLine * p;
+            out_rows += q[0];
+            part_most = std::max<uint64_t>(part_most, q[0]);
+            untouched += q[1];
+        }
         if (flags == 0) break;
-        if ((flags & 3ull) == 0) {  // only the output staging ran out: its exact need is known now
-            ocap = h[kClassOutRows];
+        counted = counted || !(flags & 3ull);
+        if ((flags & 3ull) == 0) {  // only the output staging ran out: the same chunks' need is known now, and roughly
+            ocap = kClassParts * (part_most + part_most / 4);  // how unevenly they spread over the parts
         } else if (attempt == 0) {
             cbits = std::min(cbits + 2, 24);
-            chunk = 32;
+            chunk = fills ? 16 : 32;
+            icap = lcap;
+            tbits = 10;
         } else if (attempt == 1) {
             cbits = std::min(cbits + 1, 24);
-            lcap = 1024;
+            lcap = icap = 1024;
             tbits = 11;
             chunk = 32;
         } else {
@@ -1867,8 +1900,8 @@ pp_status class_pass(pp_sum* s, const Prepared* layers, uint32_t n, const KeepPr
         if (flags & 3ull) ++attempt;
     }
     // the output layout in the spare columns: each bucket's untouched rows, then its class outputs
-    const uint64_t out_rows = h[kClassOutRows], total = h[kClassUntouched] + out_rows;
-    s->class_out_hint = out_rows + out_rows / 8;
+    const uint64_t total = untouched + out_rows;
+    s->class_out_hint = std::max(s->class_out_hint, kClassParts * (part_most + part_most / 8));
     const int in = s->cur, out = 1 - s->cur;
     if ((st = ensure_columns(s, out, total + (uint64_t)kSegAlign * B)) != PP_OK) return st;
     if ((st = ensure_buckets(s, out, B)) != PP_OK) return st;
@@ -1907,13 +1940,15 @@ pp_status class_pass(pp_sum* s, const Prepared* layers, uint32_t n, const KeepPr
         a.oc = (T*)oc;
         a.obucket = ob;
         a.ocap = ocap;
+        a.part_rows = ocap / kClassParts;
+        a.stats = d_cst;
         a.px = s->col[out].x;
         a.pz = s->col[out].z;
         a.pc = (T*)s->col[out].c;
         a.pcap = s->col[out].cap;
         a.pstart = s->bk[out].start;
         a.plen = s->bk[out].len;
-        return launch_class_place<W, T>(ctx->stream, a, out_rows);
+        return launch_class_place<W, T>(ctx->stream, a, part_most);
     });
     PP_HIP(ctx, e);
     // the longest bucket (from the lens kernel) and the layout's end (the scan's total): one synchronization
@@ -1924,8 +1959,8 @@ pp_status class_pass(pp_sum* s, const Prepared* layers, uint32_t n, const KeepPr
     s->max_bucket = (uint32_t)h[kClassLongest];
     s->tail = s->h_stats[3];
     s->has_room = true;
-    for (uint32_t l = 0; l < n && len_after; ++l) len_after[l] = h[kClassUntouched] + h[kClassLayerRows + l];
-    if (h[kClassUntouched] + h[kClassLayerRows + n - 1] != total)
+    for (uint32_t l = 0; l < n && len_after; ++l) len_after[l] = untouched + h[kClassLayerRows + l];
+    if (untouched + h[kClassLayerRows + n - 1] != total)
         return fail(ctx, PP_ERR_DRIVER, "class pass: the last layer's count disagrees with its outputs");
     *done = true;
     return PP_OK;

@@ -338,3 +338,36 @@ def test_general_table_at_2e16_terms():
         assert got == want
     finally:
         g.free()
+
+
+@pytest.mark.parametrize("num_qubits,n", [(2, 15), (9, 33), (40, 600), (70, 5_000)])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_tables_of_few_and_many_entries_equal_the_naive_layer(num_qubits, n, dtype):
+    """The two ways a layer's outputs are spread over threads (a table of under four entries by rows, of more by the
+    patterns of a class), from one nearly full class to many chunks: every output sums its sources in entry order, so
+    both equal the entry-order naive layer bit for bit."""
+    announce(f"class layers by rows and by patterns, {num_qubits} qubits n={n} {np.dtype(dtype).name}")
+    rng = np.random.default_rng([num_qubits, n])
+    kind = 1 if dtype == np.float32 else 0
+    real = np.float32 if kind else float
+    if num_qubits == 2:
+        keys = np.arange(1, 16, dtype=np.uint64).reshape(-1, 1)
+        x, z, c = keys & np.uint64(3), keys >> np.uint64(2), rng.standard_normal(15).astype(dtype)
+    else:
+        x, z, c = random_sum(rng, n, num_qubits, 0.3, dtype)
+    host = PauliSum(num_qubits, x, z, c, dtype=dtype)
+    g = host.to_device(0)
+    terms = terms_of(host, real)
+    pol = truncation.coeff(1e-6).lower()
+    keep = keep_fn(1e-6, None, real)
+    damp = [np.array([[1, 0], [0, math.sqrt(0.7)]]), np.array([[0, math.sqrt(0.3)], [0, 0]])]
+    try:
+        for kraus, qs in [([haar_unitary(rng, 2)], [0]), (damp, [num_qubits - 1]),
+                          ([haar_unitary(rng, 4)], [0, num_qubits - 1])]:
+            p, es = table_from(channel_ptm(kraus, len(qs)), qs, kind)
+            check(g, _native.lib().pp_apply_prepared(g._h, ctypes.byref(p), ctypes.byref(pol)))
+            terms = entry_order_layer(terms, qs, es, keep, real)
+            got = terms_of(g.to_host(), real)
+            assert len(g) == len(terms) and got == terms
+    finally:
+        g.free()
