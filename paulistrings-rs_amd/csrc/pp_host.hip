@@ -563,16 +563,35 @@ pp_status alloc_fixed(pp_sum* s) {
 
 // Wait on the host until a queued kernel has written `seq` to word 4 of its pinned slot, and after a long wait for the
 // stream itself (which reports a failed launch).
-pp_status wait_for_slot(pp_context* ctx, volatile const unsigned long long* h, unsigned long long seq,
+pp_status wait_for_mark(pp_context* ctx, volatile const unsigned long long* mark, unsigned long long seq,
                         const char* never) {
     const auto t0 = std::chrono::steady_clock::now();
-    while (h[4] != seq)
+    while (*mark != seq)
         if (std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(200)) {
             PP_HIP(ctx, hipStreamSynchronize(ctx->stream));
-            if (h[4] != seq) return fail(ctx, PP_ERR_DRIVER, never);
+            if (*mark != seq) return fail(ctx, PP_ERR_DRIVER, never);
             break;
         }
     return PP_OK;
+}
+pp_status wait_for_slot(pp_context* ctx, volatile const unsigned long long* h, unsigned long long seq,
+                        const char* never) {
+    return wait_for_mark(ctx, h + 4, seq, never);
+}
+
+// A layer's counters into h_stats, its rows and longest bucket summed over the layout's bucket lengths behind it (their
+// counters are zero).  The mark is the last word of the read-out slot, which read-outs and selections leave alone.  As
+// read_stats, but no copy and no stream synchronization: for layers that leave no host copy of their own in flight.
+pp_status read_layer_counts(pp_sum* s, const uint32_t* len, uint32_t num_buckets) {
+    pp_context* ctx = s->ctx;
+    if (ctx->capturing) return read_stats(s);  // refused
+    const bool one = num_buckets <= kCountBuckets;
+    if (!one) PP_HIP(ctx, launch_reduce_lens(ctx->stream, len, num_buckets, s->d_stats, nullptr));
+    const unsigned long long seq = ++s->lag_seq;
+    constexpr int kMark = 3 * kStatSlots - 1;
+    PP_HIP(ctx, launch_layer_counts(ctx->stream, one ? len : nullptr, num_buckets, s->d_stats, s->d_lag_host - kStatSlots,
+                                    s->d_lag_host + kMark, seq));
+    return wait_for_mark(ctx, s->h_lag + kMark, seq, "layer: counters never arrived");
 }
 
 pp_status clear_stats(pp_sum* s) {
@@ -1254,7 +1273,7 @@ JoinArgs<W, T> join_args(const pp_sum* src, const pp_sum* dst, int out, const Pr
 }
 
 pp_status launch_join(pp_sum* src, pp_sum* dst, int out, const Prepared& p, const KeepProgram& keep,
-                      const JoinScratch* fixed = nullptr) {
+                      const JoinScratch* fixed = nullptr, bool counted_after = false) {
     pp_context* ctx = src->ctx;
     pp_status st;
     const int in = src->cur;
@@ -1295,7 +1314,7 @@ pp_status launch_join(pp_sum* src, pp_sum* dst, int out, const Prepared& p, cons
     // Up to kJoinCountPairs pairs, the join's workgroups add the totals themselves (one same-address atomic each)
     // and the length-reduce launch is skipped; measurement keeps the reduce, which also feeds the profile counter.
     constexpr uint32_t kJoinCountPairs = 512;
-    const bool count_in_join = !timed && cosets <= kJoinCountPairs;
+    const bool count_in_join = !timed && !counted_after && cosets <= kJoinCountPairs;
     if (timed) {
         PP_HIP(ctx, hipEventCreate(&ev0));
         PP_HIP(ctx, hipEventCreate(&ev1));
@@ -1325,7 +1344,7 @@ pp_status launch_join(pp_sum* src, pp_sum* dst, int out, const Prepared& p, cons
         ctx->events.push_back({ev0, ev1});
         ctx->prof_rows_in += src->len;
     }
-    if (!count_in_join)
+    if (!count_in_join && !counted_after)
         PP_HIP(ctx, launch_reduce_lens(ctx->stream, dst->bk[out].len, B, stats, timed ? ctx->d_prof : nullptr));
     return PP_OK;
 }
@@ -1416,8 +1435,6 @@ pp_status layer_in_place(pp_sum* s, const Prepared& p, const KeepProgram& keep) 
     }
     PP_HIP(ctx, launch_fill_u64(ctx->stream, s->d_stats, kStatSlots, 0ull));
     const bool timed = ctx->profiling && !ctx->capturing;
-    constexpr uint32_t kCountPairs = 512;
-    const bool count_in_join = !timed && cosets <= kCountPairs;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     if (timed) {
         PP_HIP(ctx, hipEventCreate(&ev0));
@@ -1458,7 +1475,6 @@ pp_status layer_in_place(pp_sum* s, const Prepared& p, const KeepProgram& keep) 
             a.redo = s->d_redo;
             a.redo_count = s->d_stats + 4;
             a.redo_mode = redo_mode;
-            a.count_totals = count_in_join ? 1u : 0u;
             a.need = need;
             a.compact = in_place_compaction() ? 1u : 0u;
             if (s->pending_topn) {  // the layer reads its input through the selection
@@ -1469,11 +1485,7 @@ pp_status layer_in_place(pp_sum* s, const Prepared& p, const KeepProgram& keep) 
             return launch_rotation_inplace<W, T>(ctx->stream, a);
         });
     };
-    // the lengths come from the workgroups' own totals (few pairs) or one reduce over the buckets
-    auto count = [&]() -> pp_status {
-        if (!count_in_join) PP_HIP(ctx, launch_reduce_lens(ctx->stream, s->bk[cur].len, B, s->d_stats, nullptr));
-        return read_stats(s);
-    };
+    auto count = [&]() -> pp_status { return read_layer_counts(s, s->bk[cur].len, B); };
     PP_HIP(ctx, launch(0, scap));
     if (timed) {
         PP_HIP(ctx, hipEventRecord(ev1, ctx->stream));
@@ -1483,7 +1495,7 @@ pp_status layer_in_place(pp_sum* s, const Prepared& p, const KeepProgram& keep) 
     if ((st = count()) != PP_OK) return st;  // the one synchronization when every pair fits
     if (s->h_stats[4]) {  // queued pairs: room for their moves, then the redo launch, then the lengths again
         if ((st = grow_columns_keeping(s, cur, s->tail + s->h_stats[7], s->tail)) != PP_OK) return st;
-        if (!count_in_join) PP_HIP(ctx, launch_fill_u64(ctx->stream, s->d_stats, 2, 0ull));
+        if (B > kCountBuckets) PP_HIP(ctx, launch_fill_u64(ctx->stream, s->d_stats, 2, 0ull));
         hipEvent_t r0 = nullptr, r1 = nullptr;
         if (timed) {
             PP_HIP(ctx, hipEventCreate(&r0));
@@ -1546,9 +1558,10 @@ pp_status device_layer(pp_sum* s, const Prepared& p, const KeepProgram& keep) {
     }
     if (join_in_place(s, p)) return layer_in_place(s, p, keep);
     const int out = 1 - s->cur;
-    if ((st = launch_join(s, s, out, p, keep)) != PP_OK) return st;
+    const bool timed = ctx->profiling && !ctx->capturing;
+    if ((st = launch_join(s, s, out, p, keep, nullptr, !timed)) != PP_OK) return st;
     s->pending_topn = false;  // the join read its input through the selection
-    if ((st = read_stats(s)) != PP_OK) return st;
+    if ((st = timed ? read_stats(s) : read_layer_counts(s, s->bk[out].len, B)) != PP_OK) return st;
     if (s->h_stats[2]) return fail(ctx, PP_ERR_DRIVER, "rotation join: a pair exceeded the largest-pair bound");
     s->len = s->h_stats[0];
     s->max_bucket = (uint32_t)s->h_stats[1];

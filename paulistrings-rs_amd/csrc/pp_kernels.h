@@ -92,14 +92,13 @@ struct InplaceArgs {
     T sin_t;
     int32_t clifford;
     KeepProgram keep;
-    // [0] rows and [1] longest bucket when count_totals; [2] |= 1 redo overflow, |= 2 no room to move a pair;
+    // [0] rows and [1] longest bucket, counted after it; [2] |= 1 redo overflow, |= 2 no room to move a pair;
     // [4] queued pairs; [5] rows moved pairs took after tail_base; [6] moved pairs; [7] rows the queued pairs' moves
     // may take
     unsigned long long* stats;
     uint32_t* redo;
     unsigned long long* redo_count;
     uint32_t redo_mode;
-    uint32_t count_totals;
     uint32_t need;     // key words phase A reads of every row: bit 2w x[w], bit 2w + 1 z[w]
     uint32_t compact;  // a side left with more holes than new rows closes them in place (else the pair moves)
     // a TopN selection the layer reads its input through (the filtered launch): rows it drops are holes
@@ -301,6 +300,11 @@ template <int W, typename T>
 hipError_t launch_rotation_join(hipStream_t st, const JoinArgs<W, T>& a, uint32_t groups_per_cu, uint32_t block);
 template <int W, typename T>
 hipError_t launch_rotation_join_small(hipStream_t st, const SmallJoinArgs<W, T>& a);
+// A layer's eight counters to pinned words, then seq to mark (pinned as well).  With len (at most kCountBuckets lengths)
+// counters 0 and 1 are first set to their sum and maximum.
+constexpr uint32_t kCountBuckets = 1u << 14;
+hipError_t launch_layer_counts(hipStream_t st, const uint32_t* len, uint32_t num_buckets, unsigned long long* stats,
+                               unsigned long long* host, unsigned long long* mark, unsigned long long seq);
 // The publication of a small join's counters with no launch after it (one workgroup): as the extra workgroup of
 // k_rotation_join_small does.
 hipError_t launch_publish_counters(hipStream_t st, const uint32_t* len, uint32_t num_buckets,

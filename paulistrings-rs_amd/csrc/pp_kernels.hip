@@ -197,6 +197,61 @@ __global__ void __launch_bounds__(kBlock) k_reduce_lens(const uint32_t* __restri
     }
 }
 
+// A finished layer's counters to the host by one workgroup: with len, the rows and the longest bucket are summed here
+// first (up to kCountBuckets lengths, sixteen loads in flight per thread); then the eight words, and once they have
+// landed the sequence number the host spins on.  A copy and a stream synchronization in its place cost the host 25 us a
+// layer and the device a copy kernel; a layer's own workgroups adding to two counters cost 12 ns each, one after another.
+constexpr uint32_t kCountBlock = 1024;
+__global__ void __launch_bounds__(kCountBlock) k_layer_counts(const uint32_t* __restrict__ len, uint32_t num_buckets,
+                                                              unsigned long long* stats, unsigned long long* host,
+                                                              unsigned long long* mark, unsigned long long seq) {
+    __shared__ unsigned long long rows[kCountBlock / 64];
+    __shared__ uint32_t most[kCountBlock / 64];
+    if (len) {  // uniform
+        uint32_t n[kCountBuckets / kCountBlock];
+#pragma unroll
+        for (uint32_t k = 0; k < kCountBuckets / kCountBlock; ++k) {
+            const uint32_t i = threadIdx.x + k * kCountBlock;
+            n[k] = i < num_buckets ? len[i] : 0u;
+        }
+        unsigned long long sum = 0;
+        uint32_t longest = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < kCountBuckets / kCountBlock; ++k) {
+            sum += n[k];
+            longest = max(longest, n[k]);
+        }
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) {
+            sum += __shfl_down(sum, d, 64);
+            longest = max(longest, (uint32_t)__shfl_down((int)longest, d, 64));
+        }
+        if (lane_id() == 0) {
+            rows[wave_id()] = sum;
+            most[wave_id()] = longest;
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x) return;
+    unsigned long long v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = stats[i];
+    if (len) {
+        v[0] = v[1] = 0;
+        for (uint32_t w = 0; w < kCountBlock / 64; ++w) {
+            v[0] += rows[w];
+            v[1] = max(v[1], (unsigned long long)most[w]);
+        }
+        stats[0] = v[0];
+        stats[1] = v[1];
+    }
+    volatile unsigned long long* h = host;  // fine-grained host memory: the stores bypass the L2
+#pragma unroll
+    for (int i = 0; i < 8; ++i) h[i] = v[i];
+    __builtin_amdgcn_s_waitcnt(0);  // the words land before the mark
+    *(volatile unsigned long long*)mark = seq;
+}
+
 // ---------------------------------------------------------------------------------------------------------------
 // The rotation layer (reference semantics: engine/bucketed/rotation_layer.rs:159-229, :386-463;
 // rotation_layer/merge.rs:53-91, :209-286; the device join it replaces is kern/join.cu:42-212).
@@ -1053,10 +1108,6 @@ __global__ void __launch_bounds__(kBlock) k_rotation_pair(const InplaceArgs<W, T
     if (tid == 0) {
         a.len[b0] = fin0;
         if (pair) a.len[b1] = fin1;
-        if (a.count_totals) {
-            atomicAdd(&a.stats[0], (unsigned long long)(fin0 + fin1));
-            atomicMax(&a.stats[1], (unsigned long long)max(fin0, fin1));
-        }
     }
 }
 
@@ -1338,10 +1389,6 @@ __global__ void __launch_bounds__(kBlock) k_rotation_inplace(const InplaceArgs<W
             if (threadIdx.x == 0) {
                 a.len[b0] = fin0;
                 if (pair) a.len[b1] = fin1;
-                if (a.count_totals) {
-                    atomicAdd(&a.stats[0], (unsigned long long)(fin0 + fin1));
-                    atomicMax(&a.stats[1], (unsigned long long)max(fin0, fin1));
-                }
             }
             continue;
         }
@@ -1434,10 +1481,6 @@ __global__ void __launch_bounds__(kBlock) k_rotation_inplace(const InplaceArgs<W
                 a.bcap[b1] = seg1;
             }
             atomicAdd(&a.stats[6], 1ull);
-            if (a.count_totals) {
-                atomicAdd(&a.stats[0], (unsigned long long)(fin0 + fin1));
-                atomicMax(&a.stats[1], (unsigned long long)max(fin0, fin1));
-            }
         }
     }
 }
@@ -1936,6 +1979,14 @@ hipError_t launch_rotation_join_small(hipStream_t st, const SmallJoinArgs<W, T>&
         return hipErrorInvalidValue;
     const size_t lds = join_lds_bytes<W, T>(a.j.scap, a.j.tcap_bits);
     hipLaunchKernelGGL((k_rotation_join_small<W, T>), dim3(a.j.num_cosets + 1), dim3(kBlock), lds, st, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_layer_counts(hipStream_t st, const uint32_t* len, uint32_t num_buckets, unsigned long long* stats,
+                               unsigned long long* host, unsigned long long* mark, unsigned long long seq) {
+    if (len && num_buckets > kCountBuckets) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_layer_counts, dim3(1), dim3(len ? kCountBlock : 64), 0, st, len, num_buckets, stats, host, mark,
+                       seq);
     return hipGetLastError();
 }
 
