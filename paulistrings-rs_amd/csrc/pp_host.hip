@@ -326,6 +326,7 @@ enum ScratchSlot {
     kScrRunCounts,   // its per-bucket destination counts
     kScrDeaths,      // its per-step drops
     kScrSteps,       // its steps
+    kScrTiny,        // a tiny program's layers and counts
     kScrClassCount,  // a class pass's counters, outputs per bucket and touched rows per class bucket
     kScrClassStart,  // the class buckets' scan
     kScrClassKeep,   // its untouched rows kept per bucket
@@ -3148,7 +3149,7 @@ namespace {
 // takes the synchronous path.  Under a layer pass (TopN, ApproxTopN, the learned pass) a layer is queued while its bound
 // stays within the cap: the pass then does nothing after it, whatever its exact length.  The results are the same either
 // way: only when the host learns the counts changes.  A small layer costs 12 us queued and 30 when its counts are read
-// before the next.
+// before the next; the layers of a sum that one workgroup holds run in one launch (run_tiny_layers).
 
 constexpr uint64_t kLagMaxRows = 1ull << 20;  // above this a layer is bandwidth-bound and its synchronization noise
 constexpr uint32_t kLagDepth = 1;             // layers whose counts may still be on their way when one is queued
@@ -3194,6 +3195,90 @@ pp_status launch_join_small(pp_sum* s, int out, const Prepared& p, const KeepPro
         return launch_rotation_join_small<W, T>(ctx->stream, a);
     });
     PP_HIP(ctx, e);
+    return PP_OK;
+}
+
+// Layers [i, i + m) of a sum of at most kTinyRows rows, all of them rotations, in one launch: *done of them, the lengths
+// after each in lens.  One upload, one launch and one read-back for all of them.
+struct TinyStep {
+    uint64_t gx[4], gz[4];
+    double cos, sin;
+    bool clifford;
+    explicit TinyStep(const Prepared& p) : cos(p.cos), sin(p.sin), clifford(p.clifford) {
+        std::copy(p.gx, p.gx + 4, gx);
+        std::copy(p.gz, p.gz + 4, gz);
+    }
+};
+constexpr uint32_t kTinyLeast = 4;  // layers from which the upload and the read-back cost less than the queue's launches
+pp_status run_tiny_layers(pp_sum* s, const std::vector<TinyStep>& layers, const KeepProgram& keep, uint32_t stop,
+                          std::vector<unsigned long long>* lens, uint32_t* done) {
+    pp_context* ctx = s->ctx;
+    pp_status st;
+    const int in = s->cur, out = 1 - s->cur;
+    const uint32_t B = 1u << s->device_bits, m = (uint32_t)layers.size();
+    if ((st = ensure_columns(s, out, 2 * kTinyRows + (uint64_t)kSegAlign * B)) != PP_OK) return st;
+    if ((st = ensure_buckets(s, out, B)) != PP_OK) return st;
+    std::vector<unsigned long long> got(4 + m);
+    hipError_t e = dispatch(s, [&](auto Wc, auto Tv) {
+        constexpr int W = decltype(Wc)::value;
+        using T = decltype(Tv);
+        std::vector<TinyLayer<W, T>> prog(m);
+        for (uint32_t l = 0; l < m; ++l) {
+            const TinyStep& p = layers[l];
+            TinyLayer<W, T>& t = prog[l];
+            uint32_t gphase = 0;
+            for (int w = 0; w < W; ++w) {
+                t.gx[w] = p.gx[w];
+                t.gz[w] = p.gz[w];
+                gphase += (uint32_t)__builtin_popcountll(p.gx[w] & p.gz[w]);
+            }
+            t.gphase = gphase & 3u;
+            t.cos_t = (T)p.cos;
+            t.sin_t = (T)p.sin;
+            t.clifford = p.clifford ? 1 : 0;
+        }
+        const size_t counts = got.size() * 8, bytes = counts + m * sizeof(TinyLayer<W, T>);
+        unsigned char* block = nullptr;
+        if ((st = slot_scratch(s, kScrTiny, bytes, &block)) != PP_OK) return hipSuccess;
+        hipError_t r = hipMemcpyAsync(block + counts, prog.data(), m * sizeof(TinyLayer<W, T>), hipMemcpyHostToDevice,
+                                      ctx->stream);
+        if (r != hipSuccess) return r;
+        TinyArgs<W, T> a{};
+        a.x = s->col[in].x;
+        a.z = s->col[in].z;
+        a.c = (const T*)s->col[in].c;
+        a.cap = s->col[in].cap;
+        a.start = s->bk[in].start;
+        a.len = s->bk[in].len;
+        a.num_buckets = B;
+        a.bits = s->device_bits;
+        a.rows = s->d_rows;
+        a.layers = (const TinyLayer<W, T>*)(block + counts);
+        a.n_layers = m;
+        a.stop = stop;
+        a.keep = keep;
+        a.ox = s->col[out].x;
+        a.oz = s->col[out].z;
+        a.oc = (T*)s->col[out].c;
+        a.ocap = s->col[out].cap;
+        a.ostart = s->bk[out].start;
+        a.olen = s->bk[out].len;
+        a.orows = s->bk[out].rows;
+        a.out = (unsigned long long*)block;
+        if ((r = launch_tiny_layers<W, T>(ctx->stream, a)) != hipSuccess) return r;
+        r = hipMemcpyAsync(got.data(), block, counts, hipMemcpyDeviceToHost, ctx->stream);
+        return r == hipSuccess ? hipStreamSynchronize(ctx->stream) : r;
+    });
+    if (st != PP_OK) return st;
+    PP_HIP(ctx, e);
+    *done = (uint32_t)got[0];
+    lens->assign(got.begin() + 4, got.begin() + 4 + *done);
+    s->len = got[1];
+    s->max_bucket = (uint32_t)got[2];
+    s->tail = got[3];
+    s->cur = out;
+    s->has_room = true;
+    s->pending_topn = false;
     return PP_OK;
 }
 
@@ -3283,6 +3368,35 @@ pp_status propagate_lagged(pp_sum* s, const RunPlanner& plan, const KeepProgram&
             while (4ull * s->max_bucket > kMaxPairRows && s->device_bits < s->max_bits &&
                    s->len * 8 >= target << (s->device_bits + 1))
                 if ((st = refine_once(s)) != PP_OK) return st;
+            if (s->len > 0 && s->len <= std::min<uint64_t>(small, kTinyRows) &&
+                (1u << s->device_bits) <= kTinyBuckets && !ctx->profiling) {
+                // as many layers as follow of this kind, in one launch
+                std::vector<TinyStep> layers;
+                layers.reserve(kTinyLayers);
+                layers.emplace_back(p);
+                for (uint64_t j = i + 1; j < n && layers.size() < kTinyLayers; ++j) {
+                    const Prepared& q = plan.prepared(s, j);
+                    if (!q.rotation || q.key_preserving ||  // or the start of a permutation run
+                        (is_permutation_step(q) && j + 1 < n && is_permutation_step(plan.prepared(s, j + 1))))
+                        break;
+                    layers.emplace_back(q);
+                }
+                std::vector<unsigned long long> lens;
+                uint32_t done = 0;
+                uint64_t before = s->len;
+                if (layers.size() >= kTinyLeast &&
+                    (st = run_tiny_layers(s, layers, keep, (uint32_t)std::min<uint64_t>(small, kTinyRows), &lens,
+                                          &done)) != PP_OK)
+                    return st;
+                for (uint32_t l = 0; l < done; ++l, ++i) {
+                    plan_at(i, before);
+                    before = lens[l];
+                    if (layer_len) layer_len[i] = before;
+                }
+                known_len = s->len;
+                known_mb = s->max_bucket;
+                if (done) continue;
+            }
             known_len = s->len;
             known_mb = s->max_bucket;
         }

@@ -68,6 +68,43 @@ struct SmallJoinArgs {
     unsigned long long prev_seq;
 };
 
+// Layers of a sum of at most kTinyRows rows (k_tiny_layers), in one launch of one workgroup: layer after layer until the
+// program ends or more than `stop` rows are left, then the layout of the result.
+constexpr uint32_t kTinyRows = 512;
+constexpr uint32_t kTinyBuckets = 8;
+constexpr uint32_t kTinyLayers = 128;
+template <int W, typename T>
+struct TinyLayer {
+    uint64_t gx[W], gz[W];
+    T cos_t, sin_t;
+    uint32_t gphase;
+    int32_t clifford;
+};
+template <int W, typename T>
+struct TinyArgs {
+    const uint64_t* x;
+    const uint64_t* z;
+    const T* c;
+    uint64_t cap;
+    const uint64_t* start;
+    const uint32_t* len;  // at most kTinyRows rows in all
+    uint32_t num_buckets; // at most kTinyBuckets
+    int bits;
+    const uint64_t* rows;
+    const TinyLayer<W, T>* layers;
+    uint32_t n_layers;
+    uint32_t stop;  // at most kTinyRows
+    KeepProgram keep;
+    uint64_t* ox;  // room for 2 kTinyRows rows and kSegAlign a bucket
+    uint64_t* oz;
+    T* oc;
+    uint64_t ocap;
+    uint64_t* ostart;
+    uint32_t* olen;
+    uint32_t* orows;
+    unsigned long long* out;  // [0] layers done, [1] rows, [2] longest bucket, [3] layout end, [4 + l] rows after layer l
+};
+
 // The rotation layer in place (k_rotation_inplace): the sum's own columns and bucket arrays are read and written.
 template <int W, typename T>
 struct InplaceArgs {
@@ -305,6 +342,8 @@ hipError_t launch_rotation_join_small(hipStream_t st, const SmallJoinArgs<W, T>&
 constexpr uint32_t kCountBuckets = 1u << 14;
 hipError_t launch_layer_counts(hipStream_t st, const uint32_t* len, uint32_t num_buckets, unsigned long long* stats,
                                unsigned long long* host, unsigned long long* mark, unsigned long long seq);
+template <int W, typename T>
+hipError_t launch_tiny_layers(hipStream_t st, const TinyArgs<W, T>& a);
 // The publication of a small join's counters with no launch after it (one workgroup): as the extra workgroup of
 // k_rotation_join_small does.
 hipError_t launch_publish_counters(hipStream_t st, const uint32_t* len, uint32_t num_buckets,

@@ -772,6 +772,176 @@ __global__ void __launch_bounds__(kBlock) k_publish_counters(const uint32_t* len
     publish_counters(len, num_buckets, counters, host, seq, part);
 }
 
+// Many layers of a tiny sum by one workgroup, a row per thread in registers: each layer enters its anticommuting rows in
+// an LDS table, looks each one's partner up, and compacts what stays through LDS for the next.  The arithmetic is the
+// pair join's, row by row.  A layer is four barriers; as a launch of its own it was 8 us of kernel and 4 of gap: the 96
+// layers of a 16-qubit observable, up to 465 terms, with its uploads and its read-out, take 0.69 ms in place of 1.55.  Beyond kTinyRows a thread would hold several rows and
+// the pair join has workgroups to spread them over.
+template <int W, typename T>
+__global__ void __launch_bounds__(kTinyRows) k_tiny_layers(const TinyArgs<W, T> a) {
+    constexpr uint32_t kBits = 10;  // twice the rows
+    static_assert((1u << kBits) == 2 * kTinyRows, "table load at most 1/2");
+    __shared__ uint64_t Lx[W][2 * kTinyRows], Lz[W][2 * kTinyRows];
+    __shared__ T Lc[2 * kTinyRows];
+    __shared__ uint32_t table[1u << kBits];
+    __shared__ uint32_t scratch[2][kTinyRows / 64];
+    const uint32_t tid = threadIdx.x;
+    Key<W> k{};
+    T c = T(0);
+    uint32_t n = 0;
+    bool valid = false;
+    for (uint32_t b = 0; b < a.num_buckets; ++b) {
+        const uint32_t m = a.len[b];
+        if (!valid && tid - n < m) {
+            const uint64_t row = a.start[b] + (tid - n);
+            k = load_key<W>(a.x, a.z, a.cap, row);
+            c = a.c[row];
+            valid = true;
+        }
+        n += m;
+    }
+    TinyLayer<W, T> next = a.layers[0];
+    uint32_t l = 0;
+    for (;;) {
+        const TinyLayer<W, T> t = next;
+        if (l + 1 < a.n_layers) next = a.layers[l + 1];
+        Key<W> g;
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            g.x[w] = t.gx[w];
+            g.z[w] = t.gz[w];
+        }
+        const uint32_t supp = support_words<W>(g);
+        for (uint32_t i = tid; i < (1u << kBits); i += kTinyRows) table[i] = 0u;
+        __syncthreads();  // the rows of the layer before are read, the table is clear
+        const bool anti = valid && anticommutes_on<W>(k, g, supp);
+        uint32_t fold = 0;
+        if (anti) {
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                Lx[w][tid] = k.x[w];
+                Lz[w][tid] = k.z[w];
+            }
+            Lc[tid] = c;
+            fold = key_fold<W>(k);
+            const uint32_t h = fold_mix(fold);
+            uint32_t s = h >> (32u - kBits);
+            while (atomicCAS(&table[s], 0u, (h << 16) | (tid + 1u)) != 0u) s = (s + 1u) & ((1u << kBits) - 1u);
+        }
+        __syncthreads();
+        T own = c, fresh = T(0);
+        Key<W> q{};
+        bool f[2] = {valid && !anti && survives<W, T>(a.keep, k, c), false};
+        if (anti) {
+            q = key_xor<W>(k, g);
+            const uint32_t h = fold_mix(fold ^ key_fold<W>(g));
+            uint32_t s = h >> (32u - kBits);
+            int found = -1;
+            for (;;) {
+                const uint32_t e = table[s];
+                if (e == 0u) break;
+                if ((e & 0xFFFF0000u) == h << 16) {
+                    const uint32_t ix = (e & 0xFFFFu) - 1u;
+                    bool eq = true;
+#pragma unroll
+                    for (int w = 0; w < W; ++w) eq = eq && (Lx[w][ix] == q.x[w]) && (Lz[w][ix] == q.z[w]);
+                    if (eq) {
+                        found = (int)ix;
+                        break;
+                    }
+                }
+                s = (s + 1u) & ((1u << kBits) - 1u);
+            }
+            const T a1 = partner_amplitude_on<W, T>(found >= 0 ? q : k, g, supp, t.gphase, t.sin_t);
+            own = t.clifford ? T(0) : c * t.cos_t;
+            if (found >= 0) own = own + Lc[found] * a1;
+            f[0] = survives<W, T>(a.keep, k, own);
+            if (found < 0) {
+                fresh = c * a1;
+                f[1] = survives<W, T>(a.keep, q, fresh);
+            }
+        }
+        uint32_t off[2], tot[2];
+        block_flag_scan<2, kTinyRows / 64>(f, off, tot, scratch[l & 1u]);  // its barrier ends the lookups
+        if (f[0]) {
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                Lx[w][off[0]] = k.x[w];
+                Lz[w][off[0]] = k.z[w];
+            }
+            Lc[off[0]] = own;
+        }
+        if (f[1]) {
+            const uint32_t at = tot[0] + off[1];
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                Lx[w][at] = q.x[w];
+                Lz[w][at] = q.z[w];
+            }
+            Lc[at] = fresh;
+        }
+        n = tot[0] + tot[1];
+        if (tid == 0) a.out[4 + l] = n;
+        ++l;
+        __syncthreads();
+        if (l == a.n_layers || n > a.stop) break;  // uniform
+        valid = tid < n;
+        if (valid) {
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                k.x[w] = Lx[w][tid];
+                k.z[w] = Lz[w][tid];
+            }
+            c = Lc[tid];
+        }
+    }
+    // the layout: rows tid and tid + kTinyRows, bucket after bucket
+    Key<W> r[2];
+    uint32_t bucket[2];
+#pragma unroll
+    for (uint32_t j = 0; j < 2; ++j) {
+        const uint32_t i = tid + j * kTinyRows;
+        bucket[j] = kTinyBuckets;
+        if (i < n) {
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                r[j].x[w] = Lx[w][i];
+                r[j].z[w] = Lz[w][i];
+            }
+            bucket[j] = bucket_of<W>(r[j], a.rows, a.bits);
+        }
+    }
+    uint64_t start = 0;
+    uint32_t longest = 0;
+    for (uint32_t b = 0; b < a.num_buckets; ++b) {
+        __syncthreads();  // the scratch is free again
+        bool f[2] = {bucket[0] == b, bucket[1] == b};
+        uint32_t off[2], tot[2];
+        block_flag_scan<2, kTinyRows / 64>(f, off, tot, scratch[0]);
+#pragma unroll
+        for (uint32_t j = 0; j < 2; ++j)
+            if (f[j]) {
+                const uint64_t pos = start + (j ? tot[0] : 0u) + off[j];
+                store_key<W>(a.ox, a.oz, a.ocap, pos, r[j]);
+                store_coeff<T>(a.oc, pos, Lc[tid + j * kTinyRows]);
+            }
+        const uint32_t m = tot[0] + tot[1], room = (m + (kSegAlign - 1)) & ~(kSegAlign - 1);
+        if (tid == 0) {
+            a.ostart[b] = start;
+            a.olen[b] = m;
+            a.orows[b] = room;
+        }
+        longest = max(longest, m);
+        start += room;
+    }
+    if (tid == 0) {
+        a.out[0] = l;
+        a.out[1] = n;
+        a.out[2] = longest;
+        a.out[3] = start;
+    }
+}
+
 // ---------------------------------------------------------------------------------------------------------------
 // The rotation layer in place.  A workgroup per pair {b0, b1} reads every row of the pair, as k_rotation_join does,
 // but writes only what the layer changes: the coefficient of an anticommuting row that stays, and the new partner
@@ -1982,6 +2152,15 @@ hipError_t launch_rotation_join_small(hipStream_t st, const SmallJoinArgs<W, T>&
     return hipGetLastError();
 }
 
+template <int W, typename T>
+hipError_t launch_tiny_layers(hipStream_t st, const TinyArgs<W, T>& a) {
+    if (a.n_layers == 0 || a.n_layers > kTinyLayers || a.num_buckets == 0 || a.num_buckets > kTinyBuckets ||
+        a.num_buckets != 1u << a.bits || a.stop > kTinyRows || a.ocap < 2 * kTinyRows + kSegAlign * a.num_buckets)
+        return hipErrorInvalidValue;
+    hipLaunchKernelGGL((k_tiny_layers<W, T>), dim3(1), dim3(kTinyRows), 0, st, a);
+    return hipGetLastError();
+}
+
 hipError_t launch_layer_counts(hipStream_t st, const uint32_t* len, uint32_t num_buckets, unsigned long long* stats,
                                unsigned long long* host, unsigned long long* mark, unsigned long long seq) {
     if (len && num_buckets > kCountBuckets) return hipErrorInvalidValue;
@@ -2153,6 +2332,7 @@ hipError_t launch_check_layout(hipStream_t st, const CheckArgs<W, T>& a) {
     template size_t join_lds_bytes<W, T>(uint32_t, uint32_t);                                          \
     template hipError_t launch_rotation_join<W, T>(hipStream_t, const JoinArgs<W, T>&, uint32_t, uint32_t); \
     template hipError_t launch_rotation_join_small<W, T>(hipStream_t, const SmallJoinArgs<W, T>&);      \
+    template hipError_t launch_tiny_layers<W, T>(hipStream_t, const TinyArgs<W, T>&);                   \
     template hipError_t launch_join_batch<W, T>(hipStream_t, const JoinArgs<W, T>*, const uint32_t*,               \
                                                 const BatchAnswer*, uint32_t, uint32_t, uint32_t, uint32_t);    \
     template hipError_t launch_rescale<W, T>(hipStream_t, const RescaleArgs<W, T>&, uint32_t);          \

@@ -205,3 +205,35 @@ def test_layer_pass_joins_and_leaves_the_queue(monkeypatch, cap, kind, num_qubit
     want = run(monkeypatch, False, num_qubits, x, z, c, circ, "heisenberg", pol)
     assert_equal_runs(got, want)
     assert got[4][0] == want[4][0]  # the reference's bucket count
+
+
+@pytest.mark.parametrize("num_qubits,dtype", [(20, np.float64), (64, np.float32), (65, np.float64), (127, np.float32)])
+@pytest.mark.parametrize("n", [1, 2, 255, 511, 512, 513])
+@pytest.mark.parametrize("cap", [None, 1, 300, 700, 5_000])
+def test_tiny_layers_in_one_launch(monkeypatch, num_qubits, dtype, n, cap):
+    """Sums about the rows one workgroup holds, more layers than one launch takes, through growth past it, a cap below
+    and above it, and kinds of layer it leaves: bit for bit the layers one by one, lengths and bucket counts too."""
+    announce(f"tiny layers qubits={num_qubits} n={n} cap={cap}")
+    rng = np.random.default_rng([num_qubits, n])
+    x, z, c = random_sum(rng, n, num_qubits, 0.15)
+    c = c.astype(dtype)
+    circ = Circuit(num_qubits)
+    for _ in range(150):
+        q = int(rng.integers(0, num_qubits - 1))
+        circ.rzz(float(rng.uniform(0.05, 0.3)), q, q + 1)
+    circ.extend(mixed_circuit(rng, num_qubits, 30))
+    pol = truncation.coeff(0.03)
+    if cap is not None:
+        pol = pol & truncation.topn(cap)
+
+    def tiny(on):
+        monkeypatch.setenv("PP_LAGGED_LENGTHS", on)
+        s = PauliSum(num_qubits, x, z, c, dtype=dtype).to_device(0)
+        stats = s.propagate_with_stats(circ, policy=pol, direction="heisenberg")
+        bad = {k: v for k, v in s.check_layout().items() if v and k != "unscanned"}
+        assert not bad, bad
+        bits, h = s.bucket_bits()[0], s.to_host()
+        s.free()
+        return h.x_array(), h.z_array(), h.coefficients_array(), np.array(stats.terms_out), np.array(bits)
+
+    assert all(np.array_equal(a, b) for a, b in zip(tiny("1"), tiny("0")))
