@@ -116,7 +116,7 @@ def host_sum(x, z, c):
 
 
 def gpu_measure_in_place(x, z, c, channels, steps: int, warmup: int):
-    """Each channel as one layer in place (k_rotation_inplace) on a working sum reset from the resident input before
+    """Each channel as one layer in place (k_rotation_pair) on a working sum reset from the resident input before
     it (pp_sum_copy, outside the timed region): the layer reads every row and writes only what it changes.  A
     step's time is the sum of its 190 layer calls, each from its launch to its counts on the host."""
     from paulistrings_amd import truncation
@@ -860,7 +860,7 @@ def main() -> int:
         },
         "cpu_baseline": cpu,
         "detail": {
-            "kernel": "k_rotation_inplace",
+            "kernel": "k_rotation_pair",
             "protocol": "each channel one layer in place on a working sum reset from the resident input before it "
                         "(untimed); a step is the sum of its 190 layer calls; the in-place layer reads every row and "
                         "writes only the coefficients it changes and the new rows, so achieved (algorithmic bytes of "
@@ -868,8 +868,8 @@ def main() -> int:
             "out_of_place": oop,
             "layers": layers,
             "kernel_launches": r["launches"],
-            "launch_unit": "one layer: the first k_rotation_inplace launch, plus a second over queued pairs on the "
-                           "layers where a pair outgrew the first launch's stage",
+            "launch_unit": "one layer: the k_rotation_pair launch over every pair, plus a k_rotation_inplace launch over "
+                           "queued pairs on the layers where a pair outgrew the first launch's stage",
             "kernel_ms_per_layer": r["kernel_ms"] / max(1, layers),
             "kernel_share_of_wall": kernel_s / r["seconds"],
             "rows_in_per_layer": r["rows_in"] / max(1, layers),
