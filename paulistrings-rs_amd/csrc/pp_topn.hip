@@ -715,12 +715,17 @@ __device__ __forceinline__ bool rank_ties(const Args& a, RankScratch<W>& r, cons
 }
 template <int W, typename T, typename Args>
 __device__ __forceinline__ bool rank_boundary(const Args& a, RankScratch<W>& r, const uint64_t* su, const uint64_t* sp,
-                                              uint32_t n, uint64_t k, uint64_t& boundary, uint64_t& stay,
+                                              uint32_t n, uint64_t k, bool one, uint64_t& boundary, uint64_t& stay,
                                               uint32_t& equal) {
     const uint32_t tid = threadIdx.x;
     if (tid == 0) r.ties = 0u;
+    if (one && tid == 0) {  // every digit decided: the listed keys are one key
+        r.found[0] = su[0];
+        r.found[1] = 0;
+        r.found[2] = n;
+    }
     const uint32_t g = lanes_per_key(n);
-    for (uint32_t i0 = 0; i0 < n; i0 += kFinishBlock / g) {  // uniform
+    for (uint32_t i0 = 0; !one && i0 < n; i0 += kFinishBlock / g) {  // uniform
         const uint32_t i = i0 + tid / g;
         const uint64_t u = i < n ? su[i] : 0;
         uint32_t greater = 0, same = 0;
@@ -746,8 +751,50 @@ __device__ __forceinline__ bool rank_boundary(const Args& a, RankScratch<W>& r, 
     return stay == equal || rank_ties<W>(a, r, su, sp, n, boundary, equal, stay);
 }
 
+// A list of n keys (at most kWindowList, in [base, base + 2^shift)) cut by further digits until at most kWindowRank are left
+// or they are equal: every pass in LDS, two keys a thread, where a pass over the collected keys is up to 40 us.  A run of
+// more than kWindowRank equal keys takes five or six of them (60 000 f32 terms, 240 selections: 30.0 -> 26.5 us a finish).
+__device__ __forceinline__ void narrow_list(uint64_t* su, uint64_t* sp, uint32_t& n, uint32_t* held, uint64_t& base,
+                                            int& shift, uint64_t& k, uint32_t* hist, uint64_t* part) {
+    constexpr uint32_t kDigits = 2048;
+    static_assert(kWindowList == 2 * kFinishBlock, "two keys a thread");
+    const uint32_t tid = threadIdx.x;
+    while (n > kWindowRank && shift > 0) {  // uniform
+        const int sh = max(shift - 11, 0);
+        uint64_t u[2] = {0, 0}, p[2] = {0, 0};
+#pragma unroll
+        for (uint32_t q = 0; q < 2; ++q)
+            if (tid + q * kFinishBlock < n) {
+                u[q] = su[tid + q * kFinishBlock];
+                p[q] = sp[tid + q * kFinishBlock];
+            }
+        for (uint32_t i = tid; i < kDigits; i += kFinishBlock) hist[i] = 0u;
+        __syncthreads();
+        if (tid == 0) *held = 0u;
+#pragma unroll
+        for (uint32_t q = 0; q < 2; ++q)
+            if (tid + q * kFinishBlock < n) atomicAdd(&hist[(u[q] - base) >> sh], 1u);
+        __syncthreads();
+        uint64_t bin[3];
+        window_bin<kDigits, kFinishBlock>(hist, k, part, bin);
+        base += bin[0] << sh;
+        k -= bin[1];
+        shift = sh;
+#pragma unroll
+        for (uint32_t q = 0; q < 2; ++q)
+            if (tid + q * kFinishBlock < n && ((u[q] - base) >> sh) == 0) {
+                const uint32_t slot = atomicAdd(held, 1u);
+                su[slot] = u[q];
+                sp[slot] = p[q];
+            }
+        __syncthreads();
+        n = (uint32_t)bin[2];  // = *held
+    }
+}
+
 // The n-th key among the collected (or narrowed) ones, by one workgroup: 11-bit digits of the window until at most
-// kWindowRank keys are left or they are equal, those ranked by counting, and the keys equal to the boundary put into canonical order when
+// kWindowList keys are left, more of them on that list until at most kWindowRank are left or they are equal, those ranked
+// by counting, and the keys equal to the boundary put into canonical order when
 // only some of them stay.  Then the state the next layer reads, the answer to the host, and the counts cleared.
 template <int W, typename T>
 __global__ void __launch_bounds__(kFinishBlock) k_window_finish(const WindowArgs<W, T> a) {
@@ -775,7 +822,7 @@ __global__ void __launch_bounds__(kFinishBlock) k_window_finish(const WindowArgs
         int shift = 64;  // the keys sought lie in [base, base + 2^shift)
         if (m > kWindowRank) {
             shift = 64 - __builtin_clzll(a.hi - a.lo);
-            do {
+            while (left > kWindowList && shift > 0) {
                 const int sh = max(shift - 11, 0);
                 for (uint32_t i = tid; i < kDigits; i += kFinishBlock) hist[i] = 0u;
                 __syncthreads();
@@ -795,7 +842,7 @@ __global__ void __launch_bounds__(kFinishBlock) k_window_finish(const WindowArgs
                 k -= bin[1];
                 left = bin[2];
                 shift = sh;
-            } while (left > kWindowRank && shift > 0);
+            }
         }
         done = left <= kWindowList;  // else more equal keys than the list holds
         if (done) {
@@ -815,7 +862,9 @@ __global__ void __launch_bounds__(kFinishBlock) k_window_finish(const WindowArgs
                     }
             }
             __syncthreads();
-            done = rank_boundary<W, T>(a, ranked, su, sp, held, k, boundary, stay, equal);  // held = left
+            uint32_t n = held;  // = left
+            narrow_list(su, sp, n, &held, base, shift, k, hist, part);
+            done = rank_boundary<W, T>(a, ranked, su, sp, n, k, shift == 0, boundary, stay, equal);
         }
     }
     const bool crowded = !done && !keep_all && a.narrow && t.fullest > a.room && t.inside(a.n);  // uniform
@@ -962,7 +1011,7 @@ __global__ void __launch_bounds__(kFinishBlock) k_topn_whole(const WholeArgs<W, 
         }
         base = (bin[0] + (outside ? 0 : low)) << shift;
         k -= bin[1];
-        while (bin[2] > kWindowRank && shift > 0) {
+        while (bin[2] > kWindowList && shift > 0) {
             const int sh = max(shift - 11, 0);
             for (uint32_t i = tid; i < kDigits; i += kFinishBlock) hist[i] = 0u;
             __syncthreads();
@@ -986,7 +1035,9 @@ __global__ void __launch_bounds__(kFinishBlock) k_topn_whole(const WholeArgs<W, 
                 }
             });
             __syncthreads();
-            done = rank_boundary<W, T>(a, ranked, su, sp, held, k, boundary, stay, equal);
+            uint32_t listed = held;
+            narrow_list(su, sp, listed, &held, base, shift, k, hist, part);
+            done = rank_boundary<W, T>(a, ranked, su, sp, listed, k, shift == 0, boundary, stay, equal);
         }
     }
     if (tid == 0) {
