@@ -110,6 +110,7 @@ constexpr uint32_t kWindowStage = 1024; // a scanning workgroup's collected keys
 constexpr uint32_t kWindowRank = 256;   // keys the last workgroup ranks by counting when their digits still differ
 constexpr uint32_t kWindowList = 2048;  // and at most (a run of equal keys cannot be told apart by digits)
 constexpr uint32_t kWindowTies = 1024;  // equal keys it puts into canonical order
+constexpr uint64_t kWindowSpan = 1ull << 62;  // a window's keys span less
 enum WindowStatus : uint32_t { kWindowMissed = 1, kWindowDone = 2, kWindowCrowded = 3 };
 
 // Workgroup w of the scan adds to part w % kWindowParts of the counters (a line of their own each) and collects into that

@@ -1071,7 +1071,7 @@ hipError_t launch_topn_whole(hipStream_t st, const WholeArgs<W, T>* items, uint3
 template <int W, typename T>
 bool window_args_valid(const WindowArgs<W, T>& a) {
     return a.buckets_per_block != 0 && a.buckets_per_block <= kHistBucketsMax && a.hi > a.lo && a.n != 0 &&
-           a.hi - a.lo < (1ull << 62) && a.bin_shift >= 0 && a.bin_shift <= 63 &&
+           a.hi - a.lo < kWindowSpan && a.bin_shift >= 0 && a.bin_shift <= 63 &&
            ((a.hi - a.lo - 1) >> a.bin_shift) < kWindowBins;
 }
 
