@@ -3357,10 +3357,11 @@ pp_status propagate_lagged(pp_sum* s, const RunPlanner& plan, const KeepProgram&
         if (lag && is_permutation_step(p) && i + 1 < n &&
             is_permutation_step(plan.prepared(s, i + 1)))
             lag = false;  // the start of a permutation run: walked in one pass
-        // the rows a layer may queue from: below the in-place layer's, and under a layer pass half its cap
-        const uint64_t small = std::min({kLagMaxRows, plan.limit / 2,
-                                         ctx->tuning.join_in_place ? in_place_min_rows() - 1 : kLagMaxRows});
-        if (queued == 0 && s->len > small) lag = false;
+        // a layer queues from fewer rows than `small`: fewer than the in-place layer takes (which may be any number,
+        // 0 included), and under a layer pass at most half its cap
+        const uint64_t small = std::min({kLagMaxRows + 1, plan.limit / 2 + 1,
+                                         ctx->tuning.join_in_place ? in_place_min_rows() : UINT64_MAX});
+        if (queued == 0 && s->len >= small) lag = false;
         if (lag && queued == 0) {
             // exact counts: the device bucketing for the layers to come, fine enough that a pair stays within the
             // join's largest stage under the doubled bound (but not so fine that the next settle coarsens it back)
@@ -3368,7 +3369,8 @@ pp_status propagate_lagged(pp_sum* s, const RunPlanner& plan, const KeepProgram&
             while (4ull * s->max_bucket > kMaxPairRows && s->device_bits < s->max_bits &&
                    s->len * 8 >= target << (s->device_bits + 1))
                 if ((st = refine_once(s)) != PP_OK) return st;
-            if (s->len > 0 && s->len <= std::min<uint64_t>(small, kTinyRows) &&
+            const uint32_t tiny = (uint32_t)std::min<uint64_t>(small - 1, kTinyRows);  // the length is below small
+            if (s->len > 0 && s->len <= tiny &&
                 (1u << s->device_bits) <= kTinyBuckets && !ctx->profiling) {
                 // as many layers as follow of this kind, in one launch
                 std::vector<TinyStep> layers;
@@ -3385,8 +3387,7 @@ pp_status propagate_lagged(pp_sum* s, const RunPlanner& plan, const KeepProgram&
                 uint32_t done = 0;
                 uint64_t before = s->len;
                 if (layers.size() >= kTinyLeast &&
-                    (st = run_tiny_layers(s, layers, keep, (uint32_t)std::min<uint64_t>(small, kTinyRows), &lens,
-                                          &done)) != PP_OK)
+                    (st = run_tiny_layers(s, layers, keep, tiny, &lens, &done)) != PP_OK)
                     return st;
                 for (uint32_t l = 0; l < done; ++l, ++i) {
                     plan_at(i, before);
@@ -3401,7 +3402,7 @@ pp_status propagate_lagged(pp_sum* s, const RunPlanner& plan, const KeepProgram&
             known_mb = s->max_bucket;
         }
         const uint64_t len_hi = known_len << queued, mb_hi = known_mb << queued;
-        lag = lag && len_hi <= small && 2 * mb_hi <= kMaxPairRows;
+        lag = lag && len_hi < small && 2 * mb_hi <= kMaxPairRows;
         const int out = 1 - s->cur;
         const uint32_t B = 1u << s->device_bits;
         const uint64_t need = 2 * len_hi + (uint64_t)kSegAlign * B;
