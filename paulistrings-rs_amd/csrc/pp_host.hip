@@ -2298,8 +2298,9 @@ static pp_status upload_rows(pp_sum* s, uint32_t n, uint64_t m, int bits, unsign
 
 // The n >= 1 host terms into s's first column set, bucketed on the device into the layout the host's stable counting
 // sort would make: the arrays go up as they are, a count gives every term its bucket, a scan lays the segments out, and
-// each bucket's rows are gathered in the host's order.  *done = false, nothing kept, when a bucket is longer than
-// kUploadBucketRows.
+// each bucket's rows are gathered in the host's order.  Its arrays take as much device memory again as the sum, given back
+// on every return.  *done = false, nothing kept, when a bucket is longer than kUploadBucketRows or the memory is short
+// (PP_ERR_OUT_OF_MEMORY; a column set that could be had stays for the host's rows).
 static pp_status upload_bucketed(pp_sum* s, uint32_t n, const uint64_t* x, const uint64_t* z, const void* coeff,
                                  bool* done) {
     pp_context* ctx = s->ctx;
@@ -2430,7 +2431,9 @@ pp_status pp_sum_upload(pp_context* ctx, uint32_t num_qubits, uint32_t width, pp
     const size_t cb = s->coeff_bytes();
     if (n >= kDeviceUploadTerms && n <= UINT32_MAX) {
         bool done = false;
-        if ((st = upload_bucketed(s, (uint32_t)n, x, z, coeff, &done)) != PP_OK) return bail(st);
+        // out of memory: the host's bucketing below needs no device memory but the sum's own
+        if ((st = upload_bucketed(s, (uint32_t)n, x, z, coeff, &done)) != PP_OK && st != PP_ERR_OUT_OF_MEMORY)
+            return bail(st);
         if (done) {
             *out = s;
             return PP_OK;

@@ -1,0 +1,58 @@
+"""Calls that take more device memory than they need when there is plenty of it, with most of the device's memory taken by
+another owner: they have to fall back to what they cannot do without, with the same result."""
+
+from __future__ import annotations
+
+import contextlib
+
+import numpy as np
+import pytest
+
+from test_gpu_transfer import upload
+
+pytestmark = pytest.mark.gpu
+
+MB = 1 << 20
+
+
+@contextlib.contextmanager
+def device_memory_left(megabytes):
+    torch = pytest.importorskip("torch")
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    taken = []
+    try:
+        for _ in range(10):  # memory just freed may be reported late
+            more = torch.cuda.mem_get_info()[0] - megabytes * MB
+            if more <= 16 * MB:
+                break
+            taken.append(torch.empty(more, dtype=torch.uint8, device="cuda"))
+        assert abs(torch.cuda.mem_get_info()[0] - megabytes * MB) <= 32 * MB
+        yield
+    finally:
+        taken.clear()
+        torch.cuda.empty_cache()
+
+
+def spread_terms(n, num_qubits, dtype):
+    """n distinct one-word terms (an odd multiplier permutes the x words)."""
+    mask = np.uint64((1 << num_qubits) - 1)
+    i = np.arange(n, dtype=np.uint64)
+    x = (i * np.uint64(0x9E3779B97F4A7C15)) & mask
+    z = (i * np.uint64(0xD1B54A32D192ED03) >> np.uint64(7)) & mask
+    return x.reshape(-1, 1), z.reshape(-1, 1), (1.0 + i % 1000).astype(dtype)
+
+
+def test_an_upload_beside_little_free_memory():
+    """2^23 terms: the columns take 275 MB, the terms as they arrive, bucketed on the device, 235 MB more."""
+    x, z, c = spread_terms(1 << 23, 50, np.float32)
+    g = upload(50, x, z, c)
+    want = g.to_host()
+    g.free()
+    with device_memory_left(400):
+        g = upload(50, x, z, c)
+        assert len(g) == len(c)
+    assert not any(v for k, v in g.check_layout().items() if k != "unscanned")
+    got = g.to_host()
+    g.free()
+    assert np.array_equal(got._x, want._x) and np.array_equal(got._z, want._z) and np.array_equal(got._c, want._c)
