@@ -2429,7 +2429,7 @@ pp_status pp_sum_upload(pp_context* ctx, uint32_t num_qubits, uint32_t width, pp
         return bail(fail(ctx, PP_ERR_DRIVER, "hash rows upload"));
 
     const size_t cb = s->coeff_bytes();
-    if (n >= kDeviceUploadTerms && n <= UINT32_MAX) {
+    if (n >= kDeviceUploadTerms && n <= kUploadTerms) {
         bool done = false;
         // out of memory: the host's bucketing below needs no device memory but the sum's own
         if ((st = upload_bucketed(s, (uint32_t)n, x, z, coeff, &done)) != PP_OK && st != PP_ERR_OUT_OF_MEMORY)

@@ -13,6 +13,8 @@ namespace pp {
 // grows with its square), and the largest reference bucket a download sorts in one workgroup's LDS (the keys, the
 // coefficients and a 16-bit index per row: 84 KiB at W = 2, 104 KiB at W = 1).
 constexpr uint32_t kUploadBucketRows = 2048;
+// The most terms: a term's number, and the grid's threads past the last term, are 32-bit.
+constexpr uint64_t kUploadTerms = 0xFFFFFFFFull - kBlock;
 template <int W>
 constexpr uint32_t kSortRows = W == 1 ? 4096u : 2048u;
 constexpr uint32_t kSortParts = 256;  // device buckets one reference bucket may gather, or the other way round

@@ -199,9 +199,12 @@ __global__ void __launch_bounds__(512) k_sort_export(const SortExportArgs<W, T> 
 
 }  // namespace
 
+static_assert(kUploadTerms + kBlock - 1 < 1ull << 32, "the grid's rounding and its thread numbers stay in 32 bits");
+
 template <int W, typename T>
 hipError_t launch_upload_count(hipStream_t st, const UploadArgs<W, T>& a) {
     if (a.n == 0) return hipSuccess;
+    if (a.n > kUploadTerms) return hipErrorInvalidValue;
     hipLaunchKernelGGL((k_upload_count<W, T>), dim3((a.n + kBlock - 1) / kBlock), dim3(kBlock), 0, st, a);
     return hipGetLastError();
 }
@@ -209,6 +212,7 @@ hipError_t launch_upload_count(hipStream_t st, const UploadArgs<W, T>& a) {
 template <int W, typename T>
 hipError_t launch_upload_rows(hipStream_t st, const UploadArgs<W, T>& a) {
     if (a.n == 0) return hipSuccess;
+    if (a.n > kUploadTerms) return hipErrorInvalidValue;
     hipLaunchKernelGGL((k_upload_index<W, T>), dim3((a.n + kBlock - 1) / kBlock), dim3(kBlock), 0, st, a);
     hipLaunchKernelGGL((k_upload_rows<W, T>), dim3(a.num_buckets), dim3(kBlock), 0, st, a);
     return hipGetLastError();
