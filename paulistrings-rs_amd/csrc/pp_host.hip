@@ -285,7 +285,9 @@ struct pp_context {
     hipEvent_t stage_ev[2] = {nullptr, nullptr};
     void* class_pinned = nullptr;  // a class pass's program on its way up and its counters on their way down
     // The sums' pinned slots, carved from blocks of kSlotBlock that stay with the context: a pinned allocation of its own
-    // costs a sum 0.1 ms, and giving it back 0.2-0.4 ms.
+    // costs a sum 0.1 ms, and giving it back 0.2-0.4 ms.  Under a lock: a host language's collector may free a sum on a
+    // thread of its own while another makes one.
+    std::mutex slot_mutex;
     std::vector<void*> slot_blocks;
     std::vector<unsigned long long*> free_slots;
     hipEvent_t lag_ev[2] = {nullptr, nullptr};  // the counters of a layer queued ahead of them have arrived
@@ -525,22 +527,34 @@ pp_status read_stats(pp_sum* s) {
 constexpr size_t kSumSlotWords = 4 * kStatSlots;  // a sum's pinned words: h_stats, then the three slots of h_lag
 constexpr size_t kSlotBlock = (size_t)1 << 14;    // 64 sums' worth
 
-// A new sum's fixed device memory (one allocation: counters, read-out partials, hash rows, selection state, histograms
-// and window counts) and its pinned slots.
-pp_status alloc_fixed(pp_sum* s) {
-    pp_context* ctx = s->ctx;
+// A sum's pinned words from the context's pool (null: no pinned memory left), and back into it.
+unsigned long long* take_slot(pp_context* ctx) {
+    std::lock_guard<std::mutex> lock(ctx->slot_mutex);
     if (ctx->free_slots.empty()) {
         void* block = nullptr;
         if (hipHostMalloc(&block, kSlotBlock, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
             (void)hipGetLastError();
-            return fail(ctx, PP_ERR_OUT_OF_MEMORY, "pinned host allocation");
+            return nullptr;
         }
         ctx->slot_blocks.push_back(block);
         for (size_t w = 0; w + kSumSlotWords <= kSlotBlock / 8; w += kSumSlotWords)
             ctx->free_slots.push_back((unsigned long long*)block + w);
     }
-    s->h_stats = ctx->free_slots.back();
+    unsigned long long* const slot = ctx->free_slots.back();
     ctx->free_slots.pop_back();
+    return slot;
+}
+
+void give_slot(pp_context* ctx, unsigned long long* slot) {
+    std::lock_guard<std::mutex> lock(ctx->slot_mutex);
+    ctx->free_slots.push_back(slot);
+}
+
+// A new sum's fixed device memory (one allocation: counters, read-out partials, hash rows, selection state, histograms
+// and window counts) and its pinned slots.
+pp_status alloc_fixed(pp_sum* s) {
+    pp_context* ctx = s->ctx;
+    if ((s->h_stats = take_slot(ctx)) == nullptr) return fail(ctx, PP_ERR_OUT_OF_MEMORY, "pinned host allocation");
     std::memset(s->h_stats, 0, kSumSlotWords * sizeof(unsigned long long));
     void* dev = nullptr;
     PP_HIP(ctx, hipHostGetDevicePointer(&dev, s->h_stats, 0));
@@ -2540,7 +2554,7 @@ pp_status pp_sum_free(pp_sum* s) {
         free_buckets(s->bk[i]);
     }
     if (s->d_fixed) (void)hipFree(s->d_fixed);
-    if (s->h_stats) s->ctx->free_slots.push_back(s->h_stats);
+    if (s->h_stats) give_slot(s->ctx, s->h_stats);
     if (s->d_redo) (void)hipFree(s->d_redo);
     if (s->d_score) (void)hipFree(s->d_score);
     if (s->d_tiles) (void)hipFree(s->d_tiles);
