@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstdio>
@@ -587,6 +588,7 @@ pp_status wait_for_mark(pp_context* ctx, volatile const unsigned long long* mark
             if (*mark != seq) return fail(ctx, PP_ERR_DRIVER, never);
             break;
         }
+    std::atomic_thread_fence(std::memory_order_acquire);  // the words written before the mark are read after it
     return PP_OK;
 }
 pp_status wait_for_slot(pp_context* ctx, volatile const unsigned long long* h, unsigned long long seq,
