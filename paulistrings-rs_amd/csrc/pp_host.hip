@@ -1823,6 +1823,16 @@ pp_status class_pass(pp_sum* s, const Prepared* layers, uint32_t n, const KeepPr
     int attempt = 0;
     uint64_t untouched = 0, out_rows = 0, part_most = 0;  // counts of the pass; the fullest part of the staging
     bool counted = false;                                 // ocap is a need, not an estimate
+    // the rows that the counted outputs need, in parts as uneven as they were
+    auto need_least = [&]() { return kClassParts * std::max<uint64_t>(part_most, 1); };
+    auto give_back_staging = [&]() {
+        for (ScratchSlot slot : {kScrClassOX, kScrClassOZ, kScrClassOC, kScrClassOB}) {
+            if (s->scratch[slot]) (void)hipFree(s->scratch[slot]);
+            s->scratch[slot] = nullptr;
+            s->scratch_cap[slot] = 0;
+        }
+        s->class_out_hint = 0;
+    };
     for (;;) {
         const uint32_t C = 1u << cbits;
         ocap = (ocap + kClassParts - 1) / kClassParts * kClassParts;
@@ -1837,15 +1847,11 @@ pp_status class_pass(pp_sum* s, const Prepared* layers, uint32_t n, const KeepPr
             (st = slot_scratch(s, kScrClassOZ, (size_t)s->W * ocap * 8, &oz)) != PP_OK ||
             (st = slot_scratch(s, kScrClassOC, ocap * cb, &oc)) != PP_OK ||
             (st = slot_scratch(s, kScrClassOB, ocap * 4, &ob)) != PP_OK || (st = ensure_tiles(s, C)) != PP_OK) {
-            if (st != PP_ERR_OUT_OF_MEMORY || counted || ocap <= ocap_least + kClassParts) return st;
-            // the estimate does not fit: give back what it took, and as many rows as the outputs turn out to be
-            for (ScratchSlot slot : {kScrClassOX, kScrClassOZ, kScrClassOC, kScrClassOB}) {
-                if (s->scratch[slot]) (void)hipFree(s->scratch[slot]);
-                s->scratch[slot] = nullptr;
-                s->scratch_cap[slot] = 0;
-            }
-            s->class_out_hint = 0;
-            ocap = ocap_least;
+            // the estimate, or the need with its spare rows, does not fit: as many rows as there have to be
+            const uint64_t least = counted ? need_least() : (ocap_least + kClassParts - 1) / kClassParts * kClassParts;
+            if (st != PP_ERR_OUT_OF_MEMORY || ocap <= least) return st;
+            give_back_staging();
+            ocap = least;
             continue;
         }
         d_cst = reinterpret_cast<unsigned long long*>(d_counts);
@@ -1910,7 +1916,15 @@ pp_status class_pass(pp_sum* s, const Prepared* layers, uint32_t n, const KeepPr
             part_most = std::max<uint64_t>(part_most, q[0]);
             untouched += q[1];
         }
-        if (flags == 0) break;
+        if (flags == 0) {  // the output columns: in the room of the staging's spare rows when there is no other
+            st = ensure_columns(s, 1 - s->cur, untouched + out_rows + (uint64_t)kSegAlign * B);
+            if (st == PP_OK) break;
+            if (st != PP_ERR_OUT_OF_MEMORY || ocap <= need_least()) return st;
+            give_back_staging();
+            ocap = need_least();
+            counted = true;
+            continue;
+        }
         counted = counted || !(flags & 3ull);
         if ((flags & 3ull) == 0) {  // only the output staging ran out: the same chunks' need is known now, and roughly
             ocap = kClassParts * (part_most + part_most / 4);  // how unevenly they spread over the parts
@@ -1933,7 +1947,6 @@ pp_status class_pass(pp_sum* s, const Prepared* layers, uint32_t n, const KeepPr
     const uint64_t total = untouched + out_rows;
     s->class_out_hint = std::max(s->class_out_hint, kClassParts * (part_most + part_most / 8));
     const int in = s->cur, out = 1 - s->cur;
-    if ((st = ensure_columns(s, out, total + (uint64_t)kSegAlign * B)) != PP_OK) return st;
     if ((st = ensure_buckets(s, out, B)) != PP_OK) return st;
     hipError_t e = dispatch(s, [&](auto Wc, auto Tv) {
         constexpr int W = decltype(Wc)::value;

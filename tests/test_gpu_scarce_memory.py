@@ -8,6 +8,7 @@ import contextlib
 import numpy as np
 import pytest
 
+from paulistrings_amd import tables, truncation
 from test_gpu_transfer import upload
 
 pytestmark = pytest.mark.gpu
@@ -52,6 +53,34 @@ def test_an_upload_beside_little_free_memory():
     with device_memory_left(400):
         g = upload(50, x, z, c)
         assert len(g) == len(c)
+    assert not any(v for k, v in g.check_layout().items() if k != "unscanned")
+    got = g.to_host()
+    g.free()
+    assert np.array_equal(got._x, want._x) and np.array_equal(got._z, want._z) and np.array_equal(got._c, want._c)
+
+
+@pytest.mark.parametrize("left", [1010, 790])
+def test_a_general_table_beside_little_free_memory(left):
+    """2^22 terms through a near-identity two-qubit unitary whose small outputs are dropped.  The outputs are staged in room
+    for four times the terms, 768 MB; with 1010 MB left that fits and the columns they are placed in (112 MB) do not, with
+    790 it does not, and half of it does."""
+    n = 1 << 22
+    x, z, c = spread_terms(n, 50, np.float32)
+    rng = np.random.default_rng(3)
+    h = rng.standard_normal((4, 4)) + 1j * rng.standard_normal((4, 4))
+    w, v = np.linalg.eigh(h + h.conj().T)
+    table = tables.unitary_table((v * np.exp(-0.002j * w)) @ v.conj().T, [3, 17], np.float32)
+    assert table.n_deltas == 16
+    c = 1.0 + c / 2000
+    policy = truncation.coeff(0.5)
+    g = upload(50, x, z, c)
+    g.apply_table(table, policy)
+    want = g.to_host()
+    g.free()
+    assert len(want) == n
+    g = upload(50, x, z, c)
+    with device_memory_left(left):
+        g.apply_table(table, policy)
     assert not any(v for k, v in g.check_layout().items() if k != "unscanned")
     got = g.to_host()
     g.free()
