@@ -468,7 +468,15 @@ pp_status ensure_columns(pp_sum* s, int which, uint64_t need) {
     const uint64_t cap = (std::max<uint64_t>(need + extra, 1024) + (kSegAlign - 1)) & ~(uint64_t)(kSegAlign - 1);
     pp_status st;
     unsigned char* base = nullptr;
-    if ((st = dev_alloc(s->ctx, (void**)&base, cap * (2 * s->W * 8 + s->coeff_bytes()))) != PP_OK) return st;
+    const size_t bytes = cap * (2 * s->W * 8 + s->coeff_bytes());
+    if ((st = dev_alloc(s->ctx, (void**)&base, bytes)) == PP_ERR_OUT_OF_MEMORY && s->scratch[kScrWindow]) {
+        // a windowed selection's scratch (8 bytes a term) only saves time, and no selection is under way
+        (void)hipFree(s->scratch[kScrWindow]);
+        s->scratch[kScrWindow] = nullptr;
+        s->scratch_cap[kScrWindow] = 0;
+        st = dev_alloc(s->ctx, (void**)&base, bytes);
+    }
+    if (st != PP_OK) return st;
     c.x = (uint64_t*)base;
     c.z = (uint64_t*)(base + cap * s->W * 8);  // cap is a multiple of kSegAlign: every array starts 128-B aligned
     c.c = base + 2 * cap * s->W * 8;

@@ -85,3 +85,22 @@ def test_a_general_table_beside_little_free_memory(left):
     got = g.to_host()
     g.free()
     assert np.array_equal(got._x, want._x) and np.array_equal(got._z, want._z) and np.array_equal(got._c, want._c)
+
+
+def test_columns_beside_a_selection_s_scratch():
+    """A sum of 2^24 terms keeps 128 MB of scratch of its last selection, then takes a sum of 2^25: columns of 1020 MB in
+    place of its 510, with 448 MB left."""
+    terms = spread_terms(1 << 25, 50, np.float32)
+    src, dst = upload(50, *terms), upload(50, *(a[: 1 << 24] for a in terms))
+    for n in ((1 << 24) - 5, (1 << 24) - 10):  # the second starts from the boundary of the first
+        dst.truncate_topn(n)
+        assert len(dst) == n
+    with device_memory_left(448):
+        dst.copy_from(src)
+        dst.ctx.sync()
+    assert not any(v for k, v in dst.check_layout().items() if k != "unscanned")
+    want = src.to_host()
+    src.free()
+    got = dst.to_host()
+    dst.free()
+    assert np.array_equal(got._x, want._x) and np.array_equal(got._z, want._z) and np.array_equal(got._c, want._c)
