@@ -570,13 +570,13 @@ pp_status alloc_fixed(pp_sum* s) {
     s->h_lag = s->h_stats + kStatSlots;
     s->d_lag_host = (unsigned long long*)dev + kStatSlots;
     auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
-    const size_t stats = (kStatSlots + kReadoutGroups + 8) * 8, rows = s->rows.size() * 8;
+    const size_t stats = (kStatSlots + 2 * kReadoutGroups + 8) * 8, rows = s->rows.size() * 8;
     const size_t o_rows = up(stats), o_topn = o_rows + up(rows), o_hist = o_topn + up(sizeof(TopnState));
     const size_t o_window = o_hist + up(kSeededHistWords * 8), o_octave = o_window + up(sizeof(WindowCounts));
     pp_status st = dev_alloc(ctx, (void**)&s->d_fixed, o_octave + sizeof(OctaveCounts));
     if (st != PP_OK) return st;
     s->d_stats = (unsigned long long*)s->d_fixed;
-    s->d_lag_counters = s->d_stats + kStatSlots + kReadoutGroups;
+    s->d_lag_counters = s->d_stats + kStatSlots + 2 * kReadoutGroups;
     s->d_rows = (uint64_t*)(s->d_fixed + o_rows);
     s->d_topn = (TopnState*)(s->d_fixed + o_topn);
     s->d_hist = (unsigned long long*)(s->d_fixed + o_hist);

@@ -262,7 +262,7 @@ struct ExpectationArgs {
     uint64_t axis_z[W];
     uint64_t negative[W];
     uint32_t sieve;   // what of word 0 rules most terms out: 1 an x bit off the axis, 2 a z bit, 0 the two together
-    double* partial;  // a sum per workgroup, at most kReadoutGroups
+    double* partial;  // per workgroup, at most kReadoutGroups: its sum, and what its roundings lost
     unsigned long long* host;  // pinned: [0] the total's bits, then [4] = seq
     unsigned long long seq;
 };
