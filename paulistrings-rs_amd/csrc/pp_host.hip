@@ -457,7 +457,9 @@ void free_buckets(BucketArrays& b) {
     b = BucketArrays{};
 }
 
-pp_status ensure_columns(pp_sum* s, int which, uint64_t need) {
+// With `exact`, no headroom: for a set that takes over another's layout with the room that has.  (With headroom upon
+// headroom, a sum reset and refined again and again, or a clone of a clone, grew by a quarter each time.)
+pp_status ensure_columns(pp_sum* s, int which, uint64_t need, bool exact = false) {
     Columns& c = s->col[which];
     if (c.cap >= need && c.x) return PP_OK;
     free_columns(c);
@@ -465,7 +467,8 @@ pp_status ensure_columns(pp_sum* s, int which, uint64_t need) {
     // few times rather than every few layers (each hipFree waits for the device).  A multiple of kSegAlign, so that
     // every word column starts as aligned as the first.
     const uint64_t extra = std::max<uint64_t>(need / 4, std::min<uint64_t>(need, 1ull << 20));
-    const uint64_t cap = (std::max<uint64_t>(need + extra, 1024) + (kSegAlign - 1)) & ~(uint64_t)(kSegAlign - 1);
+    const uint64_t rows = std::max<uint64_t>(exact ? need : need + extra, 1024);
+    const uint64_t cap = (rows + (kSegAlign - 1)) & ~(uint64_t)(kSegAlign - 1);
     pp_status st;
     unsigned char* base = nullptr;
     const size_t bytes = cap * (2 * s->W * 8 + s->coeff_bytes());
@@ -786,7 +789,7 @@ pp_status refine_once(pp_sum* s) {
     const int in = s->cur, out = 1 - s->cur;
     const uint32_t B = 1u << s->device_bits;
     pp_status st;
-    if ((st = ensure_columns(s, out, s->col[in].cap)) != PP_OK) return st;
+    if ((st = ensure_columns(s, out, s->col[in].cap, true)) != PP_OK) return st;
     if ((st = ensure_buckets(s, out, 2ull * B)) != PP_OK) return st;
     if ((st = clear_stats(s)) != PP_OK) return st;
     hipError_t e = dispatch(s, [&](auto Wc, auto Tv) {
@@ -2617,7 +2620,7 @@ pp_status pp_sum_clone(const pp_sum* src_c, pp_sum** out) {
     if ((st = alloc_fixed(s)) != PP_OK) return bail(st);
     const Columns& sc = src->col[src->cur];
     const BucketArrays& sb = src->bk[src->cur];
-    if ((st = ensure_columns(s, 0, sc.cap)) != PP_OK) return bail(st);
+    if ((st = ensure_columns(s, 0, sc.cap, true)) != PP_OK) return bail(st);
     if ((st = ensure_buckets(s, 0, 1ull << src->device_bits)) != PP_OK) return bail(st);
     const uint64_t B = 1ull << src->device_bits;
     const uint64_t cap = s->col[0].cap;
