@@ -329,7 +329,8 @@ typedef struct {
     uint32_t bucket_target; /* rows per device bucket, 16..512 (default 256) */
     uint32_t stage_rows;    /* anticommuting rows a join workgroup stages in its first launch, 64..1024 (a pair
                                with more is redone by a second launch that stages the largest pair);
-                               0: the largest pair, no second launch (default) */
+                               0: the largest pair, no second launch (default).  A layer in place stages at most
+                               256 in its first launch, a row per thread: with 0 or a larger value, 256 */
     uint32_t groups_per_cu; /* the join's grid: 0xFFFFFFFF one workgroup per pair (default); 0 a persistent
                                grid of as many as fit; 1..32 persistent with at most that many per CU */
     uint32_t join_block;    /* threads per join workgroup, the rows of one pass: 256 (default) or 512 */

@@ -1450,7 +1450,8 @@ pp_status layer_in_place(pp_sum* s, const Prepared& p, const KeepProgram& keep) 
     uint32_t lcap = delta ? 2u * s->max_bucket : s->max_bucket;
     lcap = std::max<uint32_t>(64, (lcap + 63) & ~63u);
     if (lcap > kMaxPairRows) lcap = kMaxPairRows;
-    // a generator anticommutes with a fraction of a bucket: the first launch stages at most a row per thread
+    // a generator anticommutes with a fraction of a bucket: the first launch stages at most a row per thread, whatever
+    // larger number the tuning gives the out-of-place join
     const uint32_t scap = std::min<uint32_t>({ctx->tuning.stage_rows ? join_stage_rows(ctx->tuning.stage_rows, lcap)
                                                                      : (uint32_t)kBlock,
                                              (uint32_t)kBlock, lcap});

@@ -44,7 +44,8 @@ class Options(ctypes.Structure):
 
 
 class Tuning(ctypes.Structure):
-    """pp_tuning: the device path's sizes (bucket_target, stage_rows, groups_per_cu, join_block, join_in_place)."""
+    """pp_tuning: the device path's sizes (bucket_target, stage_rows, groups_per_cu, join_block, join_in_place).  A layer
+    in place stages at most 256 rows in its first launch, whatever larger number stage_rows is."""
 
     _fields_ = [("bucket_target", ctypes.c_uint32), ("stage_rows", ctypes.c_uint32),
                 ("groups_per_cu", ctypes.c_uint32), ("join_block", ctypes.c_uint32),
