@@ -261,7 +261,7 @@ struct CapturedJoin {
     pp_sum* dst;
     int src_cur, dst_cur, device_bits;
     const void* src_ptrs[5];  // x, z, c, bucket start, bucket len
-    const void* dst_ptrs[7];  // x, z, c, bucket start, bucket len, counters, redo queue
+    const void* dst_ptrs[8];  // x, z, c, bucket start, bucket len, counters, redo queue, the offset scan's tile sums
     uint64_t dst_cap;         // rows of dst's written column set
     uint64_t src_len;         // rows src held at capture: the output columns and staging were sized from them
     uint32_t src_max_bucket;
@@ -2798,10 +2798,13 @@ static pp_status download_sorted(pp_sum* s, uint64_t* x, uint64_t* z, void* coef
     const bool split = RB > B;
     const uint32_t limit = s->W == 1 ? kSortRows<1> : kSortRows<2>;
     if ((split ? RB / B : B / RB) > kSortParts || (split && s->max_bucket > limit)) return PP_OK;
-    uint64_t* d_start = nullptr;  // dense starts, then lengths, of the reference buckets
-    if ((st = slot_scratch(s, kScrCounts, (size_t)RB * 12, &d_start)) != PP_OK) return st;
-    uint32_t* const d_len = reinterpret_cast<uint32_t*>(d_start + RB);
-    if ((st = ensure_tiles(s, RB)) != PP_OK) return st;
+    // the reference buckets' dense starts, the scan's tile sums and the lengths; not the sum's own tile sums, which a
+    // captured graph that writes this sum may hold and RB buckets may outgrow
+    uint64_t* d_start = nullptr;
+    const uint64_t tiles = std::max<uint32_t>(offsets_tiles(RB), 1);
+    if ((st = slot_scratch(s, kScrCounts, (size_t)RB * 12 + tiles * 8, &d_start)) != PP_OK) return st;
+    uint64_t* const d_tiles = d_start + RB;
+    uint32_t* const d_len = reinterpret_cast<uint32_t*>(d_tiles + tiles);
     unsigned char* dev = nullptr;
     const size_t key_bytes = n * s->W * 8;
     auto args = [&](auto Wc, auto Tv) {
@@ -2830,11 +2833,11 @@ static pp_status download_sorted(pp_sum* s, uint64_t* x, uint64_t* z, void* coef
     if (split) {  // the rows of each reference bucket counted, then laid out
         e = dispatch(s, [&](auto Wc, auto Tv) { return launch_ref_counts(ctx->stream, args(Wc, Tv)); });
         if (e == hipSuccess)
-            e = launch_bucket_offsets(ctx->stream, d_len, RB, 0, 0, 0, 0, d_start, s->d_stats + 3, s->d_tiles);
+            e = launch_bucket_offsets(ctx->stream, d_len, RB, 0, 0, 0, 0, d_start, s->d_stats + 3, d_tiles);
         PP_HIP(ctx, e);
     } else {
         PP_HIP(ctx, launch_bucket_offsets(ctx->stream, s->bk[s->cur].len, B, 5, 0, RB, B / RB, d_start, s->d_stats + 3,
-                                          s->d_tiles, s->d_stats, kStatSlots, d_len));
+                                          d_tiles, s->d_stats, kStatSlots, d_len));
         PP_HIP(ctx, launch_reduce_lens(ctx->stream, d_len, RB, s->d_stats, nullptr));
         if ((st = read_stats(s)) != PP_OK) return st;
         longest = s->h_stats[1];
@@ -3021,10 +3024,10 @@ pp_status pp_apply_rotation_to(pp_sum* src, pp_sum* dst, const pp_channel* ch, i
         r.dst_cur = out;
         r.device_bits = src->device_bits;
         const void* sp[5] = {src->col[in].x, src->col[in].z, src->col[in].c, src->bk[in].start, src->bk[in].len};
-        const void* dp[7] = {dst->col[out].x, dst->col[out].z, dst->col[out].c, dst->bk[out].start,
-                             dst->bk[out].len, dst->d_stats, dst->d_redo};
+        const void* dp[8] = {dst->col[out].x, dst->col[out].z, dst->col[out].c, dst->bk[out].start,
+                             dst->bk[out].len, dst->d_stats, dst->d_redo, dst->d_tiles};
         std::copy(sp, sp + 5, r.src_ptrs);
-        std::copy(dp, dp + 7, r.dst_ptrs);
+        std::copy(dp, dp + 8, r.dst_ptrs);
         r.dst_cap = dst->col[out].cap;
         r.src_len = src->len;
         r.src_max_bucket = src->max_bucket;
@@ -4101,13 +4104,13 @@ bool captured_join_valid(const CapturedJoin& r, std::string& what) {
     const pp_sum* dst = r.dst;
     const int in = r.src_cur, out = r.dst_cur;
     const void* sp[5] = {src->col[in].x, src->col[in].z, src->col[in].c, src->bk[in].start, src->bk[in].len};
-    const void* dp[7] = {dst->col[out].x, dst->col[out].z, dst->col[out].c, dst->bk[out].start, dst->bk[out].len,
-                         dst->d_stats, dst->d_redo};
+    const void* dp[8] = {dst->col[out].x, dst->col[out].z, dst->col[out].c, dst->bk[out].start, dst->bk[out].len,
+                         dst->d_stats, dst->d_redo, dst->d_tiles};
     if (src->cur != in || src->device_bits != r.device_bits || !std::equal(sp, sp + 5, r.src_ptrs)) {
         what = "the input's columns or device bucketing changed since the capture";
         return false;
     }
-    if (dst->cur != out || dst->col[out].cap != r.dst_cap || !std::equal(dp, dp + 7, r.dst_ptrs)) {
+    if (dst->cur != out || dst->col[out].cap != r.dst_cap || !std::equal(dp, dp + 8, r.dst_ptrs)) {
         what = "the output's current columns changed since the capture (a layer in place, or a reallocation)";
         return false;
     }
