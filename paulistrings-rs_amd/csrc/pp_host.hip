@@ -651,14 +651,14 @@ pp_status ensure_tiles(pp_sum* s, uint32_t out_n) {
     return PP_OK;
 }
 
-// Slot `slot` of the sum's truncation scratch with room for `bytes` (grown to 1.5x the request when it must grow).
+// Slot `slot` of the sum's scratch with room for `bytes`; when it must grow, to `room` bytes, or to twice the request.
 template <typename P>
-pp_status slot_scratch(pp_sum* s, ScratchSlot slot, size_t bytes, P** out) {
+pp_status slot_scratch(pp_sum* s, ScratchSlot slot, size_t bytes, P** out, size_t room = 0) {
     if (s->scratch_cap[slot] < bytes || !s->scratch[slot]) {
         if (s->scratch[slot]) (void)hipFree(s->scratch[slot]);
         s->scratch[slot] = nullptr;
         s->scratch_cap[slot] = 0;
-        const size_t grown = std::max<size_t>(256, 2 * bytes);
+        const size_t grown = std::max<size_t>(256, room ? std::max(room, bytes) : 2 * bytes);
         pp_status st = dev_alloc(s->ctx, &s->scratch[slot], grown);
         if (st != PP_OK) return st;
         s->scratch_cap[slot] = grown;
@@ -1836,8 +1836,24 @@ pp_status class_pass(pp_sum* s, const Prepared* layers, uint32_t n, const KeepPr
     uint32_t lcap = 512, icap = n == 1 && fills ? 128 : 512, tbits = icap == 128 ? 8 : 10;
     uint32_t chunk = (uint32_t)std::max<uint64_t>(16, (fills ? 256 : 512) / std::min<uint64_t>(growth, 16));
     // the staging's parts hold a few chunks' outputs more than their share
-    const uint64_t ocap_least = 2 * len_in + kClassParts * 1024ull;
-    uint64_t ocap = std::max({ocap_least, s->class_out_hint, std::min<uint64_t>(growth, 16) / 4 * len_in});
+    auto whole_parts = [](uint64_t rows) { return (rows + kClassParts - 1) / kClassParts * kClassParts; };
+    const uint64_t ocap_least = whole_parts(2 * len_in + kClassParts * 1024ull);
+    // What earlier passes left serves while it holds twice the input and the last outputs.  Else an estimate, in room for
+    // four times the input; with twice that, or a second allocation where the counted outputs fit the first, a sum's first
+    // pass was slower than the pass itself (2^18 two-word terms: 1.3-2.0 ms in place of 1.0).
+    struct {
+        ScratchSlot slot;
+        size_t bytes;
+    } const staging[4] = {{kScrClassOX, s->W * 8}, {kScrClassOZ, s->W * 8}, {kScrClassOC, cb}, {kScrClassOB, 4}};
+    auto held_rows = [&]() {
+        uint64_t rows = UINT64_MAX;
+        for (const auto& a : staging) rows = std::min<uint64_t>(rows, s->scratch_cap[a.slot] / a.bytes);
+        return rows / kClassParts * kClassParts;
+    };
+    uint64_t ocap = std::max(ocap_least, whole_parts(s->class_out_hint));
+    ocap = held_rows() >= ocap ? held_rows()
+                               : std::max(ocap, whole_parts(std::min<uint64_t>(growth, 16) / 4 * len_in));
+    bool roomy = true;  // four times the input while memory allows
     uint64_t *ox = nullptr, *oz = nullptr;
     void* oc = nullptr;
     uint32_t* ob = nullptr;
@@ -1849,16 +1865,18 @@ pp_status class_pass(pp_sum* s, const Prepared* layers, uint32_t n, const KeepPr
     // the rows that the counted outputs need, in parts as uneven as they were
     auto need_least = [&]() { return kClassParts * std::max<uint64_t>(part_most, 1); };
     auto give_back_staging = [&]() {
-        for (ScratchSlot slot : {kScrClassOX, kScrClassOZ, kScrClassOC, kScrClassOB}) {
-            if (s->scratch[slot]) (void)hipFree(s->scratch[slot]);
-            s->scratch[slot] = nullptr;
-            s->scratch_cap[slot] = 0;
+        for (const auto& a : staging) {
+            if (s->scratch[a.slot]) (void)hipFree(s->scratch[a.slot]);
+            s->scratch[a.slot] = nullptr;
+            s->scratch_cap[a.slot] = 0;
         }
         s->class_out_hint = 0;
+        roomy = false;
     };
     for (;;) {
         const uint32_t C = 1u << cbits;
-        ocap = (ocap + kClassParts - 1) / kClassParts * kClassParts;
+        ocap = whole_parts(ocap);
+        const uint64_t room = roomy ? std::max(ocap, 4 * len_in) : ocap;
         // the counters, the outputs per bucket and the rows per class bucket: one block, one clear
         unsigned char* d_counts = nullptr;
         uint64_t* d_cstart = nullptr;
@@ -1866,15 +1884,15 @@ pp_status class_pass(pp_sum* s, const Prepared* layers, uint32_t n, const KeepPr
         const size_t count_bytes = kClassStatSlots * 8 + ocount_bytes + (size_t)C * 4;
         if ((st = slot_scratch(s, kScrClassCount, count_bytes, &d_counts)) != PP_OK ||
             (st = slot_scratch(s, kScrClassStart, (size_t)C * 8, &d_cstart)) != PP_OK ||
-            (st = slot_scratch(s, kScrClassOX, (size_t)s->W * ocap * 8, &ox)) != PP_OK ||
-            (st = slot_scratch(s, kScrClassOZ, (size_t)s->W * ocap * 8, &oz)) != PP_OK ||
-            (st = slot_scratch(s, kScrClassOC, ocap * cb, &oc)) != PP_OK ||
-            (st = slot_scratch(s, kScrClassOB, ocap * 4, &ob)) != PP_OK || (st = ensure_tiles(s, C)) != PP_OK) {
-            // the estimate, or the need with its spare rows, does not fit: as many rows as there have to be
-            const uint64_t least = counted ? need_least() : (ocap_least + kClassParts - 1) / kClassParts * kClassParts;
-            if (st != PP_ERR_OUT_OF_MEMORY || ocap <= least) return st;
+            (st = slot_scratch(s, kScrClassOX, s->W * 8 * ocap, &ox, s->W * 8 * room)) != PP_OK ||
+            (st = slot_scratch(s, kScrClassOZ, s->W * 8 * ocap, &oz, s->W * 8 * room)) != PP_OK ||
+            (st = slot_scratch(s, kScrClassOC, cb * ocap, &oc, cb * room)) != PP_OK ||
+            (st = slot_scratch(s, kScrClassOB, 4 * ocap, &ob, 4 * room)) != PP_OK || (st = ensure_tiles(s, C)) != PP_OK) {
+            // the room, then the estimate or the need with its spare rows, does not fit: as many rows as there have to be
+            const uint64_t least = counted ? need_least() : ocap_least;
+            if (st != PP_ERR_OUT_OF_MEMORY || (!roomy && ocap <= least)) return st;
+            if (!roomy) ocap = least;
             give_back_staging();
-            ocap = least;
             continue;
         }
         d_cst = reinterpret_cast<unsigned long long*>(d_counts);
@@ -1942,7 +1960,7 @@ pp_status class_pass(pp_sum* s, const Prepared* layers, uint32_t n, const KeepPr
         if (flags == 0) {  // the output columns: in the room of the staging's spare rows when there is no other
             st = ensure_columns(s, 1 - s->cur, untouched + out_rows + (uint64_t)kSegAlign * B);
             if (st == PP_OK) break;
-            if (st != PP_ERR_OUT_OF_MEMORY || ocap <= need_least()) return st;
+            if (st != PP_ERR_OUT_OF_MEMORY || (!roomy && ocap <= need_least())) return st;
             give_back_staging();
             ocap = need_least();
             counted = true;
@@ -1950,7 +1968,9 @@ pp_status class_pass(pp_sum* s, const Prepared* layers, uint32_t n, const KeepPr
         }
         counted = counted || !(flags & 3ull);
         if ((flags & 3ull) == 0) {  // only the output staging ran out: the same chunks' need is known now, and roughly
-            ocap = kClassParts * (part_most + part_most / 4);  // how unevenly they spread over the parts
+            const uint64_t need = need_least();               // how unevenly they spread over the parts
+            ocap = need + need / 4;
+            if (held_rows() >= need) ocap = std::min(ocap, held_rows());
         } else if (attempt == 0) {
             cbits = std::min(cbits + 2, 24);
             chunk = fills ? 16 : 32;

@@ -59,11 +59,12 @@ def test_an_upload_beside_little_free_memory():
     assert np.array_equal(got._x, want._x) and np.array_equal(got._z, want._z) and np.array_equal(got._c, want._c)
 
 
-@pytest.mark.parametrize("left", [1010, 790])
+@pytest.mark.parametrize("left", [1010, 790, 640, 540])
 def test_a_general_table_beside_little_free_memory(left):
-    """2^22 terms through a near-identity two-qubit unitary whose small outputs are dropped.  The outputs are staged in room
-    for four times the terms, 768 MB; with 1010 MB left that fits and the columns they are placed in (112 MB) do not, with
-    790 it does not, and half of it does."""
+    """2^22 terms through a near-identity two-qubit unitary whose small outputs are dropped.  The rows it moves take 190 MB,
+    the outputs are staged in room for four times the terms, 384 MB, and the columns they are placed in take 112.  With
+    640 MB left the staging fits and the columns do not, with 540 half of the staging fits; twice the staging (768 MB) would
+    leave no room for the columns with 1010."""
     n = 1 << 22
     x, z, c = spread_terms(n, 50, np.float32)
     rng = np.random.default_rng(3)
