@@ -51,6 +51,7 @@ struct ClassLayer {
     uint32_t mask;       // the patterns' live bits: 15 with two support qubits, 3 with one
     uint32_t active;     // bit s: the layer moves, rescales or fills pattern s (else s keeps key and coefficient)
     uint32_t n_entries;  // entries ascending by local delta, the identity first when present
+    uint32_t fanout;     // the most entries with an amplitude on one pattern
     uint32_t delta[kClassMaxEntries];
     double amp[kClassMaxEntries][16];  // entry e's amplitude on source pattern s, rounded to the coefficient type
 };

@@ -8,10 +8,11 @@
 // the source of pattern t ^ delta[e] in its class, with amplitude amp[e][t ^ delta[e]].  It sums the contributions of
 // the sources present in entry order (one rounded multiply and one rounded add each, as a rotation's pair update or the
 // host engine's merge), asks keep and appends it to the other set.  A rotation table (identity entry first, then the
-// generator) gives own = c cos + c_partner a1 exactly as the pair join does.  A table of few entries gives a row's
-// outputs to one thread (the source that comes first in entry order owns an output); from kClassWideEntries on every
-// pattern of a class has a thread of its own: a general two-qubit table turns the 16 to 32 rows of a workgroup's classes
-// into up to 500 outputs of 16 sources, which would leave seven of its eight waves idle.
+// generator) gives own = c cos + c_partner a1 exactly as the pair join does.  A row's outputs
+// belong to one thread (the source that comes first in entry order owns an output), or every pattern of a class has a
+// thread of its own: a general two-qubit table turns the 16 to 32 rows of a workgroup's classes into up to 500 outputs of
+// 16 sources, which would leave seven of its eight waves idle; a CNOT gives each of up to 512 rows one output, and a thread
+// for each of their 16 patterns made its pass over 1000 terms 54 us in place of 22.
 
 #include "pp_class.h"
 
@@ -111,6 +112,7 @@ __global__ void __launch_bounds__(kClassBlock) k_class_apply(const ClassArgs<W, 
     __shared__ uint32_t s_bit[kClassMaxLayers][2];
     __shared__ uint32_t s_mask[kClassMaxLayers];
     __shared__ uint32_t s_ne[kClassMaxLayers];
+    __shared__ uint32_t s_fan[kClassMaxLayers];
     __shared__ uint32_t s_off[kClassMaxLayers];
     __shared__ uint32_t s_delta[kClassMaxLayers][kClassMaxEntries];
     __shared__ uint32_t s_count[2];
@@ -136,6 +138,7 @@ __global__ void __launch_bounds__(kClassBlock) k_class_apply(const ClassArgs<W, 
         s_bit[tid][1] = L.bit[1];
         s_mask[tid] = L.mask;
         s_ne[tid] = L.n_entries;
+        s_fan[tid] = L.fanout;
         for (uint32_t e = 0; e < kClassMaxEntries; ++e) s_delta[tid][e] = L.delta[e];
     }
     __syncthreads();
@@ -249,8 +252,11 @@ __global__ void __launch_bounds__(kClassBlock) k_class_apply(const ClassArgs<W, 
                     s_bad[slot] = 1u;
                 }
             };
-            const bool wide = ne >= kClassWideEntries;  // uniform
-            const uint32_t dim = s_mask[l] + 1u;        // patterns: 16, 4 or 1
+            const uint32_t dim = s_mask[l] + 1u;  // patterns: 16, 4 or 1
+            // a thread per pattern when its rounds are fewer than the outputs that a thread per row makes one by one
+            const bool wide = ne >= kClassWideEntries &&
+                              (n * dim + kClassBlock - 1) / kClassBlock <
+                                  (n + kClassBlock - 1) / kClassBlock * s_fan[l];  // uniform
             for (uint32_t it = tid; wide && it < n * dim; it += kClassBlock) {
                 const uint32_t i = it / dim, t = it % dim;
                 if (row_rec[i] != i) continue;  // the row that holds its class's record

@@ -1743,6 +1743,11 @@ ClassLayer class_layer(const Prepared& p) {
         for (uint32_t q = 0; q < dim; ++q)
             if (L.amp[1][q] != 0.0) L.amp[0][q] = 0.0;
     for (uint32_t q = 0; q < dim; ++q) {
+        uint32_t outputs = 0;
+        for (uint32_t e = 0; e < t.n_deltas; ++e) outputs += L.amp[e][q] != 0.0;
+        L.fanout = std::max(L.fanout, outputs);
+    }
+    for (uint32_t q = 0; q < dim; ++q) {
         bool still = identity >= 0 && L.amp[identity][q] == 1.0;
         for (uint32_t e = 0; e < t.n_deltas && still; ++e)
             if ((int)e != identity) still = L.amp[e][q] == 0.0 && L.amp[e][q ^ L.delta[e]] == 0.0;
