@@ -15,8 +15,10 @@
  *     the reference's x_array()/z_array() hand them out); W is 1 (<= 64 qubits)
  *     or 2 (<= 128 qubits);
  *   - coefficients are float64 or float32 (coefficient.rs:199-200);
- *   - calls on one context are serialized by the caller; work inside a call is
- *     asynchronous on the context's stream and pp_sync() waits for it;
+ *   - calls on one context are serialized by the caller, but for pp_sum_free,
+ *     which may come from another thread (a collector's) outside a graph
+ *     capture; work inside a call is asynchronous on the context's stream and
+ *     pp_sync() waits for it;
  *   - every entry point returns a pp_status; pp_last_error() explains the last
  *     failure on a context.
  */

@@ -105,7 +105,7 @@ __global__ void __launch_bounds__(kBlock) k_ref_counts(const SortExportArgs<W, T
 // reference bucket and the keys' words (x ascending, then z), and the rows written out term-major in that order.
 // SPLIT: a device bucket of several reference buckets; else a reference bucket of one or more device buckets.
 // Latency of LDS and barriers bounds it (55 stages for 1024 rows); a workgroup's neighbours on its compute unit fill
-// the waits.  2^20 two-word f64 terms: a download of 3.8 ms, most of it the host's copies, against 13.4 ms when the
+// the waits.  2^20 two-word f64 terms: a download of 2.6 ms, most of it the host's copies, against 13.4 ms when the
 // host sorted.
 template <int W, typename T, bool SPLIT>
 __global__ void __launch_bounds__(512) k_sort_export(const SortExportArgs<W, T> a, uint32_t padded) {
