@@ -8,11 +8,11 @@
 // the source of pattern t ^ delta[e] in its class, with amplitude amp[e][t ^ delta[e]].  It sums the contributions of
 // the sources present in entry order (one rounded multiply and one rounded add each, as a rotation's pair update or the
 // host engine's merge), asks keep and appends it to the other set.  A rotation table (identity entry first, then the
-// generator) gives own = c cos + c_partner a1 exactly as the pair join does.  A row's outputs
-// belong to one thread (the source that comes first in entry order owns an output), or every pattern of a class has a
-// thread of its own: a general two-qubit table turns the 16 to 32 rows of a workgroup's classes into up to 500 outputs of
-// 16 sources, which would leave seven of its eight waves idle; a CNOT gives each of up to 512 rows one output, and a thread
-// for each of their 16 patterns made its pass over 1000 terms 54 us in place of 22.
+// generator) gives own = c cos + c_partner a1 exactly as the pair join does.  A row's outputs belong to one thread (the
+// source that comes first in entry order owns an output), or every pattern of a class has a thread of its own: a general
+// two-qubit table turns the 16 to 32 rows of a workgroup's classes into up to 500 outputs of 16 sources, which would leave
+// seven of its eight waves idle; a CNOT gives each of up to 512 rows one output, and a thread for each of their 16 patterns
+// made its pass over 1000 terms 54 us in place of 22.
 
 #include "pp_class.h"
 
