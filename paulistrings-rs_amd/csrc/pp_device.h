@@ -13,7 +13,8 @@ namespace pp {
 constexpr int kBlock = 256;  // threads per workgroup: four wave64s
 constexpr int kWaves = kBlock / 64;
 constexpr int kMaxKeepNodes = 15;
-// Bucket segments of a resident layout start on a multiple of kSegAlign rows (128 bytes of every 8-byte column),
+// Bucket segments of a resident layout start on a multiple of kSegAlign rows (128 bytes of every 8-byte column; a
+// refinement's second halves start where the first ones end, until the next layer that lays the sum out),
 // so that no cache line holds the end of one bucket and the start of the next: two workgroups, possibly on
 // different XCDs with their own L2, would each move that line.
 constexpr uint32_t kSegAlign = 16;

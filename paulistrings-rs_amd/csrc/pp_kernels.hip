@@ -2321,8 +2321,8 @@ __global__ void __launch_bounds__(kBlock) k_check_layout(const CheckArgs<W, T> a
     if (threadIdx.x < kCheckCounts) counts[threadIdx.x] = 0u;
     for (uint32_t i = threadIdx.x; i < kSlots; i += kBlock) table[i] = 0u;
     __syncthreads();
-    const bool seg_ok = (n == 0 || s0 % kSegAlign == 0) && n <= extent && (extent == 0 || s0 + extent <= a.end) &&
-                        a.end <= a.cap;
+    // (a refinement's second half starts where the first ends, aligned or not)
+    const bool seg_ok = n <= extent && (extent == 0 || s0 + extent <= a.end) && a.end <= a.cap;
     if (!seg_ok) {
         if (threadIdx.x == 0) atomicAdd(&a.out[kCheckSegments], 1ull);
         return;  // the whole workgroup: its rows are not read
